@@ -576,8 +576,7 @@ int query_lut_setup(const void* q, int q_dtype, int64_t q_seq_stride, int64_t q_
     return SVA_OK;
   }
   // one token of one sequence at D = R = 64: the decode form
-  const bool aligned = ((uintptr_t)q_proj & 15u) == 0 && ((uintptr_t)codebooks & 15u) == 0 &&
-                       (!sample || (((uintptr_t)codes & 15u) == 0 && code_head_stride % 16 == 0));
+  const bool aligned = ((uintptr_t)q_proj & 15u) == 0 && ((uintptr_t)codebooks & 15u) == 0;
   const int64_t word_room = S == 4   ? (int64_t)QD_WIDE * qd_words<4, QD_WIDE>()
                             : S == 2 ? (int64_t)QD_WIDE * qd_words<2, QD_WIDE>()
                                      : (int64_t)QD * qd_words<1>();  // sampled 16-byte words the form holds

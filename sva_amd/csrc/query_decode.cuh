@@ -8,9 +8,10 @@
 namespace sva {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(1)));  // at any address
 
-// Decode form (one token of one sequence, D = R = 64, uint8 codes, 16-byte
-// aligned code rows, 1x256, 2x256 or 4x64 codes): one 256-thread workgroup per
+// Decode form (one token of one sequence, D = R = 64, uint8 codes at any
+// address, 1x256, 2x256 or 4x64 codes): one 256-thread workgroup per
 // head with the layout's sizes at compile time.  The same arithmetic as query_lut_kernel (q_low and
 // table entries by sequential fma chains, bounds folded per subspace, the
 // floor from the same sample blocks and histogram), with the sampled code
@@ -91,7 +92,7 @@ SVA_DEV void query_decode_item(const LutParams& p, int h) {
       const int gw = smp ? min(t + i * NT, n_words - 1) : 0;
       const int b = gw / (2 * S), wi = gw % (2 * S);
       const int64_t n0 = smp ? ((int64_t)b * (N - SAMPLE_KEYS) / (nb - 1)) & ~(int64_t)15 : 0;
-      words[i] = *reinterpret_cast<const u32x4_t*>(head + n0 * S + wi * 16);
+      words[i] = *reinterpret_cast<const u32x4_any_t*>(head + n0 * S + wi * 16);
     }
   }
   const float sc = p.scale[h];

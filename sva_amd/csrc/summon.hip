@@ -385,19 +385,24 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
   // a prepared query launch (the tables this call reads): the code-class
   // path runs its decode form in one grid with the code counts; every other
   // path launches it first
-  const bool class_path = n_keys > 0 && sva::summon_class_eligible(p, items);
-  SVA_REQUIRE(stats == nullptr || (n_keys > 0 && !class_path && !sva::summon_wide_eligible(p, items) &&
-                                   sva::summon_regs_eligible(p)),
+  // (code heads off 16-byte addresses took the per-item path, which needs no
+  // workspace, before the wide kernels read codes at any address: a call
+  // whose workspace is short still takes it)
+  const bool code16 = ((uintptr_t)codes & 15u) == 0 && code_head_stride % 16 == 0;
+  const bool room = code16 || (workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
+                               workspace_bytes >= sva::summon_wide_workspace_bytes(n_seq, H, Q, n_keys, L));
+  const bool wide_path = n_keys > 0 && room && sva::summon_wide_eligible(p, items);
+  const bool class_path = wide_path && sva::summon_class_eligible(p, items);
+  SVA_REQUIRE(stats == nullptr || (n_keys > 0 && !wide_path && sva::summon_regs_eligible(p)),
               "%s: a statistics row is added on the per-item register path only", fn);
   // without shortlist outputs only the fused per-item path (strategy 3) runs
   SVA_UNSUPPORTED(sl_idx != nullptr || n_keys == 0 ||
-                      (B > 0 && !class_path && !sva::summon_wide_eligible(p, items) && sva::summon_regs_eligible(p)),
+                      (B > 0 && !wide_path && sva::summon_regs_eligible(p)),
                   "%s: these shapes keep the shortlist in memory; pass shortlist outputs", fn);
   // one token of one sequence on the per-item register path with the
   // verifier: the query, the summon and the verifier in one launch, with a
   // decode step's catalog append in front where that launch can take it
-  const bool item_one_launch = fv != nullptr && fused != nullptr && query != nullptr && n_keys > 0 && !class_path &&
-                               !sva::summon_wide_eligible(p, items);
+  const bool item_one_launch = fv != nullptr && fused != nullptr && query != nullptr && n_keys > 0 && !wide_path;
   if (append != nullptr && !(item_one_launch && sva::item_fused_eligible(p, *query, *fv, append))) {
     // the catalog's new rows on their own, before anything reads them
     const int rc = sva::write_encode_launch(*append, (hipStream_t)stream);
@@ -426,7 +431,7 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
     if (rc == SVA_OK && fused != nullptr) *fused = with_fv;
     return rc;
   }
-  if (sva::summon_wide_eligible(p, items)) {
+  if (wide_path) {
     const bool with_fv = fv != nullptr && sva::fused_verify_eligible(p, items, *fv);
     const int rc = sva::summon_wide_path(p, workspace, workspace_bytes, (hipStream_t)stream, with_fv ? fv : nullptr,
                                          overshoot);

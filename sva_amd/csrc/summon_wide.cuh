@@ -64,6 +64,18 @@ constexpr int64_t kMaxWideItems = 64;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Sixteen bytes of codes at any address.  A head's codes start wherever the
+// catalog's row count puts them (a cache of 100003 keys of two subspaces puts
+// heads 200006 bytes apart), and one global_load_dwordx4 reads them either
+// way, at worst from one more cache line a wave.  Asking for 16-byte aligned
+// heads instead sent every such cache to the per-item path: 579 us a lookup
+// of 100003 keys (2x256, 512 / 128) against 58 here.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+SVA_DEV u32x4 code_word(const uint8_t* c) { return *reinterpret_cast<const u32x4_any*>(c); }
+SVA_DEV u32x4 code_word_nt(const uint8_t* c) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(c));
+}
+
 // The fields a finish workgroup needs for its first loads lead the argument
 // block, so that they share the scalar-cache lines its first loads fetch.
 struct WideArgs {
@@ -107,14 +119,14 @@ SVA_DEV void load_chunk(const uint8_t* __restrict__ codes, int cs, int ce, u32x4
 #pragma unroll
     for (int r = 0; r < RND; ++r) {
       const int base = round_key<S>(cs, r);
-      raw[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(codes + (int64_t)base * S));
+      raw[r] = code_word_nt(codes + (int64_t)base * S);
     }
   } else {
 #pragma unroll
     for (int r = 0; r < RND; ++r) {
       const int base = round_key<S>(cs, r);
       if (base + KPT <= ce) {
-        raw[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(codes + (int64_t)base * S));
+        raw[r] = code_word_nt(codes + (int64_t)base * S);
       } else {
         uint32_t wv[4] = {0u, 0u, 0u, 0u};
         for (int j = 0; j < KPT * S; ++j)
@@ -1180,7 +1192,7 @@ SVA_DEV void overshoot_visit(const SummonParams& p, const uint8_t* __restrict__ 
     for (int u = 0; u < kOverWords; ++u) {
       const int base = (w0 + u * SB + (int)threadIdx.x) * KPW;
       if (base + KPW <= n1) {
-        w[u] = *reinterpret_cast<const u32x4*>(codes + (int64_t)base * S);
+        w[u] = code_word(codes + (int64_t)base * S);
       } else {
         uint32_t wv[4] = {0u, 0u, 0u, 0u};
         for (int j = 0; j < KPW * S; ++j)
@@ -2000,7 +2012,7 @@ struct ClassArgs {
 SVA_DEV void class_load(const uint8_t* __restrict__ codes, int k0, int ce, u32x4 (&raw)[4]) {
   if (k0 + CK_PT <= ce) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) raw[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(codes + k0 + 16 * r));
+    for (int r = 0; r < 4; ++r) raw[r] = code_word_nt(codes + k0 + 16 * r);
   } else {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

@@ -28,7 +28,6 @@ bool summon_wide_eligible(const SummonParams& p, int64_t items) {
   if (p.S != 1 && p.S != 2 && p.S != 4 && p.S != 8) return false;
   if (p.R != 64 || p.N < kWideMinKeys || p.N >= (1ll << 30) || items > kMaxWideItems) return false;
   if (p.L > FIN_MAX_L) return false;
-  if (((uintptr_t)p.codes & 15u) != 0 || p.code_hs % 16 != 0) return false;
   if (((uintptr_t)p.k_low & 15u) != 0 || p.klow_hs % 4 != 0 || ((uintptr_t)p.q_low & 15u) != 0) return false;
   if (p.mask_type != MASK_NONE && p.mask_type != MASK_BOOL && p.mask == nullptr) return false;
   return true;

@@ -71,6 +71,36 @@ def test_wide_matches_oracle(device, N, S, C):
     _check(codes, k_low, *res, 2048)
 
 
+@pytest.mark.parametrize("N,S,C,lead", [(32771, 2, 256, 0), (65537, 4, 64, 1), (49999, 1, 256, 0), (40005, 8, 32, 3),
+                                        (100003, 2, 256, 5)])
+def test_wide_codes_at_any_address(device, N, S, C, lead):
+    """Heads of N * S bytes of codes behind `lead` keys: no 16-byte address; the lookup with its verifier
+    equals the same codes held in aligned rows, bit for bit, and the oracle's shortlist and budget."""
+    from sva_amd import kernels
+
+    H, L, B = 9, 512, 128
+    codes, k_low, q, q_proj, scale, cb = _setup(device, N, S, C, seed=N % 71)
+    g = torch.Generator(device=device).manual_seed(3)
+    keys = torch.randn(3, N, 64, device=device, generator=g).to(torch.float16)
+    values = torch.randn(3, N, 64, device=device, generator=g).to(torch.float16)
+    t = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    odd = torch.zeros(H, N + lead, S, device=device, dtype=torch.uint8)[:, lead:]
+    odd.copy_(t(codes))
+    even = torch.zeros(H, (N + 15) // 16 * 16, S, device=device, dtype=torch.uint8)
+    even[:, :N] = t(codes)
+    assert odd.stride(0) % 16 != 0 or odd.data_ptr() % 16 != 0
+    outs = []
+    for c in (odd, even):
+        plan = kernels.ScanDecodePlan(device, 1, H, 1, 64, 64, S, C, L, B)
+        out = torch.empty(1, H, 1, 64, device=device, dtype=torch.float32)
+        plan.run(t(q)[None].half(), t(q_proj), t(scale), t(cb), c, k_low, keys, values, N, 0.125, out=out)
+        torch.cuda.synchronize()
+        outs.append([x.clone() for x in (out, plan.fin_idx, plan.counts[:2], plan.sl_rank.sort(-1).values)])
+        _check_decode_step(plan, codes, k_low, t(q)[None].half(), keys, values, out, L, B)
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def test_wide_massive_ties_and_repeat(device):
     # 3 codewords: the threshold bin holds ~1/9 of all keys; exact resolution
     N, S, C = 120000, 2, 256
