@@ -142,7 +142,7 @@ extern "C" int sva_decode_layer_step(sva_decode_layer* h, const void* q, int q_d
   // sampled floor (strategy 1 and 2) report overshoots, so the per-item path
   // is spared the fill of that row
   const int64_t H = h->H;
-  const int strategy = sva_summon_strategy(1, H, 1, n_keys, h->R, h->S, h->C, h->L, h->code_type, 0);
+  const int strategy = sva::summon_strategy(1, H, 1, n_keys, h->R, h->S, h->C, h->L, h->code_type, 0);
   const bool with_floor = strategy == 1 || strategy == 2;
   // the per-item register path adds the statistics itself (one launch fewer)
   unsigned long long* fused_stats = strategy == 3 ? (unsigned long long*)h->stats : nullptr;

@@ -101,6 +101,10 @@ struct FusedVerify {
   int64_t o_hs;
 };
 
+// The route of a call with these shapes (sva_summon_strategy's values, 1 and
+// 2 also below its 32768 keys).
+int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S, int64_t C, int64_t L,
+                    int code_type, int mask_type);
 int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream);
 bool summon_regs_eligible(const SummonParams& p);
 int summon_regs_path(const SummonParams& p, int64_t items, hipStream_t stream);

@@ -298,9 +298,11 @@ int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream) {
 
 }  // namespace sva
 
-extern "C" int sva_summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S,
-                                   int64_t C, int64_t L, int code_type, int mask_type) {
-  sva::SummonParams p{};
+namespace sva {
+
+int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S, int64_t C,
+                    int64_t L, int code_type, int mask_type) {
+  SummonParams p{};
   alignas(16) static const float dummy[4] = {0, 0, 0, 0};
   p.codes = dummy;
   p.ctype = code_type;
@@ -315,10 +317,18 @@ extern "C" int sva_summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t 
   p.L = (int)L;
   p.mask = dummy;
   p.mask_type = mask_type;
-  if (sva::summon_class_eligible(p, n_seq * H * Q)) return 2;
-  if (sva::summon_wide_eligible(p, n_seq * H * Q)) return 1;
+  if (summon_class_eligible(p, n_seq * H * Q)) return 2;
+  if (summon_wide_eligible(p, n_seq * H * Q)) return 1;
   p.B = 1;
-  return sva::summon_regs_eligible(p) ? 3 : 0;
+  return summon_regs_eligible(p) ? 3 : 0;
+}
+
+}  // namespace sva
+
+extern "C" int sva_summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S,
+                                   int64_t C, int64_t L, int code_type, int mask_type) {
+  const int st = sva::summon_strategy(n_seq, H, Q, n_keys, R, S, C, L, code_type, mask_type);
+  return n_keys < 32768 && (st == 1 || st == 2) ? 0 : st;
 }
 
 extern "C" size_t sva_summon_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L) {
@@ -387,9 +397,9 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
   // path launches it first
   // (code heads off 16-byte addresses took the per-item path, which needs no
   // workspace, before the wide kernels read codes at any address: a call
-  // whose workspace is short still takes it)
+  // whose workspace is short still takes it; so do caches below 32768 keys)
   const bool code16 = ((uintptr_t)codes & 15u) == 0 && code_head_stride % 16 == 0;
-  const bool room = code16 || (workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
+  const bool room = (code16 && n_keys >= 32768) || (workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
                                workspace_bytes >= sva::summon_wide_workspace_bytes(n_seq, H, Q, n_keys, L));
   const bool wide_path = n_keys > 0 && room && sva::summon_wide_eligible(p, items);
   const bool class_path = wide_path && sva::summon_class_eligible(p, items);

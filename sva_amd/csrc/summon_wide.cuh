@@ -4,7 +4,8 @@
 // workgroups for the rare all-keys select); two kernels, no workgroup ever
 // waits for another.
 //
-//   wide_scan     one workgroup per chunk of WB * 32 keys.  Loads the item's
+//   wide_scan     one workgroup per chunk of WB * KP keys (KP = 8, 16 or 32 a
+//                 thread, scan_keys_per_thread).  Loads the item's
 //                 table and floor (sva_query_lut's outputs) first, then
 //                 streams the chunk's packed uint8 codes (16-byte loads, all
 //                 in flight before use), scores every key through the table
@@ -47,9 +48,7 @@ namespace wide {
 
 constexpr int WB = 256;          // threads per scan workgroup
 constexpr int NW = WB / WAVE;    // waves per scan workgroup
-constexpr int KEYS_PT = 32;      // keys per scan thread
-constexpr int CHUNK = WB * KEYS_PT;
-constexpr int WAVE_KEYS = WAVE * KEYS_PT;  // keys (and candidate capacity) per wave
+constexpr int MAX_KP = 32;       // keys per scan thread: KP = 8, 16 or 32
 constexpr int SB = 1024;         // threads of the select kernel
 constexpr int SNW = SB / WAVE;
 constexpr int LDS_CAND = 16384;  // candidates the finish kernel stages in LDS
@@ -58,8 +57,9 @@ constexpr int STAGE_LISTS = 4096;  // lists whose staging offsets the finish ker
 // 0.125 exactly (both are the correctly rounded value of x / 8).
 constexpr float kInvSqrtR = 0.125f;
 constexpr int KL_CAP = 256;      // candidates per scan wave kept in LDS (composite and rank)
-constexpr int WG_CAP = 128;      // candidates of a scan workgroup in its compact list
-constexpr int64_t kWideMinKeys = 32768;
+constexpr int WG_CAP = 128;      // candidates of a scan workgroup in its compact list (at least: wg_cap)
+constexpr uint32_t kNoCompact = 0x80000000u;  // wg_count flag: the workgroup wrote no compact list
+constexpr int64_t kWideMinKeys = 16385;  // caches past the register path's 16384 keys
 constexpr int64_t kMaxWideItems = 64;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -81,14 +81,18 @@ SVA_DEV u32x4 code_word_nt(const uint8_t* c) {
 struct WideArgs {
   int W;               // scan workgroups per item
   int items;           // items of the call
-  uint32_t* wg_count;  // [items, W, 2] candidates and allowed keys of each scan workgroup
-  uint64_t* wg_cand;   // [items, W, WG_CAP] a workgroup's candidates in key order (when they fit)
-  float* wg_rank;      // [items, W, WG_CAP] their rank scores
+  int cap;             // entries of a compact list (wg_cap(W))
+  int span_log2;       // lists per item rounded up to a power of two (list_span(W))
+  int wave_keys;       // keys of a scan wave (64 KP), the capacity of its own list
+  int groups, per;     // KV groups the fused finish is laid out by and their heads (0: not grouped)
+  uint32_t* wg_count;  // [items, W, 2] candidates (or kNoCompact) and allowed keys of each scan workgroup
+  uint64_t* wg_cand;   // [items, W, cap] a workgroup's candidates in key order (when they fit)
+  float* wg_rank;      // [items, W, cap] their rank scores
   SummonParams p;
   uint32_t* ncand;   // [items, W * NW] candidates of each scan wave
   uint32_t* nallow;  // [items, W * NW] allowed keys of each scan wave
-  uint64_t* cand;    // [items, W * NW, WAVE_KEYS] candidate composites of each scan wave
-  float* cand_rank;  // [items, W * NW, WAVE_KEYS] rank score of each listed candidate
+  uint64_t* cand;    // [items, W * NW, wave_keys] candidate composites of each scan wave
+  float* cand_rank;  // [items, W * NW, wave_keys] rank score of each listed candidate
   FusedVerify fv;    // fv.out != nullptr: the finish kernel also runs the verifier
   int32_t* overshoot;  // [items] or nullptr: 1 where the sampled floor overshot (all-keys select), else 0
   int K;               // slices of the all-keys select per item (finish grid: items * K workgroups)
@@ -100,31 +104,32 @@ struct WideArgs {
 SVA_DEV uint32_t byte_of(const u32x4& v, int j) { return (v[j >> 2] >> (8 * (j & 3))) & 0xFFu; }
 
 // First key of round r of the calling lane: wave w of the workgroup owns keys
-// [cs + w * WAVE_KEYS, cs + (w + 1) * WAVE_KEYS), and in round r its lanes
-// take consecutive groups of 16 / S keys (one 16-byte word of codes each).
-template <int S>
+// [cs + w * 64 KP, cs + (w + 1) * 64 KP), and in round r its lanes take
+// consecutive groups of 16 / S keys (one 16-byte word of codes each).
+template <int S, int KP>
 SVA_DEV int round_key(int cs, int r) {
   constexpr int KPT = 16 / S;
-  return cs + (int)(threadIdx.x / WAVE) * WAVE_KEYS + (r * WAVE + lane_id()) * KPT;
+  return cs + (int)(threadIdx.x / WAVE) * (WAVE * KP) + (r * WAVE + lane_id()) * KPT;
 }
 
 // Loads a chunk's codes: a full chunk (FULL) with one unconditional vector
 // load per 16-byte group, straight-line so that each round waits only for
 // its own load; a partial last chunk falls back to guarded byte loads.
-template <int S, bool FULL>
-SVA_DEV void load_chunk(const uint8_t* __restrict__ codes, int cs, int ce, u32x4 (&raw)[KEYS_PT * S / 16]) {
+template <int S, int KP, bool FULL>
+SVA_DEV void load_chunk(const uint8_t* __restrict__ codes, int cs, int ce, u32x4 (&raw)[KP * S / 16]) {
   constexpr int KPT = 16 / S;
-  constexpr int RND = KEYS_PT / KPT;
+  constexpr int RND = KP / KPT;
+  static_assert(KP % KPT == 0, "whole code words per thread");
   if (FULL) {
 #pragma unroll
     for (int r = 0; r < RND; ++r) {
-      const int base = round_key<S>(cs, r);
+      const int base = round_key<S, KP>(cs, r);
       raw[r] = code_word_nt(codes + (int64_t)base * S);
     }
   } else {
 #pragma unroll
     for (int r = 0; r < RND; ++r) {
-      const int base = round_key<S>(cs, r);
+      const int base = round_key<S, KP>(cs, r);
       if (base + KPT <= ce) {
         raw[r] = code_word_nt(codes + (int64_t)base * S);
       } else {
@@ -242,10 +247,10 @@ SVA_DEV void score_round(const u32x4& raw, const ScanTables<S, SMALLC>& T, float
 }
 
 // Key index of slot i of this thread in the chunk starting at cs.
-template <int S>
+template <int S, int KP>
 SVA_DEV int slot_key(int cs, int i) {
   constexpr int KPT = 16 / S;
-  return round_key<S>(cs, i / KPT) + (i % KPT);
+  return round_key<S, KP>(cs, i / KPT) + (i % KPT);
 }
 
 template <bool FULL, bool MASKED>
@@ -310,12 +315,12 @@ SVA_DEV void append_round(const SummonParams& p, const bool (&c)[KPT], const flo
 // together rather than each behind the branch of the round before (eight
 // subspaces keep the per-round order: holding every round's sums would cost
 // them a wave per SIMD).
-template <int S, bool SMALLC, bool CHECK, bool MASKED>
-SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KEYS_PT * S / 16], const ScanTables<S, SMALLC>& T,
+template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED>
+SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16], const ScanTables<S, SMALLC>& T,
                          float t_lo, int cs, int ce, uint64_t* out, uint64_t* kc, uint32_t& wc,
                          uint32_t& n_allowed) {
   constexpr int KPT = 16 / S;
-  constexpr int RND = KEYS_PT / KPT;
+  constexpr int RND = KP / KPT;
   constexpr bool ALL_FIRST = !CHECK && S <= 4;
   if (ALL_FIRST) {
     float acc[RND][KPT];
@@ -335,7 +340,7 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KEYS_PT * S /
         bool c[KPT];
 #pragma unroll
         for (int k = 0; k < KPT; ++k) c[k] = acc[r][k] >= t_lo;
-        append_round<KPT>(p, c, acc[r], round_key<S>(cs, r), out, kc, wc);
+        append_round<KPT>(p, c, acc[r], round_key<S, KP>(cs, r), out, kc, wc);
       }
     }
   } else {
@@ -348,12 +353,12 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KEYS_PT * S /
         bool any = false;
 #pragma unroll
         for (int k = 0; k < KPT; ++k) {
-          const bool ok = key_ok<false, MASKED>(p, slot_key<S>(cs, r * KPT + k), ce);
+          const bool ok = key_ok<false, MASKED>(p, slot_key<S, KP>(cs, r * KPT + k), ce);
           n_allowed += ok;
           c[k] = ok && acc[k] >= t_lo;
           any = any || c[k];
         }
-        if (__builtin_amdgcn_ballot_w64(any) != 0ull) append_round<KPT>(p, c, acc, round_key<S>(cs, r), out, kc, wc);
+        if (__builtin_amdgcn_ballot_w64(any) != 0ull) append_round<KPT>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
       } else {
         float mx = acc[0];
 #pragma unroll
@@ -362,12 +367,12 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KEYS_PT * S /
           bool c[KPT];
 #pragma unroll
           for (int k = 0; k < KPT; ++k) c[k] = acc[k] >= t_lo;
-          append_round<KPT>(p, c, acc, round_key<S>(cs, r), out, kc, wc);
+          append_round<KPT>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
         }
       }
     }
   }
-  if (!CHECK) n_allowed = KEYS_PT;
+  if (!CHECK) n_allowed = KP;
 }
 
 // Rank scores of a scan wave's nc candidates (composites in the LDS list
@@ -435,32 +440,32 @@ struct ScanLds {
   uint32_t wcnt[NW], walw[NW];
 };
 
-template <int S, bool SMALLC, bool CHECK, bool MASKED>
+template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED>
 SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, ScanLds& L) {
 #pragma clang fp contract(off)
   const SummonParams& p = a.p;
   const int h = item % p.H;
-  const int cs = w * CHUNK;
-  const int ce = (int)min((int64_t)cs + CHUNK, p.N);
+  const int cs = w * (WB * KP);
+  const int ce = (int)min((int64_t)cs + WB * KP, p.N);
   const uint8_t* codes = (const uint8_t*)p.codes + (int64_t)h * p.code_hs;
   ScanTables<S, SMALLC> T;
   T.load(p, item);
   const float t_lo = item_floor(p, item);
   const float4 qq = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * p.R)[lane_id() & 15];
-  u32x4 raw[KEYS_PT * S / 16];
-  load_chunk<S, !CHECK>(codes, cs, ce, raw);
+  u32x4 raw[KP * S / 16];
+  load_chunk<S, KP, !CHECK>(codes, cs, ce, raw);
   T.store(tab_lds);
   __syncthreads();  // tables in LDS
   const int wid = threadIdx.x / WAVE;
   const int lane = lane_id();
   const int64_t sub = ((int64_t)item * a.W + w) * NW + wid;
-  uint64_t* out = a.cand + sub * WAVE_KEYS;
-  float* out_rank = a.cand_rank + sub * WAVE_KEYS;
+  uint64_t* out = a.cand + sub * (WAVE * KP);
+  float* out_rank = a.cand_rank + sub * (WAVE * KP);
   uint32_t n_allowed = 0;
   uint32_t wc = 0;  // candidates of this wave so far (wave-uniform)
-  scan_rounds<S, SMALLC, CHECK, MASKED>(p, raw, T, t_lo, cs, ce, out, L.kc[wid], wc, n_allowed);
+  scan_rounds<S, KP, SMALLC, CHECK, MASKED>(p, raw, T, t_lo, cs, ce, out, L.kc[wid], wc, n_allowed);
   rank_candidates(p, item, qq, L.kc[wid], L.kr[wid], out, out_rank, wc);
-  const uint32_t wa = CHECK ? wave_sum_dpp(n_allowed) : (uint32_t)(WAVE * KEYS_PT);  // every key allowed
+  const uint32_t wa = CHECK ? wave_sum_dpp(n_allowed) : (uint32_t)(WAVE * KP);  // every key allowed
   if (lane == 0) {
     a.ncand[sub] = wc;
     a.nallow[sub] = wa;
@@ -468,21 +473,24 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, Scan
     L.walw[wid] = wa;
   }
   // the workgroup's compact list: its waves' candidates in wave order (key
-  // order), when there are at most WG_CAP of them (else each wave's LDS part
+  // order), when there are at most cap of them (else each wave's LDS part
   // completes its global list); its counts either way
   __syncthreads();
   uint32_t off = 0, tot = 0, alw = 0;
+  bool fits = true;  // every wave's candidates are in LDS
 #pragma unroll
   for (int v = 0; v < NW; ++v) {
     off += v < wid ? L.wcnt[v] : 0u;
     tot += L.wcnt[v];
     alw += L.walw[v];
+    fits = fits && L.wcnt[v] <= (uint32_t)KL_CAP;
   }
+  fits = fits && tot <= (uint32_t)a.cap;
   const int64_t g = (int64_t)item * a.W + w;
-  if (tot <= (uint32_t)WG_CAP) {
+  if (fits) {
     for (uint32_t j = (uint32_t)lane; j < wc; j += WAVE) {
-      a.wg_cand[g * WG_CAP + off + j] = L.kc[wid][j];
-      a.wg_rank[g * WG_CAP + off + j] = L.kr[wid][j];
+      a.wg_cand[g * a.cap + off + j] = L.kc[wid][j];
+      a.wg_rank[g * a.cap + off + j] = L.kr[wid][j];
     }
   } else {
     const uint32_t nl = min(wc, (uint32_t)KL_CAP);
@@ -492,14 +500,50 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, Scan
     }
   }
   if (threadIdx.x == 0) {
-    a.wg_count[2 * g] = tot;
+    a.wg_count[2 * g] = fits ? tot : kNoCompact;
     a.wg_count[2 * g + 1] = alw;
   }
 }
 
+// Keys per scan thread of a call over `items` items of up to n_keys keys: the
+// largest of 32, 16 and 8 (a code word of one subspace holds 16 keys; eight
+// subspaces and masked calls have the one form of 32) that gives the chip
+// about four workgroups a CU and keeps the usual 4096 candidates of an item
+// to 64 a workgroup (W >= 64), so that the finish places a compact list with
+// one load a wave, while the lists stay within the fast finish's 256.  A
+// million keys and nine heads keep 32 (1152 workgroups); shorter caches left
+// the chip idle (100003 keys: 117 workgroups of 8192 keys, 441 of 2048) and
+// overflowed the compact lists into the finish's slower paths (4096
+// candidates over 13 lists of 128): 58 us a lookup against 32.
+inline int scan_keys_per_thread(int64_t items, int64_t n_keys, int S, bool masked) {
+  if (S == 8 || masked) return MAX_KP;
+  int kp = MAX_KP;
+  while (kp > (S == 1 ? 16 : 8)) {
+    const int64_t W = (n_keys + WB * kp - 1) / (WB * kp);
+    if ((W >= 64 && items * W >= 1024) || 2 * W > 256) break;
+    kp /= 2;
+  }
+  return kp;
+}
+
+// Entries of a compact list when an item has W of them: with few workgroups
+// an item each holds more of its candidates.  The finish's first loads cover
+// 8192 entries of all lists together (finish_fast); the lists hold twice that
+// (about four times the usual candidates), each at least WG_CAP and at most
+// what the scan's waves keep in LDS.
+__host__ __device__ inline int list_span(int W) {  // W rounded up to a power of two
+  int p = 1;
+  while (p < W) p <<= 1;
+  return p;
+}
+__host__ __device__ inline int wg_cap(int W) {
+  const int c = 16384 / list_span(W);
+  return c < WG_CAP ? WG_CAP : (c > NW * KL_CAP ? NW * KL_CAP : c);
+}
+
 // Five workgroups per CU (at most 102 VGPRs) keep every workgroup of a
 // million-key, nine-head scan resident at once (up to four subspaces).
-template <int S, bool SMALLC, bool MASKED>
+template <int S, int KP, bool SMALLC, bool MASKED>
 __global__ void __launch_bounds__(WB, S <= 4 ? 5 : 1) wide_scan_kernel(WideArgs a) {
   __shared__ __align__(16) float tab_lds[ScanTables<S, SMALLC>::LDS_FLOATS];
   __shared__ ScanLds lds;
@@ -507,10 +551,10 @@ __global__ void __launch_bounds__(WB, S <= 4 ? 5 : 1) wide_scan_kernel(WideArgs 
   const int w = blockIdx.x % a.W;
   if (blockIdx.x == 0)  // arrival counters of the finish kernel's all-keys select
     for (int i = threadIdx.x; i < a.items; i += WB) a.arrive[i] = 0u;
-  if (!MASKED && (int64_t)(w + 1) * CHUNK <= a.p.N) {
-    scan_chunk<S, SMALLC, false, false>(a, item, w, tab_lds, lds);
+  if (!MASKED && (int64_t)(w + 1) * (WB * KP) <= a.p.N) {
+    scan_chunk<S, KP, SMALLC, false, false>(a, item, w, tab_lds, lds);
   } else {
-    scan_chunk<S, SMALLC, true, MASKED>(a, item, w, tab_lds, lds);
+    scan_chunk<S, KP, SMALLC, true, MASKED>(a, item, w, tab_lds, lds);
   }
 }
 
@@ -614,7 +658,7 @@ SVA_DEV void finish_budget(const SummonParams& p, int item, int leff, int beff, 
 // lists k * DQ + q of `src` (entries past a list's count are read but
 // unused; every read stays inside the list's capacity).
 template <int DH, typename T>
-SVA_DEV void gather_lists(const T* src, int nsub, T (&v)[DH * DK]) {
+SVA_DEV void gather_lists(const T* src, int nsub, int wave_keys, T (&v)[DH * DK]) {
   const int q = threadIdx.x >> 4, l = threadIdx.x & 15;
   const int kq = (nsub + DQ - 1) / DQ;
 #pragma unroll
@@ -622,7 +666,7 @@ SVA_DEV void gather_lists(const T* src, int nsub, T (&v)[DH * DK]) {
 #pragma unroll
     for (int h = 0; h < DH; ++h) v[DH * k + h] = T(0);
     if (k < kq) {  // uniform
-      const int64_t off = (int64_t)min(k * DQ + q, nsub - 1) * WAVE_KEYS + l;
+      const int64_t off = (int64_t)min(k * DQ + q, nsub - 1) * wave_keys + l;
 #pragma unroll
       for (int h = 0; h < DH; ++h) v[DH * k + h] = src[off + 16 * h];
     }
@@ -668,7 +712,7 @@ SVA_DEV void finish_dense(const WideArgs& a, int item, int nsub, int leff, int b
   const SummonParams& p = a.p;
   const int dslots = ((int)M + SB - 1) / SB;
   float r_sp[DH * DK];
-  gather_lists<DH>(a.cand_rank + (int64_t)item * nsub * WAVE_KEYS, nsub, r_sp);
+  gather_lists<DH>(a.cand_rank + (int64_t)item * nsub * a.wave_keys, nsub, a.wave_keys, r_sp);
   uint64_t e[NPD];
   densify<DH>(e_sp, e, (uint64_t*)stage, lcnt, loff, nsub, dslots, M);
   // shortlist: the leff largest score composites
@@ -740,7 +784,8 @@ constexpr size_t kFastEnd = kFastMisc + sizeof(uint32_t) * 96;
 constexpr size_t kFastRHist = kFastComp;                                      // uint32[4096]
 constexpr size_t kFastSmallR = kFastRHist + sizeof(uint32_t) * 4096;          // float[SMALL_CAP]
 static_assert(kFastSmallR + sizeof(float) * SMALL_CAP <= kFastRank, "budget histogram over the staged composites");
-static_assert(WG_CAP == 2 * WAVE, "two compact-list entries per lane");
+static_assert(SNW * FAST_BATCH * WAVE == 8192, "wg_cap: entries the first loads cover");
+static_assert(kWideMinKeys > 2 * WB * MAX_KP, "at least three lists an item (list l and wave wid agree modulo four)");
 static_assert(kFastEnd <= kFinStage, "the fast finish stays inside the finish kernel's staging area");
 
 // Exclusive scan within a wave (all 64 lanes active).
@@ -889,8 +934,8 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
   if (W > FAST_LISTS) return false;
   const int t = threadIdx.x;
   const int lane = lane_id();
-  const int wid = t / WAVE;
-  const int64_t g0 = (int64_t)item * W;
+  const int wid = __builtin_amdgcn_readfirstlane(t / WAVE);  // list addresses on the scalar unit
+  const int g0 = __builtin_amdgcn_readfirstlane(item) * W;
   // Every load below is issued unconditionally (indices clamped to the last
   // list, values past it ignored): a load under a condition leaves the
   // compiler unsure how many loads follow an earlier one, and it then waits
@@ -900,20 +945,40 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int l = min(4 * lane + i, W - 1);
-    cnt_raw[i] = a.wg_count[2 * (g0 + l)];
-    alw_raw[i] = a.wg_count[2 * (g0 + l) + 1];
+    const uint32_t* wc = a.wg_count + 2 * (int64_t)g0;
+    cnt_raw[i] = wc[2 * l];
+    alw_raw[i] = wc[2 * l + 1];
   }
-  // the first round of this wave's lists (16 k + wid, k < FAST_BATCH), issued
-  // with the counts: the first WAVE slots of each list (a list's later slots,
-  // rarely filled, are requested after every list's first slots are placed)
+  __builtin_amdgcn_sched_barrier(0);  // loads return in order: the counts, used first, go first
+  // the first round of this wave's segments, issued with the counts.  A
+  // segment is WAVE slots of a list.  From 16 lists up (span: W rounded up to
+  // a power of two) wave wid takes the first nseg segments of lists
+  // 16 i + wid: one segment of eight lists where there are 128 lists or more
+  // (further lists in later rounds), more segments of fewer lists otherwise;
+  // below 16 lists 16 / span waves share one.  Slots past a list's nseg
+  // segments, rarely filled, are requested after every segment is placed.
+  const int cap = a.cap;
+  constexpr int LG_NW = 4, LG_FB = 3;
+  static_assert(SNW == 1 << LG_NW && FAST_BATCH == 1 << LG_FB, "list and segment numbers by shifts");
+  const int lg = a.span_log2;
+  const int nseg = 1 << max(LG_NW + LG_FB - lg, 0);     // segments of a list in the first round
+  const int pl = min(max(LG_NW + LG_FB - lg, 0), LG_FB);  // log2 of those of them that are one wave's
+  const int w0 = wid & ((1 << min(lg, LG_NW)) - 1);     // the wave's first list
+  const int s0 = lg < LG_NW ? (wid >> lg) << LG_FB : 0;  // and its first segment there
   uint64_t comp[FAST_BATCH];
   float rank[FAST_BATCH];
+  auto seg_of = [&](int r, int k, int& l, int& seg) {
+    l = (((r << (LG_FB - pl)) + (k >> pl)) << LG_NW) + w0;
+    seg = s0 + (k & ((1 << pl) - 1));
+  };
   auto load_round = [&](int r) {
 #pragma unroll
     for (int k = 0; k < FAST_BATCH; ++k) {
-      const int l = min(SNW * (r * FAST_BATCH + k) + wid, W - 1);
-      comp[k] = a.wg_cand[(g0 + l) * WG_CAP + lane];
-      rank[k] = a.wg_rank[(g0 + l) * WG_CAP + lane];
+      int l, seg;
+      seg_of(r, k, l, seg);
+      const int64_t at = (int64_t)(g0 + min(l, W - 1)) * cap + min(seg * WAVE, cap - WAVE);
+      comp[k] = (a.wg_cand + at)[lane];
+      rank[k] = (a.wg_rank + at)[lane];
     }
   };
   load_round(0);
@@ -935,7 +1000,7 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
     asum += in ? alw_raw[i] : 0u;
     loc[i] = lsum;
     lsum += tot[i];
-    over = over || tot[i] > (uint32_t)WG_CAP;
+    over = over || tot[i] == kNoCompact;
   }
   const uint32_t M = wave_sum_dpp(lsum), A = wave_sum_dpp(asum);
   const bool overflow = __builtin_amdgcn_ballot_w64(over) != 0ull;
@@ -953,7 +1018,7 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
   uint64_t* small = (uint64_t*)(lds + kFastSmall);
   const FastMisc f{(uint32_t*)(lds + kFastMisc)};
   const uint32_t base = wave_excl_scan(lsum);
-  // list 16 k + wid lives in lane (16 k + wid) / 4 at element wid % 4
+  // list l of this wave (l % 4 == wid % 4) lives in lane l / 4 at element wid % 4
   const int el = wid & 3;
   const uint32_t my_off = base + (el == 0 ? loc[0] : el == 1 ? loc[1] : el == 2 ? loc[2] : loc[3]);
   const uint32_t my_tot = el == 0 ? tot[0] : el == 1 ? tot[1] : el == 2 ? tot[2] : tot[3];
@@ -962,31 +1027,32 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
     lcomp[at] = x;
     lrank[at] = rx;
     atomicAdd(&hist[lin_bin(key2f((uint32_t)(x >> 32)), vlo, vinv)], 1u);
-    rkmin = min(rkmin, f2key(rx));
-    rkmax = max(rkmax, f2key(rx));
+    const uint32_t rk = f2key(rx);
+    rkmin = min(rkmin, rk);
+    rkmax = max(rkmax, rk);
   };
-  bool tails = false;  // some list of this wave holds more than WAVE candidates
-  for (int r = 0; r * FAST_BATCH * SNW < W; ++r) {
+  bool tails = false;  // some list of this wave holds more than its nseg segments
+  for (int r = 0; r << (LG_FB - pl + LG_NW) < W; ++r) {
     if (r > 0) load_round(r);
 #pragma unroll
     for (int k = 0; k < FAST_BATCH; ++k) {
-      const int l = SNW * (r * FAST_BATCH + k) + wid;
+      int l, seg;
+      seg_of(r, k, l, seg);
       if (l < W) {  // uniform
-        const int src = l >> 2;
-        const uint32_t o = (uint32_t)__shfl((int)my_off, src, WAVE);
-        const uint32_t c = (uint32_t)__shfl((int)my_tot, src, WAVE);
-        if ((uint32_t)lane < c) place(o + lane, comp[k], rank[k]);
-        tails = tails || c > (uint32_t)WAVE;
+        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)my_off, l >> 2);
+        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)my_tot, l >> 2);
+        const uint32_t j = (uint32_t)(seg * WAVE + lane);
+        if (j < c) place(o + j, comp[k], rank[k]);
+        tails = tails || c > (uint32_t)(nseg * WAVE);
       }
     }
   }
-  if (tails) {  // uniform: the slots past WAVE of this wave's long lists
+  if (tails) {  // uniform: the slots past the first segments of this wave's long lists (16 lists or more)
     for (int l = wid; l < W; l += SNW) {
-      const int src = l >> 2;
-      const uint32_t o = (uint32_t)__shfl((int)my_off, src, WAVE);
-      const uint32_t c = (uint32_t)__shfl((int)my_tot, src, WAVE);
-      for (uint32_t j = WAVE + lane; j < c; j += WAVE)
-        place(o + j, a.wg_cand[(g0 + l) * WG_CAP + j], a.wg_rank[(g0 + l) * WG_CAP + j]);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)my_off, l >> 2);
+      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)my_tot, l >> 2);
+      for (uint32_t j = (uint32_t)(nseg * WAVE + lane); j < c; j += WAVE)
+        place(o + j, a.wg_cand[(int64_t)(g0 + l) * cap + j], a.wg_rank[(int64_t)(g0 + l) * cap + j]);
     }
   }
   wave_min_max_u32(rkmin, rkmax);
@@ -1458,10 +1524,11 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   const int t = threadIdx.x;
   const int lane = lane_id();
   const int nsub = a.W * NW;
+  const int wave_keys = a.wave_keys, cap = a.cap;
   const uint32_t* ncand = a.ncand + (int64_t)item * nsub;
   const uint32_t* nallow = a.nallow + (int64_t)item * nsub;
-  const uint64_t* cand = a.cand + (int64_t)item * nsub * WAVE_KEYS;
-  const float* crank = a.cand_rank + (int64_t)item * nsub * WAVE_KEYS;
+  const uint64_t* cand = a.cand + (int64_t)item * nsub * wave_keys;
+  const float* crank = a.cand_rank + (int64_t)item * nsub * wave_keys;
   int32_t* out_idx = p.sl_idx + (int64_t)item * p.L;
   float* out_rank = p.sl_rank + (int64_t)item * p.L;
   // 1. list counts, their offsets in list order (nsub <= SB), totals:
@@ -1504,22 +1571,22 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   if (leff == 0) return 0;
   if (M >= (uint32_t)leff) {
     // the per-wave lists of scan workgroups that wrote a compact list hold
-    // only candidates past their wave's first KL_CAP (none: a compact list
-    // has at most WG_CAP < KL_CAP entries): copy the compact list back, one
-    // finish wave per scan workgroup
-    static_assert(WG_CAP < KL_CAP && NW == 4, "a compact list covers whole waves of four");
+    // only candidates past their wave's first KL_CAP (none: a compact list is
+    // written only when every wave's candidates fit its LDS list): copy the
+    // compact list back, one finish wave per scan workgroup
+    static_assert(NW == 4, "a compact list covers whole waves of four");
     const int wid = t / WAVE;
     for (int g = wid; g < a.W; g += SNW) {
       const int64_t gg = (int64_t)item * a.W + g;
       const uint32_t tot = a.wg_count[2 * gg];
-      if (tot > (uint32_t)WG_CAP) continue;  // uniform: its per-wave lists are whole
+      if (tot == kNoCompact) continue;  // uniform: its per-wave lists are whole
       const uint32_t p1 = ncand[g * NW], p2 = p1 + ncand[g * NW + 1], p3 = p2 + ncand[g * NW + 2];
       for (uint32_t sidx = (uint32_t)lane; sidx < tot; sidx += WAVE) {
         const int v = (sidx >= p1) + (sidx >= p2) + (sidx >= p3);
         const uint32_t o = v == 0 ? 0u : v == 1 ? p1 : v == 2 ? p2 : p3;
-        const int64_t dst = (gg * NW + v) * WAVE_KEYS + (sidx - o);
-        a.cand[dst] = a.wg_cand[gg * WG_CAP + sidx];
-        a.cand_rank[dst] = a.wg_rank[gg * WG_CAP + sidx];
+        const int64_t dst = (gg * NW + v) * wave_keys + (sidx - o);
+        a.cand[dst] = a.wg_cand[gg * cap + sidx];
+        a.cand_rank[dst] = a.wg_rank[gg * cap + sidx];
       }
     }
     __threadfence();
@@ -1531,11 +1598,11 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   if (M >= (uint32_t)leff && M <= (uint32_t)(NPD * SB) && nsub <= DL_LISTS && longest <= 48u) {
     if (longest <= 32u) {
       uint64_t e_sp[2 * DK];
-      gather_lists<2>(cand, nsub, e_sp);
+      gather_lists<2>(cand, nsub, wave_keys, e_sp);
       finish_dense<2>(a, item, nsub, leff, beff, M, c_lo, c_hi, e_sp, lds, lcnt, loff, rkb, wcnt, scratch, tl);
     } else {
       uint64_t e3[3 * DK];
-      gather_lists<3>(cand, nsub, e3);
+      gather_lists<3>(cand, nsub, wave_keys, e3);
       finish_dense<3>(a, item, nsub, leff, beff, M, c_lo, c_hi, e3, lds, lcnt, loff, rkb, wcnt, scratch, tl);
     }
     return 0;
@@ -1564,7 +1631,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
         const int sidx = k * DQ + q;
         const uint32_t c = sidx < nsub ? lcnt[sidx] : 0u;
         const uint32_t base = sidx < nsub ? loff[sidx] : 0u;
-        const int64_t off = (int64_t)sidx * WAVE_KEYS;
+        const int64_t off = (int64_t)sidx * wave_keys;
         for (uint32_t j = l; j < c; j += 16) cl[base + j] = cand[off + j];
       }
     } else {
@@ -1575,7 +1642,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
         uint32_t tot;
         const uint32_t base = carry + block_excl_scan<SB>(c, scratch, &tot);
         if (sidx < nsub) loff[sidx] = base;
-        const int64_t off = (int64_t)sidx * WAVE_KEYS;
+        const int64_t off = (int64_t)sidx * wave_keys;
         for (uint32_t j = 0; j < c; ++j) cl[base + j] = cand[off + j];
         carry += tot;
       }
@@ -1605,7 +1672,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
           else hi = mid;
         }
         const int sidx = lo - 1;
-        rnk[i] = crank[(int64_t)sidx * WAVE_KEYS + (j - loff[sidx])];
+        rnk[i] = crank[(int64_t)sidx * wave_keys + (j - loff[sidx])];
       }
     }
     compact_ordered<SB, NPT>(e, X, leff, wcnt, scratch, slots,
@@ -1618,7 +1685,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     auto visit = [&](auto&& f) {
       for (int sidx = t; sidx < nsub; sidx += SB) {
         const uint32_t c = ncand[sidx];
-        const uint64_t* src = cand + (int64_t)sidx * WAVE_KEYS;
+        const uint64_t* src = cand + (int64_t)sidx * wave_keys;
         for (uint32_t j = 0; j < c; ++j) f(src[j]);
       }
     };
@@ -1628,7 +1695,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     for (int g = 0; g < nsub; g += SB) {
       const int sidx = g + t;
       const uint32_t c = sidx < nsub ? ncand[sidx] : 0u;
-      const int64_t off = (int64_t)sidx * WAVE_KEYS;
+      const int64_t off = (int64_t)sidx * wave_keys;
       uint32_t cnt = 0;
       for (uint32_t j = 0; j < c; ++j) cnt += cand[off + j] >= X;
       uint32_t tot;
@@ -1927,12 +1994,13 @@ inline size_t verify_item_lds(int B, int D) { return sizeof(float) * ((size_t)B 
 // group's other heads.  The other workgroups take the slices > 0 in turn;
 // without a verifier, or when the groups do not fit, b takes item b % items
 // as slice b / items.
+inline bool finish_grouped(int items, int G, int K) {
+  return G > 0 && G <= 8 && items % G == 0 && G - 1 + 8 * (items / G - 1) < items * K;
+}
 SVA_DEV void finish_slot(const WideArgs& a, int b, int& item, int& slice) {
-  const int items = a.items;
-  const int G = a.fv.out != nullptr ? a.fv.G : 0;
-  const int per = G > 0 ? items / G : 0;  // heads per KV group
-  if (G > 0 && G <= 8 && G * per == items && G - 1 + 8 * (per - 1) < items * a.K) {
-    const int x = b % 8, r = b / 8;
+  const int G = a.groups, per = a.per;
+  if (G > 0) {
+    const int x = b & 7, r = b >> 3;
     if (x < G && r < per) {
       item = x * per + r;
       slice = 0;
@@ -1941,12 +2009,12 @@ SVA_DEV void finish_slot(const WideArgs& a, int b, int& item, int& slice) {
     int before = 0;  // group workgroups with a smaller index
     for (int rr = 0; rr < per; ++rr) before += min(max(b - 8 * rr, 0), G);
     const int o = b - before;
-    item = o % items;
-    slice = 1 + o / items;
+    item = o % a.items;
+    slice = 1 + o / a.items;
     return;
   }
-  item = b % items;
-  slice = b / items;
+  item = b < a.items ? b : b % a.items;  // a finish needs no division
+  slice = b < a.items ? 0 : b / a.items;
 }
 
 // Finish of an item, then (VD > 0: head_dim VD, K / V dtype VKV) its
@@ -1956,6 +2024,10 @@ template <int VD, int VKV>
 __global__ void __launch_bounds__(SB) wide_finish_kernel(WideArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ float qsh[VD > 0 ? VD : 1];  // the verifier's query row
+  // the arguments ahead of the first loads, requested together: taken where
+  // each is used they are four scalar-cache misses in turn
+  asm volatile("" ::"s"(a.W), "s"(a.wg_count), "s"(a.wg_cand), "s"(a.wg_rank), "s"(a.p.range), "s"(a.overshoot));
+  if (VD > 0) asm volatile("" ::"s"(a.fv.q), "s"(a.fv.q_hs), "s"(a.fv.q_dtype));
   int item, slice;
   finish_slot(a, (int)blockIdx.x, item, slice);
   // the query row is requested before the finish starts and parked in LDS
@@ -2283,9 +2355,41 @@ inline size_t over_bytes(int64_t items, int64_t L) {
 }
 inline size_t counters_bytes(int64_t items, int64_t W) {
   return align256((size_t)(2 * items * W * NW) * sizeof(uint32_t)) + align256((size_t)(2 * items * W) * sizeof(uint32_t)) +
-         align256((size_t)(items * W * WG_CAP) * (sizeof(uint64_t) + sizeof(float)));
+         align256((size_t)(items * W * wg_cap((int)W)) * (sizeof(uint64_t) + sizeof(float)));
 }
 
+// the scan waves' own lists (composites, then ranks), kp keys a thread
+inline size_t lists_bytes(int64_t items, int64_t W, int kp) {
+  return align256((size_t)items * (size_t)W * (size_t)(WB * kp) * (sizeof(uint64_t) + sizeof(float)));
+}
+
+// The scan of S-subspace codes, kp keys a thread (kp < MAX_KP: unmasked, S <= 4).
+template <int S, int KP, bool SMALLC, bool MASKED>
+int launch_wide(const WideArgs& a, int64_t items, hipStream_t stream) {
+  hipLaunchKernelGGL((wide_scan_kernel<S, KP, SMALLC, MASKED>), dim3((unsigned)(items * a.W)), dim3(WB), 0, stream, a);
+  SVA_CHECK_LAUNCH("wide_scan_kernel");
+  return SVA_OK;
+}
+
+template <int S>
+int launch_wide_s(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
+  const bool small_c = a.p.C <= 64;
+  if (masked)
+    return small_c ? launch_wide<S, MAX_KP, true, true>(a, items, stream)
+                   : launch_wide<S, MAX_KP, false, true>(a, items, stream);
+  if constexpr (S >= 2 && S <= 4) {
+    if (kp == 8)
+      return small_c ? launch_wide<S, 8, true, false>(a, items, stream)
+                     : launch_wide<S, 8, false, false>(a, items, stream);
+  }
+  if constexpr (S <= 4) {
+    if (kp == 16)
+      return small_c ? launch_wide<S, 16, true, false>(a, items, stream)
+                     : launch_wide<S, 16, false, false>(a, items, stream);
+  }
+  return small_c ? launch_wide<S, MAX_KP, true, false>(a, items, stream)
+                 : launch_wide<S, MAX_KP, false, false>(a, items, stream);
+}
 
 template <int VD, int VKV>
 int launch_finish(const WideArgs& a, int64_t items, hipStream_t stream) {
@@ -2305,7 +2409,11 @@ int launch_class_budget(const ClassArgs& a, int64_t items, hipStream_t stream) {
 
 // Launchers, defined one translation unit per kernel family or verifier
 // variant (head_dim, K / V dtype) so that the variants compile in parallel.
-int launch_scan(const WideArgs& a, int64_t items, bool masked, hipStream_t stream);
+int launch_scan(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
+int launch_scan_1(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
+int launch_scan_2(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
+int launch_scan_4(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
+int launch_scan_8(const WideArgs& a, int64_t items, bool masked, hipStream_t stream);
 int launch_class(const ClassArgs& a, int64_t items, bool masked, const QueryLaunch* query, hipStream_t stream);
 int launch_finish_nov(const WideArgs& a, int64_t items, hipStream_t stream);
 int launch_class_budget_nov(const ClassArgs& a, int64_t items, hipStream_t stream);

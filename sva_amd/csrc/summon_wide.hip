@@ -36,9 +36,13 @@ bool summon_wide_eligible(const SummonParams& p, int64_t items) {
 size_t summon_wide_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L) {
   const int64_t items = n_seq * H * Q;
   if (n_seq != 1 || Q != 1 || n_keys < kWideMinKeys || items > kMaxWideItems) return 256;
-  const int64_t W = (n_keys + CHUNK - 1) / CHUNK;
-  return counters_bytes(items, W) + align256((size_t)items * (size_t)W * CHUNK * (sizeof(uint64_t) + sizeof(float))) +
-         over_bytes(items, std::max<int64_t>(L, 1));
+  // the largest over the chunk sizes a call may take (scan_keys_per_thread)
+  size_t most = 0;
+  for (int kp = 8; kp <= MAX_KP; kp *= 2) {
+    const int64_t W = (n_keys + WB * kp - 1) / (WB * kp);
+    most = std::max(most, counters_bytes(items, W) + lists_bytes(items, W, kp));
+  }
+  return most + over_bytes(items, std::max<int64_t>(L, 1));
 }
 
 bool summon_class_eligible(const SummonParams& p, int64_t items) {
@@ -88,9 +92,15 @@ int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_by
   const size_t need = summon_wide_workspace_bytes(1, p.H, 1, p.N, p.L);
   SVA_REQUIRE(workspace != nullptr && workspace_bytes >= need && ((uintptr_t)workspace & 255u) == 0,
               "sva_summon: workspace of %zu bytes (256-byte aligned) required, got %zu", need, workspace_bytes);
+  // a bool mask allows every key (the reference's `mask > -1e4` rule)
+  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
+  const int kp = scan_keys_per_thread(items, p.N, p.S, masked);
   WideArgs a;
   a.p = p;
-  a.W = (int)((p.N + CHUNK - 1) / CHUNK);
+  a.W = (int)((p.N + WB * kp - 1) / (WB * kp));
+  a.cap = wg_cap(a.W);
+  a.span_log2 = __builtin_ctz((unsigned)list_span(a.W));
+  a.wave_keys = WAVE * kp;
   a.overshoot = overshoot;
   a.fv = FusedVerify{};
   a.fv.out = nullptr;
@@ -103,20 +113,19 @@ int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_by
   a.nallow = a.ncand + items * a.W * NW;
   a.wg_count = (uint32_t*)(ws + align256((size_t)(2 * items * a.W * NW) * sizeof(uint32_t)));
   a.wg_cand = (uint64_t*)((char*)a.wg_count + align256((size_t)(2 * items * a.W) * sizeof(uint32_t)));
-  a.wg_rank = (float*)(a.wg_cand + items * a.W * WG_CAP);
+  a.wg_rank = (float*)(a.wg_cand + items * a.W * a.cap);
   a.cand = (uint64_t*)(ws + counters_bytes(items, a.W));
-  a.cand_rank = (float*)(ws + counters_bytes(items, a.W) + (size_t)items * (size_t)a.W * CHUNK * sizeof(uint64_t));
+  a.cand_rank = (float*)(a.cand + items * a.W * NW * a.wave_keys);
   a.items = (int)items;
   a.K = over_slices(items);
-  char* over = ws + counters_bytes(items, a.W) +
-               align256((size_t)items * (size_t)a.W * CHUNK * (sizeof(uint64_t) + sizeof(float)));
+  a.groups = a.fv.out != nullptr && finish_grouped((int)items, a.fv.G, a.K) ? a.fv.G : 0;
+  a.per = a.groups > 0 ? (int)items / a.groups : 0;
+  char* over = ws + counters_bytes(items, a.W) + lists_bytes(items, a.W, kp);
   a.arrive = (uint32_t*)over;
   a.slice_n = (uint32_t*)(over + align256((size_t)items * sizeof(uint32_t)));
   a.slice_list = (uint64_t*)(over + align256((size_t)items * sizeof(uint32_t)) +
                              align256((size_t)(items * a.K) * sizeof(uint32_t)));
-  // a bool mask allows every key (the reference's `mask > -1e4` rule)
-  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
-  const int rc = launch_scan(a, items, masked, stream);
+  const int rc = launch_scan(a, items, masked, kp, stream);
   if (rc != SVA_OK) return rc;
   return launch_finish_any(a, items, stream);
 }

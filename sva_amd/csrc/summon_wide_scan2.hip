@@ -1,0 +1,12 @@
+// Scan kernels of the long-context summon: 2 subspaces.
+#include "summon_wide.cuh"
+
+namespace sva {
+namespace wide {
+
+int launch_scan_2(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
+  return launch_wide_s<2>(a, items, masked, kp, stream);
+}
+
+}  // namespace wide
+}  // namespace sva

@@ -101,6 +101,35 @@ def test_wide_codes_at_any_address(device, N, S, C, lead):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("N,S,C,H,L,B,few", [
+    (16385, 2, 256, 9, 2048, 512, False),   # the shortest scan: nine lists of 2048 keys, the last of one key
+    (16385, 4, 64, 3, 512, 128, False),
+    (18432, 2, 64, 9, 2048, 2048, True),    # whole chunks; three codes, a boundary class of thousands
+    (16400, 8, 32, 9, 1024, 256, False),    # eight subspaces: three lists of 8192 keys
+    (30001, 1, 256, 9, 2048, 512, False),   # code classes
+    (65537, 2, 256, 1, 2048, 512, False),   # one item: chunks of 2048 keys, 33 lists
+    (262144, 4, 64, 9, 2048, 512, False),   # 128 lists of 2048 keys
+    (540000, 4, 64, 9, 2048, 512, False),   # 132 lists of 4096 keys: a second round of lists
+    (524289, 1, 200, 2, 7168, 512, False),
+])
+def test_scan_chunks_match_oracle(device, N, S, C, H, L, B, few):
+    """Every chunk size of the scan and its list layout in the finish, short caches first."""
+    from sva_amd import kernels
+
+    codes, k_low, q, q_proj, scale, cb = _setup(device, N, S, C, H=H, seed=(N + L) % 73, few=few)
+    g = torch.Generator(device=device).manual_seed(5)
+    keys = torch.randn(H, N, 64, device=device, generator=g).to(torch.bfloat16)
+    values = torch.randn(H, N, 64, device=device, generator=g).to(torch.bfloat16)
+    t = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    qb = t(q)[None].to(torch.bfloat16)
+    plan = kernels.ScanDecodePlan(device, 1, H, 1, 64, 64, S, C, L, B)
+    out = torch.empty(1, H, 1, 64, device=device, dtype=torch.float32)
+    for _ in range(2):  # the second over the first one's workspace
+        plan.run(qb, t(q_proj), t(scale), t(cb), t(codes), k_low, keys, values, N, 0.125, out=out)
+    torch.cuda.synchronize()
+    _check_decode_step(plan, codes, k_low, qb, keys, values, out, L, B)
+
+
 def test_wide_massive_ties_and_repeat(device):
     # 3 codewords: the threshold bin holds ~1/9 of all keys; exact resolution
     N, S, C = 120000, 2, 256
