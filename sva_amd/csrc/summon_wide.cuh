@@ -61,6 +61,12 @@ constexpr int WG_CAP = 128;      // candidates of a scan workgroup in its compac
 constexpr uint32_t kNoCompact = 0x80000000u;  // wg_count flag: the workgroup wrote no compact list
 constexpr int64_t kWideMinKeys = 16385;  // caches past the register path's 16384 keys
 constexpr int64_t kMaxWideItems = 64;
+// Several tokens or sequences (item_at): compact lists of MULTI_CAP entries,
+// as many items a launch as MULTI_BYTES of them hold.
+constexpr int MULTI_CAP = 512;
+constexpr int64_t MULTI_BYTES = 256ll << 20;
+constexpr int64_t kMultiMaxItems = 1 << 16;
+constexpr int64_t kMultiMaxKeys = 256ll * WB * MAX_KP;  // the fast finish's 256 lists
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -84,6 +90,7 @@ struct WideArgs {
   int cap;             // entries of a compact list (wg_cap(W))
   int span_log2;       // lists per item rounded up to a power of two (list_span(W))
   int wave_keys;       // keys of a scan wave (64 KP), the capacity of its own list
+  int item0;           // multi calls: the first item of this launch
   int groups, per;     // KV groups the fused finish is laid out by and their heads (0: not grouped)
   uint32_t* wg_count;  // [items, W, 2] candidates (or kNoCompact) and allowed keys of each scan workgroup
   uint64_t* wg_cand;   // [items, W, cap] a workgroup's candidates in key order (when they fit)
@@ -91,6 +98,8 @@ struct WideArgs {
   SummonParams p;
   uint32_t* ncand;   // [items, W * NW] candidates of each scan wave
   uint32_t* nallow;  // [items, W * NW] allowed keys of each scan wave
+  // the waves' own lists (none in a multi call: an item whose candidates
+  // outgrow a compact list goes to the all-keys select instead)
   uint64_t* cand;    // [items, W * NW, wave_keys] candidate composites of each scan wave
   float* cand_rank;  // [items, W * NW, wave_keys] rank score of each listed candidate
   FusedVerify fv;    // fv.out != nullptr: the finish kernel also runs the verifier
@@ -100,6 +109,31 @@ struct WideArgs {
   uint32_t* slice_n;   // [items, K] entries of each slice list
   uint64_t* slice_list;  // [items, K, L] each slice's top composites in key order
 };
+
+// Where an item's keys are: query head h, the first n keys of its sequence
+// (causal: a token sees no later key), which starts at catalog row off.
+struct ItemAt {
+  int h, n;
+  int64_t off;
+};
+template <bool MULTI>
+SVA_DEV ItemAt item_at(const WideArgs& a, int item) {
+  const SummonParams& p = a.p;
+  if (!MULTI) return ItemAt{item, (int)p.N, 0};  // one token of one sequence: item = head
+  const int g = a.item0 + item;
+  const int t = g % p.Q, bh = g / p.Q;
+  const int h = bh % p.H, b = bh / p.H;
+  const int64_t len = min(p.lens != nullptr ? p.lens[b] : p.N, p.N);
+  // a bool mask allows every key (the reference's `mask > -1e4` rule)
+  const int64_t n = p.mask_type == MASK_NONE ? len - p.Q + t + 1 : len;
+  return ItemAt{h, (int)max(n, (int64_t)0), p.offs != nullptr ? p.offs[b] : 0};
+}
+SVA_DEV const uint8_t* item_codes(const SummonParams& p, const ItemAt& it) {
+  return (const uint8_t*)p.codes + (int64_t)it.h * p.code_hs + it.off * p.S;
+}
+SVA_DEV const float* item_klow(const SummonParams& p, const ItemAt& it) {
+  return p.k_low + (int64_t)it.h * p.klow_hs + it.off * 64;
+}
 
 SVA_DEV uint32_t byte_of(const u32x4& v, int j) { return (v[j >> 2] >> (8 * (j & 3))) & 0xFFu; }
 
@@ -280,7 +314,7 @@ typedef __attribute__((address_space(3))) float lds_f32;
 // keys in order), as composites of the exact score acc / sqrt(R): the first
 // KL_CAP to the wave's LDS list `kc`, later ones to its global list `out`
 // (the LDS part follows there only if the workgroup has no compact list).
-template <int KPT>
+template <int KPT, bool MULTI>
 SVA_DEV void append_round(const SummonParams& p, const bool (&c)[KPT], const float (&acc)[KPT], int n0, uint64_t* out,
                           uint64_t* kc, uint32_t& wc) {
 #pragma clang fp contract(off)
@@ -298,7 +332,7 @@ SVA_DEV void append_round(const SummonParams& p, const bool (&c)[KPT], const flo
       const uint64_t x = composite(f2key(acc[k] * kInvSqrtR), (uint32_t)(n0 + k));
       if (o < (uint32_t)KL_CAP) {
         ((lds_u64*)kc)[o] = x;
-      } else {
+      } else if (!MULTI) {
         out[o] = x;
       }
       ++o;
@@ -315,7 +349,7 @@ SVA_DEV void append_round(const SummonParams& p, const bool (&c)[KPT], const flo
 // together rather than each behind the branch of the round before (eight
 // subspaces keep the per-round order: holding every round's sums would cost
 // them a wave per SIMD).
-template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED>
+template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED, bool MULTI>
 SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16], const ScanTables<S, SMALLC>& T,
                          float t_lo, int cs, int ce, uint64_t* out, uint64_t* kc, uint32_t& wc,
                          uint32_t& n_allowed) {
@@ -340,7 +374,7 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16],
         bool c[KPT];
 #pragma unroll
         for (int k = 0; k < KPT; ++k) c[k] = acc[r][k] >= t_lo;
-        append_round<KPT>(p, c, acc[r], round_key<S, KP>(cs, r), out, kc, wc);
+        append_round<KPT, MULTI>(p, c, acc[r], round_key<S, KP>(cs, r), out, kc, wc);
       }
     }
   } else {
@@ -358,7 +392,7 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16],
           c[k] = ok && acc[k] >= t_lo;
           any = any || c[k];
         }
-        if (__builtin_amdgcn_ballot_w64(any) != 0ull) append_round<KPT>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
+        if (__builtin_amdgcn_ballot_w64(any) != 0ull) append_round<KPT, MULTI>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
       } else {
         float mx = acc[0];
 #pragma unroll
@@ -367,7 +401,7 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16],
           bool c[KPT];
 #pragma unroll
           for (int k = 0; k < KPT; ++k) c[k] = acc[k] >= t_lo;
-          append_round<KPT>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
+          append_round<KPT, MULTI>(p, c, acc, round_key<S, KP>(cs, r), out, kc, wc);
         }
       }
     }
@@ -385,12 +419,11 @@ SVA_DEV void scan_rounds(const SummonParams& p, const u32x4 (&raw)[KP * S / 16],
 // only for their keys' LDS reads (a possible global key read would make each
 // row load wait for every load before it).
 template <bool LDS_ONLY>
-SVA_DEV void rank_list(const SummonParams& p, int item, const float4 qq, const uint64_t* kc, float* kr,
+SVA_DEV void rank_list(const SummonParams& p, const float* klow, const float4 qq, const uint64_t* kc, float* kr,
                        const uint64_t* out, float* rank, uint32_t nc) {
 #pragma clang fp contract(off)
   const int j = lane_id() & 15;
   const int row = lane_id() >> 4;
-  const float* klow = p.k_low + (int64_t)(item % p.H) * p.klow_hs;
   constexpr int RU = 4;
   for (uint32_t c0 = 0; c0 < nc; c0 += 4 * RU) {
     float4 rv[RU];
@@ -417,13 +450,13 @@ SVA_DEV void rank_list(const SummonParams& p, int item, const float4 qq, const u
   }
 }
 
-SVA_DEV void rank_candidates(const SummonParams& p, int item, const float4 qq, const uint64_t* kc, float* kr,
+SVA_DEV void rank_candidates(const SummonParams& p, const float* klow, const float4 qq, const uint64_t* kc, float* kr,
                              const uint64_t* out, float* rank, uint32_t nc) {
   if (nc <= (uint32_t)KL_CAP) {
-    rank_list<true>(p, item, qq, kc, kr, out, rank, nc);
+    rank_list<true>(p, klow, qq, kc, kr, out, rank, nc);
   } else {
     __threadfence();  // keys past the LDS list are read back from `out`
-    rank_list<false>(p, item, qq, kc, kr, out, rank, nc);
+    rank_list<false>(p, klow, qq, kc, kr, out, rank, nc);
   }
 }
 
@@ -440,14 +473,13 @@ struct ScanLds {
   uint32_t wcnt[NW], walw[NW];
 };
 
-template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED>
-SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, ScanLds& L) {
+template <int S, int KP, bool SMALLC, bool CHECK, bool MASKED, bool MULTI>
+SVA_DEV void scan_chunk(const WideArgs& a, int item, const ItemAt& it, int w, float* tab_lds, ScanLds& L) {
 #pragma clang fp contract(off)
   const SummonParams& p = a.p;
-  const int h = item % p.H;
   const int cs = w * (WB * KP);
-  const int ce = (int)min((int64_t)cs + WB * KP, p.N);
-  const uint8_t* codes = (const uint8_t*)p.codes + (int64_t)h * p.code_hs;
+  const int ce = min(cs + WB * KP, it.n);
+  const uint8_t* codes = item_codes(p, it);
   ScanTables<S, SMALLC> T;
   T.load(p, item);
   const float t_lo = item_floor(p, item);
@@ -459,16 +491,22 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, Scan
   const int wid = threadIdx.x / WAVE;
   const int lane = lane_id();
   const int64_t sub = ((int64_t)item * a.W + w) * NW + wid;
-  uint64_t* out = a.cand + sub * (WAVE * KP);
-  float* out_rank = a.cand_rank + sub * (WAVE * KP);
+  uint64_t* out = MULTI ? nullptr : a.cand + sub * (WAVE * KP);
+  float* out_rank = MULTI ? nullptr : a.cand_rank + sub * (WAVE * KP);
   uint32_t n_allowed = 0;
   uint32_t wc = 0;  // candidates of this wave so far (wave-uniform)
-  scan_rounds<S, KP, SMALLC, CHECK, MASKED>(p, raw, T, t_lo, cs, ce, out, L.kc[wid], wc, n_allowed);
-  rank_candidates(p, item, qq, L.kc[wid], L.kr[wid], out, out_rank, wc);
+  scan_rounds<S, KP, SMALLC, CHECK, MASKED, MULTI>(p, raw, T, t_lo, cs, ce, out, L.kc[wid], wc, n_allowed);
+  if (MULTI) {  // without lists of their own the waves rank what LDS holds: more is never used
+    rank_list<true>(p, item_klow(p, it), qq, L.kc[wid], L.kr[wid], out, out_rank, min(wc, (uint32_t)KL_CAP));
+  } else {
+    rank_candidates(p, item_klow(p, it), qq, L.kc[wid], L.kr[wid], out, out_rank, wc);
+  }
   const uint32_t wa = CHECK ? wave_sum_dpp(n_allowed) : (uint32_t)(WAVE * KP);  // every key allowed
   if (lane == 0) {
-    a.ncand[sub] = wc;
-    a.nallow[sub] = wa;
+    if (!MULTI) {
+      a.ncand[sub] = wc;
+      a.nallow[sub] = wa;
+    }
     L.wcnt[wid] = wc;
     L.walw[wid] = wa;
   }
@@ -492,7 +530,7 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, int w, float* tab_lds, Scan
       a.wg_cand[g * a.cap + off + j] = L.kc[wid][j];
       a.wg_rank[g * a.cap + off + j] = L.kr[wid][j];
     }
-  } else {
+  } else if (!MULTI) {
     const uint32_t nl = min(wc, (uint32_t)KL_CAP);
     for (uint32_t j = (uint32_t)lane; j < nl; j += WAVE) {
       out[j] = L.kc[wid][j];
@@ -543,7 +581,7 @@ __host__ __device__ inline int wg_cap(int W) {
 
 // Five workgroups per CU (at most 102 VGPRs) keep every workgroup of a
 // million-key, nine-head scan resident at once (up to four subspaces).
-template <int S, int KP, bool SMALLC, bool MASKED>
+template <int S, int KP, bool SMALLC, bool MASKED, bool MULTI>
 __global__ void __launch_bounds__(WB, S <= 4 ? 5 : 1) wide_scan_kernel(WideArgs a) {
   __shared__ __align__(16) float tab_lds[ScanTables<S, SMALLC>::LDS_FLOATS];
   __shared__ ScanLds lds;
@@ -551,10 +589,13 @@ __global__ void __launch_bounds__(WB, S <= 4 ? 5 : 1) wide_scan_kernel(WideArgs 
   const int w = blockIdx.x % a.W;
   if (blockIdx.x == 0)  // arrival counters of the finish kernel's all-keys select
     for (int i = threadIdx.x; i < a.items; i += WB) a.arrive[i] = 0u;
-  if (!MASKED && (int64_t)(w + 1) * (WB * KP) <= a.p.N) {
-    scan_chunk<S, KP, SMALLC, false, false>(a, item, w, tab_lds, lds);
-  } else {
-    scan_chunk<S, KP, SMALLC, true, MASKED>(a, item, w, tab_lds, lds);
+  const ItemAt it = item_at<MULTI>(a, item);
+  if (!MASKED && (int64_t)(w + 1) * (WB * KP) <= it.n) {
+    scan_chunk<S, KP, SMALLC, false, false, MULTI>(a, item, it, w, tab_lds, lds);
+  } else if (!MULTI || w * (WB * KP) < it.n) {
+    scan_chunk<S, KP, SMALLC, true, MASKED, MULTI>(a, item, it, w, tab_lds, lds);
+  } else if (threadIdx.x < 2) {  // past the item's keys (a multi call: the lists of shorter items are empty)
+    a.wg_count[2 * ((int64_t)item * a.W + w) + threadIdx.x] = 0u;
   }
 }
 
@@ -595,11 +636,10 @@ constexpr int NPD = 7;              // dense slots per thread
 
 // Rank score of a 64-float k_low row in torch's sum order, computed here
 // for the all-keys path: rows r of sl, one 16-lane DPP row each.
-SVA_DEV void rank_rows(const SummonParams& p, int item, const uint32_t* sl, int n, float* out) {
+SVA_DEV void rank_rows(const SummonParams& p, int item, const float* klow, const uint32_t* sl, int n, float* out) {
 #pragma clang fp contract(off)
   const int j = lane_id() & 15;
   const float4 qq = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * p.R)[j];
-  const float* klow = p.k_low + (int64_t)(item % p.H) * p.klow_hs;
   for (int r = threadIdx.x >> 4; r < n; r += SB / 16) {
     const float dot = rank_dot64_row16(reinterpret_cast<const float4*>(klow + (int64_t)sl[r] * p.R)[j], qq);
     if (j == 0) out[r] = dot * kInvSqrtR;
@@ -924,8 +964,12 @@ SVA_DEV uint64_t fast_select(const uint64_t (&e)[NPD], const float (&v)[NPD], in
 // 4096 / (hi - lo), or 0 (one bin) when the range is empty.
 SVA_DEV float lin_scale(float lo, float hi) { return hi > lo ? 4096.0f / (hi - lo) : 0.0f; }
 
-// The fast finish of an item; false (uniformly, before any output or LDS
-// write) when its conditions do not hold.
+// The fast finish of an item; false (uniformly, before any list output) when
+// its conditions do not hold.  A tie class too large to rank directly sends a
+// one-token item to the general paths; a multi call has none of their lists
+// and resolves it by the general register select here (inlined into the
+// one-token finish it cost 2 us of its 20).
+template <bool MULTI>
 SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32_t* rkb, uint32_t* wcnt,
                          uint32_t* scratch, const TopLds& tl, int32_t* kidl, int& beff_out) {
 #pragma clang fp contract(off)
@@ -1081,7 +1125,7 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
   uint64_t X = 1ull;
   // the budget select's histogram is built by the shortlist select, over the
   // rank range of every candidate
-  const bool fuse = (uint32_t)leff < M && p.B > 0 && beff < leff;
+  bool fuse = (uint32_t)leff < M && p.B > 0 && beff < leff;
   const RankFuse rf{(uint32_t*)(lds + kFastRHist), (float*)(lds + kFastSmallR), key2f(rklo),
                     lin_scale(key2f(rklo), key2f(rkhi))};
   if ((uint32_t)leff < M) {
@@ -1092,7 +1136,10 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
              : fast_select(e, sv, dslots, leff, vlo, vinv, hist, small, f, &exact, true);
     if (!exact) {
       __syncthreads();
-      return false;  // a tie class too large to rank directly: the general paths
+      if constexpr (!MULTI) return false;
+      X = select_top_regs<SB, NPD>(e, leff, ((uint64_t)f2key(p.range[4 * item + 1] * kInvSqrtR) << 32) | 0xFFFFFFFFull,
+                                   (uint64_t)f2key(vlo) << 32, tl, dslots, true);
+      fuse = false;  // no rank histogram was built
     }
   }
   // budget composites of the shortlist: (rank key, key index)
@@ -1114,7 +1161,9 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
     XB = fast_select(rc, rv, dslots, beff, rf.rlo, rf.rinv, rf.rhist, small, f, &ex2, true);
     if (!ex2) {
       __syncthreads();
-      return false;
+      if constexpr (!MULTI) return false;
+      XB = select_top_regs<SB, NPD>(rc, beff, ((uint64_t)rkhi << 32) | 0xFFFFFFFFull, (uint64_t)rklo << 32, tl,
+                                    dslots, true);
     }
   } else if (p.B > 0 && beff < leff) {
     wave_min_max_u32(rmin, rmax);
@@ -1134,7 +1183,9 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
     XB = fast_select(rc, rv, dslots, beff, rlo, lin_scale(rlo, key2f(hi)), hist, small, f, &ex2);
     if (!ex2) {
       __syncthreads();
-      return false;
+      if constexpr (!MULTI) return false;
+      XB = select_top_regs<SB, NPD>(rc, beff, ((uint64_t)hi << 32) | 0xFFFFFFFFull, (uint64_t)lo << 32, tl, dslots,
+                                    true);
     }
   }
   // outputs in list order (ascending key order): per (slot, wave) counts of
@@ -1250,7 +1301,8 @@ SVA_DEV void overshoot_visit(const SummonParams& p, const uint8_t* __restrict__ 
   const int C = p.C;
   const uint32_t cm = (uint32_t)(C - 1);
   const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
-  const int wbeg = n0 / KPW, wend = (n1 + KPW - 1) / KPW;
+  // (a slice past a short item's keys starts at its last key's end, not on a word: nothing to visit)
+  const int wbeg = n0 / KPW, wend = n0 < n1 ? (n1 + KPW - 1) / KPW : wbeg;
   // word w0 + u * SB + t for u < kOverWords: every load instruction of a wave reads 1 KB in a row
   for (int w0 = wbeg; w0 < wend; w0 += kOverWords * SB) {
     u32x4 w[kOverWords];
@@ -1346,7 +1398,8 @@ SVA_DEV Boundary hist_boundary(const uint32_t* hist, uint32_t k, uint32_t* scrat
 // Exact composite of key n (0 when masked out), scalar: the tie-class fallback's visitor.
 SVA_DEV uint64_t key_composite(const SummonParams& p, const uint8_t* codes, const float* lut_l, int n) {
 #pragma clang fp contract(off)
-  if (!mask_allows(p.mask, n, p.mask_type)) return 0ull;
+  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
+  if (masked && !mask_allows(p.mask, n, p.mask_type)) return 0ull;
   // the reference's exact score ((0 + T0[c0]) + T1[c1]) + ... then / sqrt(R)
   float acc = 0.0f;
   for (int s2 = 0; s2 < p.S; ++s2) {
@@ -1360,14 +1413,13 @@ SVA_DEV uint64_t key_composite(const SummonParams& p, const uint8_t* codes, cons
 // The top min(k, allowed) composites of keys [n0, n1) of an item, in key
 // order, to out (global); returns their number (block-uniform).
 template <int S>
-SVA_DEV uint32_t slice_select(const SummonParams& p, int item, uint32_t k, int n0, int n1, const float* lut_l,
+SVA_DEV uint32_t slice_select(const SummonParams& p, int item, const uint8_t* codes, uint32_t k, int n0, int n1, const float* lut_l,
                               unsigned char* lds, uint32_t* scratch, uint32_t* shared, uint64_t* shared64,
                               uint64_t* __restrict__ out) {
   const int t = threadIdx.x;
   uint32_t* hist = (uint32_t*)(lds + kFinHist);
   uint64_t* lst = (uint64_t*)(lds + kOverList);
   uint64_t* bnd = (uint64_t*)(lds + kOverBnd);
-  const uint8_t* codes = (const uint8_t*)p.codes + (int64_t)(item % p.H) * p.code_hs;
   const float lo = p.range[4 * item] * kInvSqrtR, hi = p.range[4 * item + 1] * kInvSqrtR;
   const float inv_w = lin_scale(lo, hi);
   reinterpret_cast<uint4*>(hist)[t] = uint4{0u, 0u, 0u, 0u};
@@ -1504,6 +1556,7 @@ SVA_DEV void merge_slices(const WideArgs& a, int item, uint32_t leff, unsigned c
 // (budget list in LDS) or 0 (in the budget output) when this workgroup
 // finished the item, -1 when it has nothing more to do (a slice workgroup
 // whose item's floor held, or that did not complete the item's last slice).
+template <bool MULTI>
 SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* lds, int32_t* kidl, int& beff_out) {
 #pragma clang fp contract(off)
   uint64_t* cl = (uint64_t*)lds;                                   // staged candidates [LDS_CAND]
@@ -1520,9 +1573,10 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   uint32_t* loff = (uint32_t*)(lds + kFinLoff);
   const TopLds tl{hist, small, scratch, shared, shared64};
   const SummonParams& p = a.p;
-  if (slice == 0 && finish_fast(a, item, lds, rkb, wcnt, scratch, tl, kidl, beff_out)) return kidl != nullptr ? 1 : 0;
+  if (slice == 0 && finish_fast<MULTI>(a, item, lds, rkb, wcnt, scratch, tl, kidl, beff_out)) return kidl != nullptr ? 1 : 0;
   const int t = threadIdx.x;
   const int lane = lane_id();
+  const ItemAt it = item_at<MULTI>(a, item);
   const int nsub = a.W * NW;
   const int wave_keys = a.wave_keys, cap = a.cap;
   const uint32_t* ncand = a.ncand + (int64_t)item * nsub;
@@ -1540,9 +1594,25 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     rkb[1] = 0u;
   }
   uint32_t m = 0, al = 0;
-  for (int sidx = t; sidx < nsub; sidx += SB) {
-    m += ncand[sidx];
-    al += nallow[sidx];
+  if (!MULTI) {
+    for (int sidx = t; sidx < nsub; sidx += SB) {
+      m += ncand[sidx];
+      al += nallow[sidx];
+    }
+  } else {
+    // no lists of the waves' own: the fast finish took the item unless a
+    // compact list overflowed or the candidates outgrow it, and then every
+    // key is selected over (M below leff)
+    bool no = a.W > FAST_LISTS;
+    for (int l = t; l < a.W; l += SB) {
+      const uint32_t c = a.wg_count[2 * ((int64_t)item * a.W + l)];
+      no = no || c == kNoCompact;
+      m += c == kNoCompact ? 0u : c;
+      al += a.wg_count[2 * ((int64_t)item * a.W + l) + 1];
+    }
+    uint32_t total;
+    block_excl_scan<SB>(m, scratch, &total);
+    if (__syncthreads_or(no || total > (uint32_t)FAST_M)) m = 0u;
   }
   if (nsub <= SB) lcnt[t] = m;
   uint32_t M;
@@ -1569,7 +1639,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     if (p.B > 0) p.fin_count[item] = beff;
   }
   if (leff == 0) return 0;
-  if (M >= (uint32_t)leff) {
+  if (!MULTI && M >= (uint32_t)leff) {
     // the per-wave lists of scan workgroups that wrote a compact list hold
     // only candidates past their wave's first KL_CAP (none: a compact list is
     // written only when every wave's candidates fit its LDS list): copy the
@@ -1595,7 +1665,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   // bounds of every candidate composite: sums in [floor, upper bound of any sum]
   const uint64_t c_lo = (uint64_t)f2key(item_floor(p, item) * kInvSqrtR) << 32;
   const uint64_t c_hi = ((uint64_t)f2key(p.range[4 * item + 1] * kInvSqrtR) << 32) | 0xFFFFFFFFull;
-  if (M >= (uint32_t)leff && M <= (uint32_t)(NPD * SB) && nsub <= DL_LISTS && longest <= 48u) {
+  if (!MULTI && M >= (uint32_t)leff && M <= (uint32_t)(NPD * SB) && nsub <= DL_LISTS && longest <= 48u) {
     if (longest <= 32u) {
       uint64_t e_sp[2 * DK];
       gather_lists<2>(cand, nsub, wave_keys, e_sp);
@@ -1618,7 +1688,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     kmax = max(kmax, rkey);
   };
   bool dense = true;  // rank composites in rk (else sl + ranks in LDS)
-  if (M >= (uint32_t)leff && M <= (uint32_t)LDS_CAND && nsub <= STAGE_LISTS) {
+  if (!MULTI && M >= (uint32_t)leff && M <= (uint32_t)LDS_CAND && nsub <= STAGE_LISTS) {
     // staged: lists into LDS in list order
     if (nsub <= SB) {
       loff[t] = block_excl_scan<SB>(m, scratch, nullptr);
@@ -1677,7 +1747,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     }
     compact_ordered<SB, NPT>(e, X, leff, wcnt, scratch, slots,
                              [&](uint32_t o, uint64_t x, int i) { emit(o, x, rnk[i]); });
-  } else if (M >= (uint32_t)leff) {
+  } else if (!MULTI && M >= (uint32_t)leff) {
     // lists: select straight from the per-wave lists in global memory
     dense = false;
     float* rkf = (float*)rk;
@@ -1716,7 +1786,8 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     // all keys: the sampled floor overshot; this workgroup selects slice `slice`
     dense = false;
     if (t == 0 && slice == 0 && a.overshoot != nullptr) a.overshoot[item] = 1;
-    const int N = (int)p.N, K = a.K;
+    const int N = it.n, K = a.K;
+    const uint8_t* codes = item_codes(p, it);
     // the item's table in LDS: the slice select scores every key of the slice from it
     float* lut_l = (float*)(lds + kFinLut);
     const float* lut_g = p.lut + (int64_t)item * p.S * p.C;
@@ -1727,10 +1798,10 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     uint64_t* out = a.slice_list + ((int64_t)item * K + slice) * p.L;
     uint32_t nj;
     switch (p.S) {
-      case 1: nj = slice_select<1>(p, item, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
-      case 2: nj = slice_select<2>(p, item, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
-      case 4: nj = slice_select<4>(p, item, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
-      default: nj = slice_select<8>(p, item, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
+      case 1: nj = slice_select<1>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
+      case 2: nj = slice_select<2>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
+      case 4: nj = slice_select<4>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
+      default: nj = slice_select<8>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
     }
     // publish the slice (release), then count it in; the item's last slice finishes the item
     if (t == 0) a.slice_n[(int64_t)item * K + slice] = nj;
@@ -1745,7 +1816,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     if (shared[0] == 0u) return -1;
     __threadfence();  // acquire: the other slices' lists
     merge_slices(a, item, (uint32_t)leff, lds, sl, lcnt, scratch, shared, shared64);
-    rank_rows(p, item, sl, leff, (float*)rk);
+    rank_rows(p, item, item_klow(p, it), sl, leff, (float*)rk);
   }
   // bounds of the emitted rank keys (direct and staged paths) for the budget select
   wave_min_max_u32(kmin, kmax);
@@ -2020,7 +2091,7 @@ SVA_DEV void finish_slot(const WideArgs& a, int b, int& item, int& slice) {
 // Finish of an item, then (VD > 0: head_dim VD, K / V dtype VKV) its
 // verifier.  Workgroup b takes the item and slice finish_slot gives it;
 // slice 0 is the item's finish, slices > 0 serve the all-keys select.
-template <int VD, int VKV>
+template <int VD, int VKV, bool MULTI>
 __global__ void __launch_bounds__(SB) wide_finish_kernel(WideArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ float qsh[VD > 0 ? VD : 1];  // the verifier's query row
@@ -2037,7 +2108,7 @@ __global__ void __launch_bounds__(SB) wide_finish_kernel(WideArgs a) {
   if (slice == 0 && threadIdx.x == 0 && a.overshoot != nullptr) a.overshoot[item] = 0;  // the all-keys select sets 1
   const bool keep = VD > 0 && a.p.B <= kVerifyKidCap - SNW * (VD + 2) - SNW - 1;
   int beff = 0;
-  const int done = finish_item(a, item, slice, lds, keep ? (int32_t*)(lds + kVerifyKid) : nullptr, beff);
+  const int done = finish_item<MULTI>(a, item, slice, lds, keep ? (int32_t*)(lds + kVerifyKid) : nullptr, beff);
   if (done < 0) return;  // block-uniform
   if (VD > 0) {
     if ((int)threadIdx.x < VD) qsh[threadIdx.x] = elem_from_bits(qbits, a.fv.q_dtype);
@@ -2364,37 +2435,39 @@ inline size_t lists_bytes(int64_t items, int64_t W, int kp) {
 }
 
 // The scan of S-subspace codes, kp keys a thread (kp < MAX_KP: unmasked, S <= 4).
-template <int S, int KP, bool SMALLC, bool MASKED>
+template <int S, int KP, bool SMALLC, bool MASKED, bool MULTI>
 int launch_wide(const WideArgs& a, int64_t items, hipStream_t stream) {
-  hipLaunchKernelGGL((wide_scan_kernel<S, KP, SMALLC, MASKED>), dim3((unsigned)(items * a.W)), dim3(WB), 0, stream, a);
+  hipLaunchKernelGGL((wide_scan_kernel<S, KP, SMALLC, MASKED, MULTI>), dim3((unsigned)(items * a.W)), dim3(WB), 0, stream, a);
   SVA_CHECK_LAUNCH("wide_scan_kernel");
   return SVA_OK;
 }
 
-template <int S>
-int launch_wide_s(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
-  const bool small_c = a.p.C <= 64;
-  if (masked)
-    return small_c ? launch_wide<S, MAX_KP, true, true>(a, items, stream)
-                   : launch_wide<S, MAX_KP, false, true>(a, items, stream);
-  if constexpr (S >= 2 && S <= 4) {
-    if (kp == 8)
-      return small_c ? launch_wide<S, 8, true, false>(a, items, stream)
-                     : launch_wide<S, 8, false, false>(a, items, stream);
-  }
-  if constexpr (S <= 4) {
-    if (kp == 16)
-      return small_c ? launch_wide<S, 16, true, false>(a, items, stream)
-                     : launch_wide<S, 16, false, false>(a, items, stream);
-  }
-  return small_c ? launch_wide<S, MAX_KP, true, false>(a, items, stream)
-                 : launch_wide<S, MAX_KP, false, false>(a, items, stream);
+template <int S, int KP, bool MULTI>
+int launch_wide_c(const WideArgs& a, int64_t items, hipStream_t stream) {
+  return a.p.C <= 64 ? launch_wide<S, KP, true, false, MULTI>(a, items, stream)
+                     : launch_wide<S, KP, false, false, MULTI>(a, items, stream);
 }
 
-template <int VD, int VKV>
+template <int S, bool MULTI>
+int launch_wide_s(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
+  if constexpr (!MULTI) {
+    if (masked)
+      return a.p.C <= 64 ? launch_wide<S, MAX_KP, true, true, false>(a, items, stream)
+                         : launch_wide<S, MAX_KP, false, true, false>(a, items, stream);
+  }
+  if constexpr (S >= 2 && S <= 4) {
+    if (kp == 8) return launch_wide_c<S, 8, MULTI>(a, items, stream);
+  }
+  if constexpr (S <= 4) {
+    if (kp == 16) return launch_wide_c<S, 16, MULTI>(a, items, stream);
+  }
+  return launch_wide_c<S, MAX_KP, MULTI>(a, items, stream);
+}
+
+template <int VD, int VKV, bool MULTI = false>
 int launch_finish(const WideArgs& a, int64_t items, hipStream_t stream) {
-  SVA_SET_MAX_LDS_ONCE((wide_finish_kernel<VD, VKV>), kFinLds, "hipFuncSetAttribute(wide_finish_kernel)");
-  hipLaunchKernelGGL((wide_finish_kernel<VD, VKV>), dim3((unsigned)(items * a.K)), dim3(SB), kFinLds, stream, a);
+  SVA_SET_MAX_LDS_ONCE((wide_finish_kernel<VD, VKV, MULTI>), kFinLds, "hipFuncSetAttribute(wide_finish_kernel)");
+  hipLaunchKernelGGL((wide_finish_kernel<VD, VKV, MULTI>), dim3((unsigned)(items * a.K)), dim3(SB), kFinLds, stream, a);
   SVA_CHECK_LAUNCH("wide_finish_kernel");
   return SVA_OK;
 }
@@ -2413,8 +2486,11 @@ int launch_scan(const WideArgs& a, int64_t items, bool masked, int kp, hipStream
 int launch_scan_1(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
 int launch_scan_2(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
 int launch_scan_4(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
-int launch_scan_8(const WideArgs& a, int64_t items, bool masked, hipStream_t stream);
+int launch_scan_8(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream);
+int launch_multi_scan(const WideArgs& a, int64_t items, int kp, hipStream_t stream);
+int launch_multi_finish(const WideArgs& a, int64_t items, hipStream_t stream);
 int launch_class(const ClassArgs& a, int64_t items, bool masked, const QueryLaunch* query, hipStream_t stream);
+int launch_multi_floor(const WideArgs& a, int64_t items, float* range, hipStream_t stream);
 int launch_finish_nov(const WideArgs& a, int64_t items, hipStream_t stream);
 int launch_class_budget_nov(const ClassArgs& a, int64_t items, hipStream_t stream);
 int launch_finish_v64_bf16(const WideArgs& a, int64_t items, hipStream_t stream);

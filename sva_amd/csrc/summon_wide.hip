@@ -33,9 +33,9 @@ bool summon_wide_eligible(const SummonParams& p, int64_t items) {
   return true;
 }
 
-size_t summon_wide_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L) {
-  const int64_t items = n_seq * H * Q;
-  if (n_seq != 1 || Q != 1 || n_keys < kWideMinKeys || items > kMaxWideItems) return 256;
+namespace {
+
+size_t wide_bytes(int64_t items, int64_t n_keys, int64_t L) {
   // the largest over the chunk sizes a call may take (scan_keys_per_thread)
   size_t most = 0;
   for (int kp = 8; kp <= MAX_KP; kp *= 2) {
@@ -43,6 +43,99 @@ size_t summon_wide_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t 
     most = std::max(most, counters_bytes(items, W) + lists_bytes(items, W, kp));
   }
   return most + over_bytes(items, std::max<int64_t>(L, 1));
+}
+
+}  // namespace
+
+size_t summon_wide_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L) {
+  const int64_t items = n_seq * H * Q;
+  if (n_keys < kWideMinKeys) return 256;
+  // (a packed batch of one sequence and token is a multi call with these sizes too)
+  const size_t multi = summon_multi_workspace_bytes(items, n_keys, L);
+  if (n_seq != 1 || Q != 1 || items > kMaxWideItems) return multi;
+  return std::max(multi, wide_bytes(items, n_keys, L));
+}
+
+// Where it replaces one workgroup per item: caches past the register path's
+// 16384 keys (below, an item's keys sit in one workgroup's registers), uint8
+// codes, no value mask, and shortlists whose usual 2 L candidates the fast
+// finish holds.  Four tokens over 262144 keys (4x64, 2048 / 512): 2860 us an
+// item a workgroup, 53 here.
+bool summon_multi_eligible(const SummonParams& p, int64_t items) {
+  if (p.ctype != CODE_U8 || p.C > 256 || p.R != 64) return false;
+  if (p.S != 1 && p.S != 2 && p.S != 4 && p.S != 8) return false;
+  if (p.N < kWideMinKeys || p.N > kMultiMaxKeys || items > kMultiMaxItems) return false;
+  if (2 * p.L > FAST_M || p.sl_idx == nullptr) return false;
+  if (((uintptr_t)p.k_low & 15u) != 0 || p.klow_hs % 4 != 0 || ((uintptr_t)p.q_low & 15u) != 0) return false;
+  return p.mask_type == MASK_NONE || p.mask_type == MASK_BOOL;
+}
+
+namespace {
+
+// Items a launch takes: the candidate lists of a group stay within MULTI_BYTES.
+int64_t multi_group(int64_t items, int64_t W) {
+  const int64_t most = std::max<int64_t>(64, MULTI_BYTES / (W * MULTI_CAP * 12));
+  const int64_t groups = (items + most - 1) / most;
+  return (items + groups - 1) / groups;
+}
+size_t multi_lists_bytes(int64_t group, int64_t W) {
+  return align256((size_t)(2 * group * W) * sizeof(uint32_t)) +
+         align256((size_t)(group * W * MULTI_CAP) * (sizeof(uint64_t) + sizeof(float)));
+}
+
+}  // namespace
+
+size_t summon_multi_workspace_bytes(int64_t items, int64_t n_keys, int64_t L) {
+  if (n_keys < kWideMinKeys || n_keys > kMultiMaxKeys || items > kMultiMaxItems || 2 * L > FAST_M) return 256;
+  size_t most = 0;  // over the chunk sizes a call may take
+  for (int kp = 8; kp <= MAX_KP; kp *= 2) {
+    const int64_t W = (n_keys + WB * kp - 1) / (WB * kp);
+    const int64_t group = multi_group(items, W);
+    most = std::max(most, multi_lists_bytes(group, W) + over_bytes(group, std::max<int64_t>(L, 1)));
+  }
+  return align256((size_t)(4 * items) * sizeof(float)) + most;
+}
+
+int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, hipStream_t stream) {
+  const int kp = scan_keys_per_thread(items, p.N, p.S, false);
+  WideArgs a{};
+  a.p = p;
+  a.W = (int)((p.N + WB * kp - 1) / (WB * kp));
+  a.cap = MULTI_CAP;
+  a.span_log2 = __builtin_ctz((unsigned)list_span(a.W));
+  a.wave_keys = WAVE * kp;
+  const int64_t group = multi_group(items, a.W);
+  char* ws = (char*)workspace;
+  float* range = (float*)ws;  // the items' bounds and floors
+  ws += align256((size_t)(4 * items) * sizeof(float));
+  a.wg_count = (uint32_t*)ws;
+  a.wg_cand = (uint64_t*)(ws + align256((size_t)(2 * group * a.W) * sizeof(uint32_t)));
+  a.wg_rank = (float*)(a.wg_cand + group * a.W * MULTI_CAP);
+  a.K = over_slices(group);
+  char* over = ws + multi_lists_bytes(group, a.W);
+  a.arrive = (uint32_t*)over;
+  a.slice_n = (uint32_t*)(over + align256((size_t)group * sizeof(uint32_t)));
+  a.slice_list = (uint64_t*)(over + align256((size_t)group * sizeof(uint32_t)) +
+                             align256((size_t)(group * a.K) * sizeof(uint32_t)));
+  int rc = launch_multi_floor(a, items, range, stream);
+  for (int64_t g = 0; rc == SVA_OK && g < items; g += group) {
+    const int64_t n = std::min(group, items - g);
+    a.item0 = (int)g;
+    a.items = (int)n;
+    a.p.lut = p.lut + g * p.S * p.C;
+    a.p.range = range + 4 * g;
+    a.p.q_low = p.q_low + g * p.R;
+    a.p.sl_idx = p.sl_idx + g * p.L;
+    a.p.sl_rank = p.sl_rank + g * p.L;
+    a.p.sl_count = p.sl_count + g;
+    if (p.B > 0) {
+      a.p.fin_idx = p.fin_idx + g * p.B;
+      a.p.fin_count = p.fin_count + g;
+    }
+    rc = launch_multi_scan(a, n, kp, stream);
+    if (rc == SVA_OK) rc = launch_multi_finish(a, n, stream);
+  }
+  return rc;
 }
 
 bool summon_class_eligible(const SummonParams& p, int64_t items) {
@@ -89,13 +182,13 @@ bool fused_verify_eligible(const SummonParams& p, int64_t items, const FusedVeri
 int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_bytes, hipStream_t stream,
                      const FusedVerify* fv, int32_t* overshoot) {
   const int64_t items = (int64_t)p.H;  // one sequence, q = 1
-  const size_t need = summon_wide_workspace_bytes(1, p.H, 1, p.N, p.L);
+  const size_t need = wide_bytes(items, p.N, p.L);
   SVA_REQUIRE(workspace != nullptr && workspace_bytes >= need && ((uintptr_t)workspace & 255u) == 0,
               "sva_summon: workspace of %zu bytes (256-byte aligned) required, got %zu", need, workspace_bytes);
   // a bool mask allows every key (the reference's `mask > -1e4` rule)
   const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
   const int kp = scan_keys_per_thread(items, p.N, p.S, masked);
-  WideArgs a;
+  WideArgs a{};
   a.p = p;
   a.W = (int)((p.N + WB * kp - 1) / (WB * kp));
   a.cap = wg_cap(a.W);

@@ -5,7 +5,7 @@ namespace sva {
 namespace wide {
 
 int launch_scan_1(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
-  return launch_wide_s<1>(a, items, masked, kp, stream);
+  return launch_wide_s<1, false>(a, items, masked, kp, stream);
 }
 
 }  // namespace wide

@@ -5,7 +5,7 @@ namespace sva {
 namespace wide {
 
 int launch_scan_2(const WideArgs& a, int64_t items, bool masked, int kp, hipStream_t stream) {
-  return launch_wide_s<2>(a, items, masked, kp, stream);
+  return launch_wide_s<2, false>(a, items, masked, kp, stream);
 }
 
 }  // namespace wide

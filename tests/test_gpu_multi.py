@@ -1,0 +1,88 @@
+"""The long-context summon of several tokens or sequences (many workgroups
+per item) against one workgroup per item on the same inputs: shortlists in
+key order, rank scores, budgets and counts equal bit for bit.  A call whose
+workspace is short takes the one-workgroup form, which the oracle checks
+elsewhere; here the first items are checked against the oracle too."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _select(lut, rng, q_low, codes, k_low, n_keys, L, B, ws_bytes, offs=None, lens=None, mask_type=0):
+    from sva_amd import kernels
+    from sva_amd._lib import check, code_type, lib, ptr, stream_handle
+
+    n_seq, H, Q, S, C = lut.shape
+    items = n_seq * H * Q
+    dev = lut.device
+    sl_idx = torch.full((items, L), -1, device=dev, dtype=torch.int32)
+    sl_rank = torch.zeros(items, L, device=dev)
+    counts = torch.full((2, items), -1, device=dev, dtype=torch.int32)
+    fin = torch.full((items, B), -1, device=dev, dtype=torch.int32)
+    ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    check(lib().sva_summon_select(
+        ptr(lut), ptr(rng), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low), k_low.stride(0),
+        ptr(offs), ptr(lens), n_seq, H, Q, n_keys, 64, S, C, L, None, mask_type, 0, ptr(sl_idx), ptr(sl_rank),
+        counts[0].data_ptr(), B, ptr(fin), counts[1].data_ptr(), ptr(ws), ws.numel(), stream_handle(dev)), "select")
+    torch.cuda.synchronize()
+    return sl_idx, sl_rank, counts, fin
+
+
+@pytest.mark.parametrize("n_seq,Q,lens,S,C,H,L,B,few,mask_type", [
+    (1, 2, (16385,), 2, 256, 3, 512, 128, False, 0),           # the shortest cache: nine lists, the last of one key
+    (1, 4, (70001,), 4, 64, 9, 2048, 512, False, 0),           # odd heads of codes
+    (1, 3, (40000,), 1, 256, 2, 2048, 512, False, 0),          # one subspace: tie classes of 156 keys
+    (1, 2, (50000,), 2, 256, 2, 1024, 1024, True, 0),          # three codes: a boundary class of thousands
+    (1, 2, (33333,), 8, 32, 2, 512, 128, False, 0),            # eight subspaces
+    (1, 5, (20000,), 2, 64, 2, 3584, 700, False, 4),           # the largest shortlist; a bool mask allows every key
+    (1, 70, (17000,), 2, 256, 9, 512, 128, False, 0),          # hundreds of items
+    (4, 1, (30000, 1, 5000, 16999), 2, 256, 3, 2048, 512, False, 0),   # packed: short and one-key sequences
+    (3, 3, (2, 20001, 4096), 4, 64, 2, 512, 128, False, 0),    # fewer keys than tokens: empty items
+    (2, 2, (600, 16500), 1, 100, 2, 2048, 512, False, 0),
+    (1, 2, (300000,), 2, 256, 1, 64, 16, False, 0),            # a small shortlist
+])
+def test_multi_equals_item_path(device, n_seq, Q, lens, S, C, H, L, B, few, mask_type):
+    from sva_amd import kernels
+    from sva_amd._lib import lib
+
+    rows = sum(lens)
+    g = torch.Generator(device=device).manual_seed(rows % 97 + Q)
+    codes = torch.randint(0, 3 if few else C, (H, rows, S), device=device, generator=g).to(torch.uint8)
+    k_low = torch.randn(H, rows, 64, device=device, generator=g)
+    q = torch.randn(n_seq, H, Q, 64, device=device, generator=g)
+    q_proj = torch.randn(H, 64, 64, device=device, generator=g) / 8
+    cb = torch.randn(H, S, C, 64 // S, device=device, generator=g)
+    q_low, lut, rng = kernels.query_lut(q, q_proj, torch.ones(H, device=device), cb)
+    offs = lens_t = None
+    if n_seq > 1:
+        offs = torch.tensor([0, *lens[:-1]], device=device).cumsum(0)
+        lens_t = torch.tensor(lens, device=device)
+    n = max(lens)
+    need = int(lib().sva_summon_workspace_bytes(n_seq, H, Q, n, L))
+    assert need > 256
+    got = _select(lut, rng, q_low, codes, k_low, n, L, B, need, offs, lens_t, mask_type)
+    ref = _select(lut, rng, q_low, codes, k_low, n, L, B, 256, offs, lens_t, mask_type)
+    assert torch.equal(got[2], ref[2])
+    for item in range(got[2].shape[1]):
+        cnt, fc = int(ref[2][0, item]), int(ref[2][1, item])
+        for a, b, m in ((got[0], ref[0], cnt), (got[1].view(torch.int32), ref[1].view(torch.int32), cnt),
+                        (got[3], ref[3], fc)):
+            assert torch.equal(a[item, :m], b[item, :m]), f"item {item}"
+    # the oracle on the last sequence's first head and last token
+    b, item = n_seq - 1, ((n_seq - 1) * H) * Q + Q - 1
+    o = rows - lens[-1]
+    ql = q_low[b, 0, Q - 1].cpu().numpy()
+    scores = oracle.pq_scores_from_lut(lut[b, 0, Q - 1].cpu().numpy(), codes[0, o:].contiguous().cpu().numpy(), 64)
+    want = np.sort(oracle.topk(scores, L))
+    cnt = int(got[2][0, item])
+    assert cnt == len(want)
+    np.testing.assert_array_equal(got[0][item, :cnt].cpu().numpy(), want)
+    ranks = oracle.rank_scores(k_low[0, o:].cpu().numpy(), want, ql, 64)
+    np.testing.assert_array_equal(got[1][item, :cnt].cpu().numpy().view(np.uint32), ranks.view(np.uint32))
