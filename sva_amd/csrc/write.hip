@@ -663,6 +663,7 @@ int write_encode_launch(const WriteParams& p, hipStream_t stream) {
   }
   const int64_t es = p.kv_dtype == 0 ? 4 : 2;
   const bool rows_aligned = ((uintptr_t)p.keys & 15u) == 0 && (p.kv_hs * es) % 16 == 0 && (p.kv_rs * es) % 16 == 0;
+  if (rows_aligned && sva::write_split_eligible(p)) return sva::write_split_launch(p, stream);
   if (rows_aligned && R == 64 && (D == 64 || D == 128)) {
     if (S == 2 && C == 256)
       return D == 64 ? launch_persistent<64, 2, 32, 256>(p, tiles, stream)

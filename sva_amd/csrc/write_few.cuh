@@ -27,6 +27,11 @@ struct WriteParams {
   int64_t seq_kv, seq_rows;
 };
 
+// The bulk form for head_dim = rank = 64 and 16-byte aligned rows
+// (write_split.hip).
+bool write_split_eligible(const WriteParams& p);
+int write_split_launch(const WriteParams& p, hipStream_t stream);
+
 // A decode step's append (at most FEW_ROWS rows): one workgroup per head,
 // the arithmetic of sva_write_encode's tiled kernels with the work spread
 // over the threads instead of over a tile of rows: thread (row, r) forms

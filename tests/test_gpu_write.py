@@ -148,3 +148,55 @@ def test_batch_encode_equals_each_sequence(device, S, C, kv_dtype, n_rows):
     assert torch.equal(k_low, ref_low), "k_low differs"
     assert torch.equal(codes, ref_codes), "codes differ"
     assert bool((k_low[:, :row0] == 7.0).all()) and bool((codes[:, cap - 1] == 9).all()), "rows outside the range written"
+
+
+@pytest.mark.parametrize("S,C", [(2, 256), (4, 64), (1, 256)])
+@pytest.mark.parametrize("kv_dtype,n_rows,kind", [
+    (torch.bfloat16, 8191, "plain"),    # the fp32 form's last size at six heads
+    (torch.bfloat16, 8192, "plain"), (torch.float16, 8193, "plain"), (torch.float32, 8223, "plain"),
+    (torch.bfloat16, 20011, "plain"),
+    (torch.float32, 8300, "close"),     # codewords 1e-4 apart: the halves decide almost no row
+    (torch.bfloat16, 8300, "twins"),    # every codeword twice: the first index wins
+    (torch.float32, 8300, "far"),       # rows beyond the halves' range, infinities and NaN among them
+    (torch.float32, 8300, "tiny"),      # values of 1e-30
+    (torch.float32, 8300, "wild"),      # an infinite and a NaN codeword
+    (torch.bfloat16, 8300, "zero"),     # all-zero codebooks
+])
+def test_bulk_codes_equal_fp32_distances(device, S, C, kv_dtype, n_rows, kind):
+    """The bulk form (49152 rows over all heads and more) decides most rows by split half-precision scores; keys at odd addresses take the fp32 form
+    (the chains the oracle checks above).  Same k_low bits, same codes, rows outside the range untouched."""
+    from sva_amd import kernels
+
+    H, G, D, R, row0, rows = 6, 3, 64, 64, 3, n_rows + 5
+    g = torch.Generator(device=device).manual_seed(n_rows + S)
+    keys = torch.randn(G, rows, D, device=device, generator=g)
+    k_proj = torch.randn(H, D, R, device=device, generator=g) / 8.0
+    cb = torch.randn(H, S, C, R // S, device=device, generator=g)
+    if kind == "close":
+        cb = cb[:, :, :1] + 1e-4 * cb
+    elif kind == "twins":
+        cb[:, :, C // 2:] = cb[:, :, :C // 2]
+    elif kind == "far":
+        keys[:, ::3] *= 1e6
+        keys[:, 1::50] = float("inf")
+        keys[:, 2::50, 5] = float("nan")
+    elif kind == "tiny":
+        keys, cb = keys * 1e-30, cb * 1e-30
+    elif kind == "wild":
+        cb[0, 0, 3, 2], cb[1, 0, 5] = float("inf"), float("nan")
+    elif kind == "zero":
+        cb.zero_()
+    keys = keys.to(kv_dtype)
+    odd = torch.zeros(G, rows, D + 1, device=device, dtype=kv_dtype)[:, :, 1:]
+    odd.copy_(keys)
+    outs = []
+    for k in (keys, odd):
+        k_low = torch.full((H, rows, R), 7.0, device=device)
+        codes = torch.full((H, rows, S), 9, device=device, dtype=torch.uint8)
+        kernels.write_encode(k, k_proj, cb, k_low, codes, row0, n_rows)
+        outs.append((k_low.view(torch.int32), codes))
+    torch.cuda.synchronize()
+    if kind != "far":  # NaN payloads are not defined
+        assert torch.equal(outs[0][0], outs[1][0]), "k_low differs"
+    assert torch.equal(outs[0][1], outs[1][1]), f"{int((outs[0][1] != outs[1][1]).sum())} codes differ"
+    assert bool((outs[0][1][:, :row0] == 9).all()) and bool((outs[0][1][:, row0 + n_rows:] == 9).all())
