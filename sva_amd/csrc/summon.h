@@ -18,13 +18,17 @@ constexpr int kMaxLds = 160 * 1024;  // LDS per workgroup on gfx950
 // samples above the L-th largest key is ~Poisson(n_s L / N); k is about
 // twice that mean and at least SAMPLE_MIN_RANK, so an overshoot is rare
 // (about 1e-4 at 1M keys, L = 2048, 8K samples).
+// SAMPLE_MIN_CAND keeps a floor under short shortlists; twice a shortlist of
+// 512 is enough (at 1M keys 4 samples expected above it and rank 16: an
+// overshoot in 2e5 heads), and 4096 candidates there cost the scan their rank
+// rows: 512 / 128 over 100003 keys 31.5 us a lookup, 27.2 at 1024.
 constexpr int SAMPLE_KEYS = 32;
 constexpr int SAMPLE_BINS = 1024;
 constexpr int SAMPLE_MIN_BLOCKS = 64;
 constexpr int SAMPLE_MAX_BYTES = 32768;
 constexpr int SAMPLE_MAX_BLOCKS = 256;  // at most 8K sampled keys
 constexpr double SAMPLE_TARGET = 2.0;
-constexpr double SAMPLE_MIN_CAND = 4096.0;
+constexpr double SAMPLE_MIN_CAND = 1024.0;
 constexpr int SAMPLE_MIN_RANK = 16;
 constexpr int SAMPLE_MAX_S = 8;  // subspaces of the sampled scan
 
