@@ -5,14 +5,17 @@
 //   out  = attn_output + corr.to(attn dtype)             (in the attn dtype)
 // down [rank, 2 * hidden] and up [hidden, rank] are fp32 (nn.Linear weights).
 //
-// One workgroup per TOK tokens: the tokens' inputs are staged in LDS as
-// fp32, each thread forms down-projection outputs (token, o) as a
-// sequential fma chain over the 2 * hidden inputs, the GELU values go to
-// LDS, then each output (token, j) is a sequential chain over the rank.
-// Consecutive threads take consecutive tokens of one output, so a wave's
-// weight loads read a few rows (the same address across a row's tokens)
-// rather than one row per lane; the staged rows are padded by a float so
-// that the tokens' reads of one column fall in different LDS banks.
+// One workgroup of 16 waves per NT tokens, their inputs staged in LDS as fp32.
+// Down: a wave per output o, its lanes along the 2 * hidden inputs (coalesced
+// weight rows, each read once for the NT tokens), then one wave sum a token.
+// Up: a thread per output j over the rank's GELU values; its first weights are
+// requested at entry and wait through the down projection.  A decode step's
+// few tokens are bound by the latency of weights that miss the L2 (the layer
+// runs once a step): a workgroup a token takes 8 tokens, hidden 576, rank 16 in
+// 15.1 us (most of it the call), where one workgroup for all of them, a sequential chain of 1152
+// a thread, took 33.5.  Many tokens share a workgroup's weight reads (NT up to
+// 8) once the chip is full.
+#include <algorithm>
 #include <cmath>
 
 #include "capi_internal.h"
@@ -23,9 +26,10 @@ using namespace sva;
 
 namespace {
 
-constexpr int AB = 256;          // threads per workgroup
+constexpr int AB = 1024;         // threads per workgroup
 constexpr int MAX_RANK = 64;
-constexpr int MAX_TOK = 16;
+constexpr int MAX_TOK = 8;
+constexpr int UPF = 16;          // up weights a thread requests at entry
 
 struct AdapterParams {
   const void* hidden;
@@ -38,7 +42,7 @@ struct AdapterParams {
   const float* up;    // [H, rank]
   float scale;
   int64_t T;
-  int H, rank, tok;
+  int H, rank;
   void* out;
   int o_dtype;
   int64_t o_rs;
@@ -56,120 +60,157 @@ SVA_DEV float round_to(float v, int dtype) {
   return __half2float(__float2half_rn(v));
 }
 
+__host__ __device__ inline int adapter_row(int H) { return (2 * H + 3) & ~3; }  // floats of a staged token
+
+template <int NT>
 __global__ void __launch_bounds__(AB) residual_adapter_kernel(AdapterParams p) {
 #pragma clang fp contract(off)
-  extern __shared__ __align__(16) float xs[];  // [tok][2 * H + 1], then z [tok][rank + 1]
-  const int H2 = 2 * p.H;
-  const int XS = H2 + 1, ZS = p.rank + 1;  // padded row strides
-  float* z = xs + p.tok * XS;
-  const int64_t t0 = (int64_t)blockIdx.x * p.tok;
-  const int nt = (int)min((int64_t)p.tok, p.T - t0);
-  // Both weight matrices requested by every thread at entry, one float per
-  // 128-byte line: they miss the L2 at every call (the layer runs once a
-  // step), and the chains below would otherwise wait on one miss after
-  // another.  The values are folded into a word that is stored only in a case
-  // that cannot occur (a negative token count), so the loads are kept.
-  float touch = 0.0f;
+  extern __shared__ __align__(16) float xs[];  // [NT][adapter_row], then z [NT][MAX_RANK]
+  const int H = p.H, H2 = 2 * H, XS = adapter_row(H), rank = p.rank;
+  float* z = xs + NT * XS;
+  const int64_t t0 = (int64_t)blockIdx.x * NT;
+  const int nt = (int)min((int64_t)NT, p.T - t0);
+  const int t = threadIdx.x, lane = lane_id();
+  const int wid = __builtin_amdgcn_readfirstlane(t / WAVE);
+  const bool vec_up = ((uintptr_t)p.up & 15u) == 0 && rank % 4 == 0;
+  const bool vec_down = ((uintptr_t)p.down & 15u) == 0 && H2 % 4 == 0;
+  // up: the first weights of output j = t (clamped; used where vec_up)
+  float4 uw[UPF / 4];
   {
-    const int64_t nd = (int64_t)p.rank * H2, nall = nd + (int64_t)p.H * p.rank;  // floats
-    auto at = [&](int64_t f) { return f < nd ? p.down[f] : p.up[f - nd]; };
-    constexpr int TU = 16;  // the first TU lines a thread, requested together (indices clamped)
-    float v[TU];
+    const float4* row = reinterpret_cast<const float4*>(p.up + (vec_up ? (int64_t)min(t, H - 1) * rank : 0));
 #pragma unroll
-    for (int u = 0; u < TU; ++u) v[u] = at(min(((int64_t)threadIdx.x + (int64_t)u * AB) * 32, nall - 1));
-#pragma unroll
-    for (int u = 0; u < TU; ++u) touch += v[u];
-    for (int64_t f = ((int64_t)threadIdx.x + (int64_t)TU * AB) * 32; f < nall; f += (int64_t)AB * 32) touch += at(f);
+    for (int u = 0; u < UPF / 4; ++u) uw[u] = vec_up ? row[min(u, rank / 4 - 1)] : float4{0.0f, 0.0f, 0.0f, 0.0f};
   }
   {
     // the inputs, SU elements a thread per batch: raw bits requested first
     // (indices clamped, every load unconditional), converted at the store
-    constexpr int SU = 8;
+    constexpr int SU = 4;
     const int total = nt * H2;
-    for (int e0 = threadIdx.x; e0 < total; e0 += SU * AB) {
+    for (int e0 = t; e0 < total; e0 += SU * AB) {
       uint32_t bits[SU];
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
         const int e = min(e0 + u * AB, total - 1);
-        const int t = e / H2, k = e - t * H2;
-        const bool hid = k < p.H;
-        bits[u] = load_elem_bits(hid ? p.hidden : p.attn, hid ? (t0 + t) * p.h_rs + k : (t0 + t) * p.a_rs + (k - p.H),
+        const int q = e / H2, k = e - q * H2;
+        const bool hid = k < H;
+        bits[u] = load_elem_bits(hid ? p.hidden : p.attn, hid ? (t0 + q) * p.h_rs + k : (t0 + q) * p.a_rs + (k - H),
                                  hid ? p.h_dtype : p.a_dtype);
       }
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
         const int e = e0 + u * AB;
         if (e < total) {
-          const int t = e / H2, k = e - t * H2;
-          xs[t * XS + k] = elem_from_bits(bits[u], k < p.H ? p.h_dtype : p.a_dtype);
+          const int q = e / H2, k = e - q * H2;
+          xs[q * XS + k] = elem_from_bits(bits[u], k < H ? p.h_dtype : p.a_dtype);
         }
       }
     }
+    // tokens past the last one and the padding: zeros (their results are not stored)
+    for (int e = t; e < NT * (XS - H2); e += AB) xs[(e / (XS - H2)) * XS + H2 + e % (XS - H2)] = 0.0f;
+    for (int e = nt * XS + t; e < NT * XS; e += AB) xs[e] = 0.0f;
   }
+  // down: this wave's first output's weights requested ahead of the barrier
+  constexpr int V = 8;  // float4s a lane holds: 2048 inputs a round
+  float4 dw[V];
+  auto load_row = [&](int o, int k0) {
+    const float4* row = reinterpret_cast<const float4*>(p.down + (int64_t)o * H2);
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const int q = k0 / 4 + lane + WAVE * u;
+      dw[u] = q < H2 / 4 ? row[q] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  };
+  if (vec_down && wid < rank) load_row(wid, 0);
   __syncthreads();
-  // the weight rows as float4 where aligned: a chain of 2H steps is bound by
-  // its loads unless the next 32 weights are in flight while the current 32
-  // are used (the same fma chain, in k order)
-  constexpr int V = 8;  // float4s per batch
-  const bool vec = ((uintptr_t)p.down & 15u) == 0 && ((uintptr_t)p.up & 15u) == 0 && H2 % (4 * V) == 0 &&
-                   p.rank % 4 == 0;
-  for (int e = threadIdx.x; e < nt * p.rank; e += AB) {
-    const int o = e / nt, t = e - o * nt;
-    const float* x = xs + t * XS;
-    const float* w = p.down + (int64_t)o * H2;
-    float acc = 0.0f;
-    if (vec) {
-      const float4* w4 = reinterpret_cast<const float4*>(w);
-      const int nb = H2 / (4 * V);
-      float4 cur[V], nxt[V];
+  for (int o = wid; o < rank; o += AB / WAVE) {
+    float acc[NT];
 #pragma unroll
-      for (int u = 0; u < V; ++u) cur[u] = w4[u];
-      for (int b = 0; b < nb; ++b) {
-        const int bn = min(b + 1, nb - 1);  // the last batch loads itself again: every load unconditional
-#pragma unroll
-        for (int u = 0; u < V; ++u) nxt[u] = w4[bn * V + u];
+    for (int q = 0; q < NT; ++q) acc[q] = 0.0f;
+    if (vec_down) {
+      for (int k0 = 0; k0 < H2; k0 += 4 * WAVE * V) {
+        if (o != wid || k0 > 0) load_row(o, k0);
 #pragma unroll
         for (int u = 0; u < V; ++u) {
-          const float* xk = x + (b * V + u) * 4;
-          acc = __builtin_fmaf(xk[0], cur[u].x, acc);
-          acc = __builtin_fmaf(xk[1], cur[u].y, acc);
-          acc = __builtin_fmaf(xk[2], cur[u].z, acc);
-          acc = __builtin_fmaf(xk[3], cur[u].w, acc);
-        }
+          const int k = k0 + 4 * (lane + WAVE * u);
+          if (k0 + 4 * WAVE * u < H2) {  // uniform
 #pragma unroll
-        for (int u = 0; u < V; ++u) cur[u] = nxt[u];
+            for (int q = 0; q < NT; ++q) {
+              const float4 x = *reinterpret_cast<const float4*>(xs + q * XS + min(k, XS - 4));
+              acc[q] = __builtin_fmaf(x.x, dw[u].x, acc[q]);
+              acc[q] = __builtin_fmaf(x.y, dw[u].y, acc[q]);
+              acc[q] = __builtin_fmaf(x.z, dw[u].z, acc[q]);
+              acc[q] = __builtin_fmaf(x.w, dw[u].w, acc[q]);
+            }
+          }
+        }
       }
     } else {
-      for (int k = 0; k < H2; ++k) acc = __builtin_fmaf(x[k], w[k], acc);
+      const float* row = p.down + (int64_t)o * H2;
+      for (int k = lane; k < H2; k += WAVE) {
+        const float w = row[k];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) acc[q] = __builtin_fmaf(xs[q * XS + k], w, acc[q]);
+      }
     }
-    z[t * ZS + o] = 0.5f * acc * (1.0f + erff(acc * 0.70710678118654752f));  // F.gelu (erf form)
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      const float v = wave_sum(acc[q]);
+      if (lane == q) z[q * MAX_RANK + o] = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));  // F.gelu (erf form)
+    }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < nt * p.H; e += AB) {
-    const int j = e / nt, t = e - j * nt;
-    const float* zz = z + t * ZS;
-    const float* w = p.up + (int64_t)j * p.rank;
-    float acc = 0.0f;
-    if (vec && p.rank == MAX_RANK) {  // the row's 64 weights requested at once
-      const float4* w4 = reinterpret_cast<const float4*>(w);
-      float4 wv[MAX_RANK / 4];
+  for (int j = t; j < H; j += AB) {
+    const float* w = p.up + (int64_t)j * rank;
+    float acc[NT];
 #pragma unroll
-      for (int u = 0; u < MAX_RANK / 4; ++u) wv[u] = w4[u];
+    for (int q = 0; q < NT; ++q) acc[q] = 0.0f;
+    if (vec_up) {
+      for (int o = 0; o < rank; o += UPF) {
+        if (j != t || o > 0) {
 #pragma unroll
-      for (int u = 0; u < MAX_RANK / 4; ++u) {
-        acc = __builtin_fmaf(zz[4 * u], wv[u].x, acc);
-        acc = __builtin_fmaf(zz[4 * u + 1], wv[u].y, acc);
-        acc = __builtin_fmaf(zz[4 * u + 2], wv[u].z, acc);
-        acc = __builtin_fmaf(zz[4 * u + 3], wv[u].w, acc);
+          for (int u = 0; u < UPF / 4; ++u)
+            uw[u] = reinterpret_cast<const float4*>(w)[min(o / 4 + u, rank / 4 - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < UPF / 4; ++u) {
+          if (o + 4 * u < rank) {  // uniform
+#pragma unroll
+            for (int q = 0; q < NT; ++q) {
+              const float4 zz = *reinterpret_cast<const float4*>(z + q * MAX_RANK + o + 4 * u);
+              acc[q] = __builtin_fmaf(zz.x, uw[u].x, acc[q]);
+              acc[q] = __builtin_fmaf(zz.y, uw[u].y, acc[q]);
+              acc[q] = __builtin_fmaf(zz.z, uw[u].z, acc[q]);
+              acc[q] = __builtin_fmaf(zz.w, uw[u].w, acc[q]);
+            }
+          }
+        }
       }
     } else {
-      for (int o = 0; o < p.rank; ++o) acc = __builtin_fmaf(zz[o], w[o], acc);
+      for (int o = 0; o < rank; ++o) {
+        const float wv = w[o];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) acc[q] = __builtin_fmaf(z[q * MAX_RANK + o], wv, acc[q]);
+      }
     }
-    const float corr = round_to(acc * p.scale, p.a_dtype);
-    const float a = xs[t * XS + p.H + j];
-    store_elem(p.out, (t0 + t) * p.o_rs + j, p.o_dtype, a + corr);
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      if (q < nt) {  // uniform
+        const float corr = round_to(acc[q] * p.scale, p.a_dtype);
+        store_elem(p.out, (t0 + q) * p.o_rs + j, p.o_dtype, xs[q * XS + H + j] + corr);
+      }
+    }
   }
-  if (p.T < 0) store_elem(p.out, threadIdx.x, p.o_dtype, touch);  // never: keeps the requests above
+}
+
+template <int NT>
+int launch_adapter(const AdapterParams& p, hipStream_t stream) {
+  const int64_t blocks = (p.T + NT - 1) / NT;
+  SVA_REQUIRE(blocks < (1ll << 31), "sva_residual_adapter: too many tokens");
+  const size_t lds = sizeof(float) * (size_t)NT * (size_t)(adapter_row(p.H) + MAX_RANK);
+  SVA_SET_MAX_LDS_ONCE(residual_adapter_kernel<NT>, sva::kMaxLds, "hipFuncSetAttribute(residual_adapter_kernel)");
+  hipLaunchKernelGGL(residual_adapter_kernel<NT>, dim3((unsigned)blocks), dim3(AB), lds, stream, p);
+  SVA_CHECK_LAUNCH("residual_adapter_kernel");
+  return SVA_OK;
 }
 
 }  // namespace
@@ -187,15 +228,6 @@ extern "C" int sva_residual_adapter(const void* hidden, int hidden_dtype, int64_
                   out_dtype <= 2,
               "sva_residual_adapter: bad dtype");
   if (n_tokens == 0) return SVA_OK;
-  // tokens per workgroup: as many as fit 64 KB of staged fp32 inputs (rows padded by a float), at most MAX_TOK
-  const int64_t per_tok = sizeof(float) * (2 * hidden_size + 1 + rank + 1);
-  const int tok = (int)std::max<int64_t>(1, std::min<int64_t>(MAX_TOK, (64 * 1024) / per_tok));
-  const size_t lds = (size_t)tok * (size_t)per_tok;
-  SVA_UNSUPPORTED(lds <= (size_t)sva::kMaxLds, "sva_residual_adapter: hidden size %lld needs %zu bytes of LDS",
-                  (long long)hidden_size, lds);
-  const int64_t blocks = (n_tokens + tok - 1) / tok;
-  SVA_REQUIRE(blocks < (1ll << 31), "sva_residual_adapter: too many tokens");
-  SVA_SET_MAX_LDS_ONCE(residual_adapter_kernel, sva::kMaxLds, "hipFuncSetAttribute(residual_adapter_kernel)");
   AdapterParams p;
   p.hidden = hidden;
   p.h_dtype = hidden_dtype;
@@ -209,12 +241,15 @@ extern "C" int sva_residual_adapter(const void* hidden, int hidden_dtype, int64_
   p.T = n_tokens;
   p.H = (int)hidden_size;
   p.rank = (int)rank;
-  p.tok = tok;
   p.out = out;
   p.o_dtype = out_dtype;
   p.o_rs = out_row_stride;
-  hipLaunchKernelGGL(residual_adapter_kernel, dim3((unsigned)blocks), dim3(AB), lds, (hipStream_t)stream, p);
-  SVA_CHECK_LAUNCH("residual_adapter_kernel");
-  return SVA_OK;
+  // tokens a workgroup shares its weight reads over: one until every CU has a
+  // workgroup, then more, while two workgroups' inputs fit a CU's LDS
+  const int64_t room = (72 * 1024) / (int64_t)(sizeof(float) * (adapter_row(p.H) + MAX_RANK));
+  const int64_t want = std::min<int64_t>({(n_tokens + 255) / 256, room, MAX_TOK});
+  if (want >= 8) return launch_adapter<8>(p, (hipStream_t)stream);
+  if (want >= 4) return launch_adapter<4>(p, (hipStream_t)stream);
+  if (want >= 2) return launch_adapter<2>(p, (hipStream_t)stream);
+  return launch_adapter<1>(p, (hipStream_t)stream);
 }
-

@@ -39,6 +39,39 @@ def test_residual_adapter_matches_oracle(device, T, H, rank, dtype):
     assert err <= tol, f"rel err {err}"
 
 
+@pytest.mark.parametrize("T,H,rank,dtype,odd", [
+    (1, 5, 1, torch.float32, False),        # fewer inputs than lanes
+    (257, 130, 7, torch.float16, False),    # two tokens a workgroup, the last alone; rows of 260 inputs
+    (1025, 576, 20, torch.float32, False),  # four to eight tokens a workgroup, a rank past the prefetched weights
+    (2049, 576, 16, torch.bfloat16, True),  # weights at odd addresses
+    (2, 1500, 64, torch.float32, False),    # more outputs than threads
+    (3, 8192, 3, torch.float32, False),     # the widest model
+])
+def test_adapter_workgroup_shapes(device, T, H, rank, dtype, odd):
+    """Every token count a workgroup takes and both weight layouts, against float64: sums of at most 2 H + rank
+    fp32 products in any order are within (2 H + rank) 2^-24 of their absolute sum, far inside 1e-5."""
+    from sva_amd import kernels
+
+    g = torch.Generator(device=device).manual_seed(T + H)
+    h = torch.randn(T, H, device=device, generator=g).to(dtype)
+    a = torch.randn(T, H, device=device, generator=g).to(dtype)
+
+    def weight(rows, cols, std):
+        w = torch.randn(rows, cols, device=device, generator=g) * std
+        if not odd:
+            return w
+        buf = torch.empty(rows * cols + 1, device=device)[1:].view(rows, cols)
+        return buf.copy_(w)
+
+    down, up = weight(rank, 2 * H, 0.02), weight(H, rank, 0.5)
+    out = kernels.residual_adapter(h, a, down, up, 0.75)
+    x = torch.cat([h, a], -1).double()
+    corr = torch.nn.functional.gelu(x @ down.double().T) @ up.double().T * 0.75
+    ref = a.double() + corr.to(dtype).double()
+    err = float((out.double() - ref).abs().max() / ref.abs().max())
+    assert err <= {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 2e-2}[dtype], f"rel err {err}"
+
+
 class _Fixed(nn.Module):
     def __init__(self, out):
         super().__init__()
