@@ -29,13 +29,18 @@ namespace {
 
 struct ItemLds {
   // offsets (bytes) of the dynamic LDS regions
-  int tab, ql, hist, scratch, shared, slidx, keys, total;
+  int tab, ql, hist, scratch, shared, wcnt, slidx, keys, total;
 };
+
+// The linear-bin select of keys held in LDS (see summon_item_kernel).
+constexpr int LIN_BINS = 4096;
+constexpr int LIN_CAP = 1024;   // boundary-bin members ranked directly
+constexpr int LIN_ITERS = 40;   // rounds of ITEM_BLOCK keys (163840 bytes of LDS hold fewer)
 
 // idx16: shortlist slots as uint16 (every key index below 65536), which
 // leaves room for the keys of caches of about 35K keys at L = 8192.
 __host__ __device__ inline ItemLds item_lds_layout(int S, int C, int R, int L, int64_t N, bool keys_in_lds,
-                                                   bool idx16) {
+                                                   bool idx16, bool lin) {
   ItemLds l;
   int o = 0;
   l.tab = o;
@@ -48,16 +53,23 @@ __host__ __device__ inline ItemLds item_lds_layout(int S, int C, int R, int L, i
   o = align16(o + 4 * (ITEM_BLOCK / WAVE + 1));
   l.shared = o;
   o = align16(o + 4 * 4);
+  l.wcnt = o;
+  if (lin) o = align16(o + 4 * LIN_ITERS * (ITEM_BLOCK / WAVE));
+  // the shortlist's slots; until they are written, the bins and then the
+  // boundary members of the linear-bin select
   l.slidx = o;
-  o = align16(o + (idx16 ? 2 : 4) * L);
+  const int slots = (idx16 ? 2 : 4) * L;
+  o = align16(o + (lin && slots < 4 * LIN_BINS ? 4 * LIN_BINS : slots));
   l.keys = o;
   if (keys_in_lds) o = align16(o + (int)(4 * N));
   l.total = o;
   return l;
 }
 
-// flags: bit 0 the keys sit in LDS, bit 1 the shortlist slots are uint16
-// (item_lds_layout's idx16; the host sets both from the largest length).
+// flags: bit 0 the keys sit in LDS, bit 1 the shortlist slots are uint16,
+// bit 2 LDS has room for the linear-bin select (item_lds_layout's arguments;
+// the host sets them from the largest length), bit 3 the rank scores are left
+// to rescore_kernel.
 __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p, int flags) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) unsigned char lds[];
@@ -67,8 +79,8 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   const int b = item / (p.Q * p.H);
   const int64_t len = p.lens ? p.lens[b] : p.N;
   const int64_t off = p.offs ? p.offs[b] : 0;
-  const bool keys_in_lds = (flags & 1) != 0, idx16 = (flags & 2) != 0;
-  const ItemLds L = item_lds_layout(p.S, p.C, p.R, p.L, len, keys_in_lds, idx16);
+  const bool keys_in_lds = (flags & 1) != 0, idx16 = (flags & 2) != 0, lin = (flags & 4) != 0;
+  const ItemLds L = item_lds_layout(p.S, p.C, p.R, p.L, len, keys_in_lds, idx16, lin);
   float* tab = (float*)(lds + L.tab);
   float* ql = (float*)(lds + L.ql);
   uint32_t* hist = (uint32_t*)(lds + L.hist);
@@ -111,6 +123,30 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
     return f2key(r64 ? acc * 0.125f : acc / sqrt_r);
   };
 
+  // The linear-bin select (keys in LDS, finite bounds of any score): every key
+  // is counted in one of LIN_BINS bins linear in [lo, hi] as it is scored, the
+  // bin holding the L-th largest is found by one scan, and only its members
+  // are ranked.  Bins spread what a radix digit concentrates (the keys of a
+  // few exponents: LDS atomics on the same words, four passes of them), and
+  // the compaction reads keys in lane order, not in thread-contiguous
+  // segments that meet in two banks.  72 items of 32768 keys, 2x256, 8192 of
+  // them kept: the kernel 92 us against 125 (44 with the rank scores apart).
+  const float lo_s = r64 ? p.range[4 * item] * 0.125f : p.range[4 * item] / sqrt_r;
+  const float hi_s = r64 ? p.range[4 * item + 1] * 0.125f : p.range[4 * item + 1] / sqrt_r;
+  const float span = hi_s - lo_s;
+  const bool linear = lin && span > 0.0f && span < INFINITY;
+  const float inv_w = (float)LIN_BINS / span;
+  uint32_t* bins = (uint32_t*)(lds + L.slidx);
+  // a non-decreasing function of the score
+  auto bin_of = [&](uint32_t k) {
+    const float b = (key2f(k) - lo_s) * inv_w;
+    return b < 1.0f ? 0 : (b >= (float)(LIN_BINS - 1) ? LIN_BINS - 1 : (int)b);
+  };
+  if (linear) {
+    static_assert(LIN_BINS == 4 * ITEM_BLOCK, "four bins a thread");
+    reinterpret_cast<uint4*>(bins)[threadIdx.x] = uint4{0u, 0u, 0u, 0u};
+    __syncthreads();
+  }
   uint32_t cnt = 0;
   const bool u8w = p.ctype == CODE_U8 && (S == 1 || S == 2 || S == 4) && code_base % S == 0 &&
                    ((uintptr_t)p.codes % (uintptr_t)S) == 0;
@@ -146,6 +182,7 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
           }
           cnt += k != 0u;
           keys[n] = k;
+          if (linear && k != 0u) atomicAdd(&bins[bin_of(k)], 1u);
         }
       }
     }
@@ -154,6 +191,7 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
       const uint32_t k = compute_key(n);
       cnt += k != 0u;
       if (keys_in_lds) keys[n] = k;
+      if (linear && k != 0u) atomicAdd(&bins[bin_of(k)], 1u);
     }
   }
   uint32_t allowed_total;
@@ -166,40 +204,132 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
 
   auto get_key = [&](int64_t n) -> uint32_t { return keys_in_lds ? keys[n] : compute_key(n); };
 
-  uint32_t T;
-  int keq;
-  radix_select_u32<ITEM_BLOCK>([&](int i) { return get_key(i); }, (int)len, leff, hist, scratch, shared, &T, &keq);
-
-  // compaction in key-index order over thread-contiguous segments
-  const int64_t seg = (len + ITEM_BLOCK - 1) / ITEM_BLOCK;
-  const int64_t lo = min((int64_t)threadIdx.x * seg, len);
-  const int64_t hi = min(lo + seg, len);
-  uint32_t gt = 0, eq = 0;
-  for (int64_t n = lo; n < hi; ++n) {
-    const uint32_t k = get_key(n);
-    gt += k > T;
-    eq += k == T;
-  }
-  const uint32_t eq_before = block_excl_scan<ITEM_BLOCK>(eq, scratch, nullptr);
-  const int take_eq = max(0, min((int)eq, keq - (int)eq_before));
-  uint32_t pos = block_excl_scan<ITEM_BLOCK>(gt + (uint32_t)take_eq, scratch, nullptr);
-  int taken = 0;
-  for (int64_t n = lo; n < hi; ++n) {
-    const uint32_t k = get_key(n);
-    if (k > T) {
-      set_slot(pos++, n);
-    } else if (k == T && taken < take_eq) {
-      set_slot(pos++, n);
-      ++taken;
+  uint32_t T = 0u;
+  int keq = 0x7FFFFFFF;  // every allowed key (T = 0 is no key's)
+  bool done = false;
+  if (linear && leff < (int)allowed_total) {
+    // thread t owns bins 4 t .. 4 t + 3 counted from the top
+    const uint4 hv = reinterpret_cast<const uint4*>(bins)[ITEM_BLOCK - 1 - threadIdx.x];
+    const uint32_t c[4] = {hv.w, hv.z, hv.y, hv.x};
+    uint32_t a = block_excl_scan<ITEM_BLOCK>(c[0] + c[1] + c[2] + c[3], scratch, nullptr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (a < (uint32_t)leff && a + c[j] >= (uint32_t)leff) {
+        shared[0] = (uint32_t)(LIN_BINS - 1 - 4 * (int)threadIdx.x - j);
+        shared[1] = a;
+        shared[2] = c[j];
+      }
+      a += c[j];
     }
+    if (threadIdx.x == 0) shared[3] = 0u;
+    __syncthreads();
+    const int bb = (int)shared[0];
+    const uint32_t need = (uint32_t)leff - shared[1], members = shared[2];
+    done = members <= (uint32_t)LIN_CAP;
+    if (done) {
+      uint64_t* mem = (uint64_t*)bins;  // every thread has read its bins
+      for (int64_t n = threadIdx.x; n < len; n += ITEM_BLOCK) {
+        const uint32_t k = keys[n];
+        if (k != 0u && bin_of(k) == bb) mem[atomicAdd(&shared[3], 1u)] = composite(k, (uint32_t)n);
+      }
+      __syncthreads();
+      // the need-th largest by (key, lower index first), and how many of its key are taken
+      if (threadIdx.x < members) {
+        const uint64_t x = mem[threadIdx.x];
+        uint32_t above = 0, above_key = 0;
+        for (uint32_t o = 0; o < members; ++o) {
+          above += mem[o] > x ? 1u : 0u;
+          above_key += (mem[o] >> 32) > (x >> 32) ? 1u : 0u;
+        }
+        if (above == need - 1u) {
+          shared[0] = (uint32_t)(x >> 32);
+          shared[1] = need - above_key;
+        }
+      }
+      __syncthreads();
+      T = shared[0];
+      keq = (int)shared[1];
+    }
+    __syncthreads();
+  } else if (linear) {
+    done = true;
   }
-  __syncthreads();
+  if (linear && done) {
+    // compaction in key-index order: round i of the block takes keys
+    // i ITEM_BLOCK .., so (round, wave, lane) is key order; per (round, wave)
+    // counts of both kinds in one word, one scan, then the slots
+    uint32_t* wcnt = (uint32_t*)(lds + L.wcnt);
+    const int lane = lane_id(), wid = (int)threadIdx.x / WAVE;
+    const int rounds = (int)((len + ITEM_BLOCK - 1) / ITEM_BLOCK);
+    uint64_t gm = 0ull, em = 0ull;  // bit i: this thread's key of round i
+    for (int i = 0; i < rounds; ++i) {
+      const int64_t n = (int64_t)i * ITEM_BLOCK + threadIdx.x;
+      const uint32_t k = n < len ? keys[n] : 0u;
+      const bool g = k > T, e = k != 0u && k == T;
+      gm |= (uint64_t)g << i;
+      em |= (uint64_t)e << i;
+      const uint64_t gb = __builtin_amdgcn_ballot_w64(g), eb = __builtin_amdgcn_ballot_w64(e);
+      if (lane == 0) wcnt[i * (ITEM_BLOCK / WAVE) + wid] = (uint32_t)__popcll(gb) | ((uint32_t)__popcll(eb) << 16);
+    }
+    __syncthreads();
+    constexpr int NWV = ITEM_BLOCK / WAVE;
+    static_assert(LIN_ITERS * NWV <= ITEM_BLOCK, "one count a thread");
+    const int nc = rounds * NWV;
+    const uint32_t mine = (int)threadIdx.x < nc ? wcnt[threadIdx.x] : 0u;
+    const uint32_t base_eq = block_excl_scan<ITEM_BLOCK>(mine >> 16, scratch, nullptr);
+    const uint32_t base_gt = block_excl_scan<ITEM_BLOCK>(mine & 0xFFFFu, scratch, nullptr);
+    if ((int)threadIdx.x < nc) wcnt[threadIdx.x] = base_gt | (min(base_eq, 0xFFFFu) << 16);
+    __syncthreads();
+    for (int i = 0; i < rounds; ++i) {
+      const bool g = ((gm >> i) & 1ull) != 0ull, e = ((em >> i) & 1ull) != 0ull;
+      const uint64_t gb = __builtin_amdgcn_ballot_w64(g), eb = __builtin_amdgcn_ballot_w64(e);
+      if (!g && !e) continue;
+      const uint32_t w = wcnt[i * NWV + wid];
+      const uint32_t gp = (w & 0xFFFFu) + __builtin_amdgcn_mbcnt_hi((uint32_t)(gb >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)gb, 0u));
+      const uint32_t ep = (w >> 16) + __builtin_amdgcn_mbcnt_hi((uint32_t)(eb >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)eb, 0u));
+      const int64_t n = (int64_t)i * ITEM_BLOCK + threadIdx.x;
+      if (g) set_slot(gp + min(ep, (uint32_t)keq), n);
+      else if (ep < (uint32_t)keq) set_slot(gp + ep, n);
+    }
+    __syncthreads();
+  } else {
+    radix_select_u32<ITEM_BLOCK>([&](int i) { return get_key(i); }, (int)len, leff, hist, scratch, shared, &T, &keq);
+
+    // compaction in key-index order over thread-contiguous segments
+    const int64_t seg = (len + ITEM_BLOCK - 1) / ITEM_BLOCK;
+    const int64_t lo = min((int64_t)threadIdx.x * seg, len);
+    const int64_t hi = min(lo + seg, len);
+    uint32_t gt = 0, eq = 0;
+    for (int64_t n = lo; n < hi; ++n) {
+      const uint32_t k = get_key(n);
+      gt += k > T;
+      eq += k == T;
+    }
+    const uint32_t eq_before = block_excl_scan<ITEM_BLOCK>(eq, scratch, nullptr);
+    const int take_eq = max(0, min((int)eq, keq - (int)eq_before));
+    uint32_t pos = block_excl_scan<ITEM_BLOCK>(gt + (uint32_t)take_eq, scratch, nullptr);
+    int taken = 0;
+    for (int64_t n = lo; n < hi; ++n) {
+      const uint32_t k = get_key(n);
+      if (k > T) {
+        set_slot(pos++, n);
+      } else if (k == T && taken < take_eq) {
+        set_slot(pos++, n);
+        ++taken;
+      }
+    }
+    __syncthreads();
+  }
 
   // exact low-rank rescore of the shortlist (torch's sum order)
   const float* kl = p.k_low + (int64_t)h * p.klow_hs + off * p.R;
   int32_t* out_idx = p.sl_idx + (int64_t)item * p.L;
   float* out_rank = p.sl_rank + (int64_t)item * p.L;
-  if (r64 && ((uintptr_t)kl & 15u) == 0) {  // block-uniform
+  if ((flags & 8) != 0) {
+    for (int j = threadIdx.x; j < leff; j += ITEM_BLOCK) out_idx[j] = (int32_t)slot(j);
+  } else if (r64 && ((uintptr_t)kl & 15u) == 0) {  // block-uniform
     // lane octet o takes shortlist entries o, o + 128, ...: eight lanes per
     // row, two 16-byte loads each (a row's two 128-byte lines), REG_OCT
     // rows in flight; rank_dot64_oct8 sums in torch_order_dot64's order
@@ -235,6 +365,51 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   if (threadIdx.x == 0) p.sl_count[item] = leff;
 }
 
+
+// The rank scores of shortlists (rank_dot64_oct8, R = 64) over the whole chip:
+// a workgroup per RS_PER entries of an item.  Few items with long shortlists
+// are bound by the rows they gather, and one CU an item reads them at a CU's
+// rate: 72 items of 8192 rows (151 MB) 34 us here, in the item kernel 48
+// of its 92.
+constexpr int RS_BLOCK = 256;
+constexpr int RS_PER = 512;
+constexpr int64_t RS_MAX_ITEMS = 128;  // items up to half the CUs
+constexpr int RS_MIN_L = 2048;         // and shortlists of at least four workgroups
+
+__global__ void __launch_bounds__(RS_BLOCK) rescore_kernel(SummonParams p) {
+#pragma clang fp contract(off)
+  const int item = blockIdx.y;
+  const int h = (item / p.Q) % p.H, b = item / (p.Q * p.H);
+  const int leff = p.sl_count[item];
+  const int j0 = (int)blockIdx.x * RS_PER, j1 = min(leff, j0 + RS_PER);
+  if (j0 >= j1) return;
+  const float* kl = p.k_low + (int64_t)h * p.klow_hs + (p.offs ? p.offs[b] : 0) * 64;
+  const int oct = (int)threadIdx.x >> 3, c = (int)threadIdx.x & 7;
+  const float4* q4 = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * 64);
+  const float4 q0 = q4[c], q1 = q4[8 + c];
+  const float4* kl4 = reinterpret_cast<const float4*>(kl);
+  const int32_t* idx = p.sl_idx + (int64_t)item * p.L;
+  float* out = p.sl_rank + (int64_t)item * p.L;
+  constexpr int U = 8, STEP = RS_BLOCK / 8;
+  static_assert(RS_PER % (U * STEP) == 0, "whole rounds");
+  for (int r = j0; r < j1; r += U * STEP) {
+    int64_t n[U];
+    float4 r0[U], r1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) n[u] = idx[min(r + u * STEP + oct, j1 - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      r0[u] = kl4[n[u] * 16 + c];
+      r1[u] = kl4[n[u] * 16 + 8 + c];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = r + u * STEP + oct;
+      const float dot = rank_dot64_oct8(r0[u], r1[u], q0, q1);
+      if (c == 0 && j < j1) out[j] = dot * 0.125f;
+    }
+  }
+}
 
 // items: n_seq * H * Q; workgroups take head-major item ranges per XCD
 // (xcd_range_item), so one XCD's L2 holds the k_low rows of one or two heads.
@@ -286,13 +461,23 @@ int summon_regs_path(const SummonParams& p, int64_t items, hipStream_t stream) {
 
 int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream) {
   const bool idx16 = p.N <= 65536;  // every sequence's length is at most N
-  const bool keys_fit = item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, idx16).total <= kMaxLds;
-  const ItemLds layout = item_lds_layout(p.S, p.C, p.R, p.L, p.N, keys_fit, idx16);
+  const bool lin_fit = p.N <= (int64_t)LIN_ITERS * ITEM_BLOCK &&
+                       item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, idx16, true).total <= kMaxLds;
+  const bool keys_fit = lin_fit || (p.N <= kMaxLds / 4 &&
+                                    item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, idx16, false).total <= kMaxLds);
+  const ItemLds layout = item_lds_layout(p.S, p.C, p.R, p.L, p.N, keys_fit, idx16, lin_fit);
   SVA_UNSUPPORTED(layout.total <= kMaxLds, "sva_summon: shortlist %d with %dx%d codes exceeds LDS", p.L, p.S, p.C);
+  const bool apart = items <= RS_MAX_ITEMS && p.L >= RS_MIN_L && p.R == 64 && ((uintptr_t)p.k_low & 15u) == 0 &&
+                     p.klow_hs % 4 == 0 && ((uintptr_t)p.q_low & 15u) == 0;
   SVA_SET_MAX_LDS_ONCE(summon_item_kernel, kMaxLds, "hipFuncSetAttribute(summon_item_kernel)");
   hipLaunchKernelGGL(summon_item_kernel, dim3((unsigned)items), dim3(ITEM_BLOCK), (size_t)layout.total, stream, p,
-                     (keys_fit ? 1 : 0) | (idx16 ? 2 : 0));
+                     (keys_fit ? 1 : 0) | (idx16 ? 2 : 0) | (lin_fit ? 4 : 0) | (apart ? 8 : 0));
   SVA_CHECK_LAUNCH("summon_item_kernel");
+  if (apart) {
+    hipLaunchKernelGGL(rescore_kernel, dim3((unsigned)((p.L + RS_PER - 1) / RS_PER), (unsigned)items), dim3(RS_BLOCK), 0,
+                       stream, p);
+    SVA_CHECK_LAUNCH("rescore_kernel");
+  }
   return SVA_OK;
 }
 

@@ -86,3 +86,49 @@ def test_multi_equals_item_path(device, n_seq, Q, lens, S, C, H, L, B, few, mask
     np.testing.assert_array_equal(got[0][item, :cnt].cpu().numpy(), want)
     ranks = oracle.rank_scores(k_low[0, o:].cpu().numpy(), want, ql, 64)
     np.testing.assert_array_equal(got[1][item, :cnt].cpu().numpy().view(np.uint32), ranks.view(np.uint32))
+
+
+@pytest.mark.parametrize("N,S,C,L,kind", [
+    (32768, 2, 256, 8192, "plain"),     # keys and bins in LDS, the batch decode's shape
+    (33001, 4, 64, 8192, "plain"),      # the last round of 1024 keys partial
+    (35500, 2, 256, 512, "plain"),      # about the longest cache with its keys in LDS
+    (39000, 2, 64, 16, "plain"),        # keys in LDS without room for the bins: radix passes
+    (20000, 1, 256, 4000, "plain"),     # 256 scores: boundary bins of 80 equal keys
+    (20000, 2, 256, 4000, "few"),       # three codes: a boundary bin of thousands, radix passes
+    (5000, 2, 256, 4999, "plain"),      # all but one key
+    (3000, 2, 256, 8192, "plain"),      # every key
+    (17000, 2, 256, 5000, "wide"),      # a table with an infinity: no finite bounds, radix passes
+    (17000, 2, 256, 5000, "mask"),      # a float mask
+])
+def test_item_select_matches_oracle(device, N, S, C, L, kind):
+    """One workgroup an item (shortlists past the multi path's 3584, or masked): shortlist in key order against
+    the oracle, ranks bit for bit."""
+    from sva_amd import kernels
+
+    H, Q = 2, 2
+    g = torch.Generator(device=device).manual_seed(N + L)
+    codes = torch.randint(0, 3 if kind == "few" else C, (H, N, S), device=device, generator=g).to(torch.uint8)
+    k_low = torch.randn(H, N, 64, device=device, generator=g)
+    q_low = torch.randn(1, H, Q, 64, device=device, generator=g)
+    cb = torch.randn(H, S, C, 64 // S, device=device, generator=g)
+    eye = torch.eye(64, device=device).expand(H, 64, 64).contiguous()
+    q_low, lut, rng = kernels.query_lut(q_low, eye, torch.ones(H, device=device), cb)
+    if kind == "wide":
+        lut[0, 0, 0, 0, 7] = float("inf")
+        rng[0, 0, 0, 1] = float("inf")
+    mask = None
+    if kind in ("mask", "plain") and L <= 3584 or kind == "mask":
+        keep = torch.rand(Q, N, device=device, generator=g) < (0.5 if kind == "mask" else 2.0)
+        mask = torch.where(keep, 0.0, torch.finfo(torch.float32).min)[None, None]
+    idx, rank, count = kernels.summon(lut, rng, q_low, codes, k_low, N, L, mask=mask)
+    torch.cuda.synchronize()
+    for h in range(H):
+        for t in range(Q):
+            scores = oracle.pq_scores_from_lut(lut[0, h, t].cpu().numpy(), codes[h].cpu().numpy(), 64)
+            ok = np.arange(N) <= N - Q + t if mask is None else (mask[0, 0, t] > -1e4).cpu().numpy()
+            want = np.sort(oracle.topk(scores, L, allowed=ok))
+            n = int(count[h * Q + t])
+            assert n == len(want)
+            np.testing.assert_array_equal(idx[h * Q + t, :n].cpu().numpy(), want)
+            ref = oracle.rank_scores(k_low[h].cpu().numpy(), want, q_low[0, h, t].cpu().numpy(), 64)
+            np.testing.assert_array_equal(rank[h * Q + t, :n].cpu().numpy().view(np.uint32), ref.view(np.uint32))
