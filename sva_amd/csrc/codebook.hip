@@ -16,7 +16,14 @@ using namespace sva;
 //   count = member count (or the sum of their weights)
 //   centroid = sums / count, or the previous centroid for an empty cell
 // with every sum taken in ascending key order (what index_add_ does on the CPU).
+// A cell is one serial chain of additions, bound by its loads: a member's id,
+// then its row.  CU_U members' ids and then their rows are requested together
+// (indices clamped to the last member) and added in order: nine heads of 16384
+// keys, 2x256, 27 us where one member after the other took 65 (the
+// first iterations' largest cells hold hundreds).
 namespace {
+
+constexpr int CU_U = 16;
 
 __global__ void __launch_bounds__(64) centroid_update_kernel(const float* __restrict__ x, int64_t x_hs, int R, int S,
                                                              int C, int64_t n_rows, const float* __restrict__ w,
@@ -36,15 +43,22 @@ __global__ void __launch_bounds__(64) centroid_update_kernel(const float* __rest
   const float* wh = w ? w + (int64_t)h * n_rows : nullptr;
   float acc = 0.0f, cnt = 0.0f;
   if (d < sub) {
-    for (int i = o0; i < o1; ++i) {
-      const int64_t n = mem[i];
-      const float v = xh[n * R + d];
-      if (wh) {
-        const float wn = wh[n];
-        acc = acc + wn * v;
-        cnt = cnt + wn;
-      } else {
-        acc = acc + v;
+    for (int i = o0; i < o1; i += CU_U) {
+      int64_t n[CU_U];
+      float v[CU_U], wn[CU_U];
+#pragma unroll
+      for (int u = 0; u < CU_U; ++u) n[u] = mem[min(i + u, o1 - 1)];
+#pragma unroll
+      for (int u = 0; u < CU_U; ++u) {
+        v[u] = xh[n[u] * R + d];
+        wn[u] = wh != nullptr ? wh[n[u]] : 1.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < CU_U; ++u) {
+        if (i + u < o1) {  // uniform
+          acc = wh != nullptr ? acc + wn[u] * v[u] : acc + v[u];
+          cnt = cnt + wn[u];
+        }
       }
     }
     if (!wh) cnt = (float)(o1 - o0);

@@ -94,3 +94,45 @@ def test_default_initialisation_is_seeded(device):
     assert torch.equal(a, b)
     small = codebooks.fit_product_codebooks(xt[:, :100], 2, 256, 1, seed=7)
     assert small.shape == (2, 2, 100, 32)  # min(codewords, rows) as the reference
+
+
+@pytest.mark.parametrize("N,C,code_dtype", [(1, 1, torch.uint8), (63, 5, torch.uint8), (1024, 256, torch.uint8),
+                                            (1025, 3, torch.int16), (16385, 1024, torch.int32), (40001, 200, torch.uint8)])
+def test_postings_wave_ranges(device, N, C, code_dtype):
+    """Rows that leave waves of the build empty, partial or with several rounds: cells in ascending key order."""
+    from sva_amd import inverted
+
+    g = torch.Generator(device=device).manual_seed(N + C)
+    codes = torch.randint(0, C, (2, N + 3, 2), device=device, generator=g).to(code_dtype)
+    post = inverted.build_postings(codes, N, C)
+    for h in range(2):
+        for s in range(2):
+            c = codes[h, :N, s].long()
+            counts = torch.bincount(c, minlength=C)
+            assert torch.equal(post.ids[h, s, :N].long(), torch.sort(c, stable=True).indices)
+            assert torch.equal(post.offsets[h, s, 1:].long(), counts.cumsum(0)) and int(post.offsets[h, s, 0]) == 0
+            assert int(post.max_count[h, s]) == int(counts.max())
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_centroid_update_cell_sizes(device, weighted):
+    """Cells of none to 49 members (batches of 16 with every remainder): sums in ascending key order, bit for bit."""
+    from sva_amd._lib import check, lib, ptr, stream_handle
+
+    C, sub = 50, 8
+    labels = torch.repeat_interleave(torch.arange(C), torch.arange(C))
+    labels = labels[torch.randperm(len(labels), generator=torch.Generator().manual_seed(1))]
+    n = len(labels)
+    g = torch.Generator().manual_seed(2)
+    x, w, prev = torch.randn(1, n, sub, generator=g), torch.rand(1, n, generator=g) + 0.1, torch.randn(1, 1, C, sub, generator=g)
+    from sva_amd import inverted
+
+    post = inverted.build_postings(labels.to(device, torch.uint8)[None, :, None].contiguous(), n, C)
+    xd, wd, pd, nxt = x.to(device), w.to(device), prev.to(device), torch.empty(1, 1, C, sub, device=device)
+    check(lib().sva_centroid_update(ptr(xd), xd.stride(0), n, 1, sub, 1, C, ptr(wd) if weighted else None,
+                                    ptr(post.offsets), ptr(post.ids), ptr(pd), ptr(nxt), stream_handle(xd.device)), "update")
+    rows = x[0] * w[0][:, None] if weighted else x[0]
+    total = torch.zeros(C, sub).index_add_(0, labels, rows)
+    count = torch.zeros(C).index_add_(0, labels, w[0]) if weighted else torch.bincount(labels, minlength=C).float()
+    want = torch.where(count[:, None] > 0, total / count.clamp_min(1e-30)[:, None], prev[0, 0])
+    assert torch.equal(nxt[0, 0].cpu(), want)
