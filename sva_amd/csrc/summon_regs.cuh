@@ -27,6 +27,35 @@ __host__ __device__ inline int align16(int x) { return (x + 15) & ~15; }
 // select writes it.
 constexpr int REG_MAX_L = 2048;
 
+// The rem-th largest (with repeats) of the cb <= TOP_SMALL keys in s.small into
+// s.shared[0], and how many keys equal to it are taken into s.shared[1] (the
+// caller synchronizes before and after).
+SVA_DEV void rank_last_bucket(const TopLds& s, uint32_t cb, int rem) {
+  const int t = (int)threadIdx.x;
+  // 16 lanes per key: lane g counts the bucket's keys 4g .. 4g+3 above
+  // it (low half) and at or above it (high half)
+  const int i = t >> 4, g = t & 15;
+  const uint32_t v = i < (int)cb ? (uint32_t)s.small[i] : 0u;
+  uint32_t cnt = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = 4 * g + j;
+    if (o < (int)cb) {
+      const uint32_t y = (uint32_t)s.small[o];
+      cnt += (y > v ? 1u : 0u) + (y >= v ? 0x10000u : 0u);
+    }
+  }
+  cnt += row_shr0<1>(cnt);
+  cnt += row_shr0<2>(cnt);
+  cnt += row_shr0<4>(cnt);
+  cnt += row_shr0<8>(cnt);
+  // keys equal to the rem-th largest write the same words
+  if (g == 15 && i < (int)cb && (cnt & 0xFFFFu) < (uint32_t)rem && (cnt >> 16) >= (uint32_t)rem) {
+    s.shared[0] = v;
+    s.shared[1] = (uint32_t)rem - (cnt & 0xFFFFu);
+  }
+}
+
 // The k-th largest 32-bit key among the nonzero composites of the slots (the
 // key is a composite's high word): T and need such that the k largest by
 // (key desc, index asc) are the elements with key > T and the first need
@@ -132,30 +161,7 @@ SVA_DEV void select_key_regs(const uint64_t (&e)[NPT], int slots, int k, uint32_
         }
       }
       __syncthreads();
-      {
-        // 16 lanes per key: lane g counts the bucket's keys 4g .. 4g+3 above
-        // it (low half) and at or above it (high half)
-        const int i = t >> 4, g = t & 15;
-        const uint32_t v = i < (int)cb ? (uint32_t)s.small[i] : 0u;
-        uint32_t cnt = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int o = 4 * g + j;
-          if (o < (int)cb) {
-            const uint32_t y = (uint32_t)s.small[o];
-            cnt += (y > v ? 1u : 0u) + (y >= v ? 0x10000u : 0u);
-          }
-        }
-        cnt += row_shr0<1>(cnt);
-        cnt += row_shr0<2>(cnt);
-        cnt += row_shr0<4>(cnt);
-        cnt += row_shr0<8>(cnt);
-        // keys equal to the rem-th largest write the same words
-        if (g == 15 && i < (int)cb && (cnt & 0xFFFFu) < (uint32_t)rem && (cnt >> 16) >= (uint32_t)rem) {
-          s.shared[0] = v;
-          s.shared[1] = (uint32_t)rem - (cnt & 0xFFFFu);
-        }
-      }
+      rank_last_bucket(s, cb, rem);
       __syncthreads();
       *T_out = s.shared[0];
       *need_out = (int)s.shared[1];
@@ -285,8 +291,27 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
       if ((okm >> i) & 1u) e[i] = cw[(int64_t)i * ITEM_BLOCK + threadIdx.x];
   }
   for (int e2 = threadIdx.x; e2 < SC; e2 += ITEM_BLOCK) tab[e2] = lsrc[e2];
+  // The shortlist's select starts with the scores: each key is counted, as it
+  // is scored, in one of 4096 bins linear in the table's bounds [lo, hi]; one
+  // scan gives the allowed keys and the bin of the L-th largest, whose few
+  // members are ranked.  The radix select (a pass over a thread's keys for
+  // their common bits, then one or two histogram passes) remains for bounds
+  // that are not finite and for bins of more than TOP_SMALL.  Bound by the
+  // wave's VALU issue, of which the radix select was a fifth: 4096 x 9 items
+  // of up to 8192 keys, 2x256, 2048 kept, 1911 us against 2211; up to 4096
+  // keys 1338 against 1434; the one-launch lookup at 8192 keys 43.2 against
+  // 45.5.
+  const float lo_s = p.range[4 * item] * inv_sqrt_r, hi_s = p.range[4 * item + 1] * inv_sqrt_r;
+  const float span = hi_s - lo_s;
+  const float inv_w = (float)TOP_BINS / span, b0 = -lo_s * inv_w;
+  const bool linear = span > 0.0f && span < INFINITY && inv_w < INFINITY;  // uniform
+  static_assert(TOP_BINS == 4 * ITEM_BLOCK, "four bins a thread");
+  // a non-decreasing function of the score (one rounding of an increasing one)
+  auto bin_of = [&](float v) {
+    return (uint32_t)__builtin_amdgcn_fmed3f(__builtin_fmaf(v, inv_w, b0), 0.0f, (float)(TOP_BINS - 1));
+  };
+  reinterpret_cast<uint4*>(tl.hist)[threadIdx.x] = uint4{0u, 0u, 0u, 0u};
   __syncthreads();
-  uint32_t kor = 0u, kand = 0xFFFFFFFFu;
   uint32_t cnt = 0;
 #pragma unroll
   for (int i = 0; i < NPT; ++i) {
@@ -307,15 +332,21 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
           acc = acc + tab[s * C + c];
         }
       }
-      const uint32_t key = f2key(acc * inv_sqrt_r);
-      e[i] = composite(key, (uint32_t)n);
-      kor |= key;
-      kand &= key;
-      ++cnt;
+      const float v = acc * inv_sqrt_r;
+      e[i] = composite(f2key(v), (uint32_t)n);
+      if (linear) atomicAdd(&tl.hist[bin_of(v)], 1u);
+      else ++cnt;
     }
   }
   uint32_t allowed_total;
-  block_excl_scan<ITEM_BLOCK>(cnt, tl.scratch, &allowed_total);
+  uint32_t hc[4] = {0u, 0u, 0u, 0u};  // bins 4 t .. 4 t + 3 counted from the top
+  if (linear) {
+    __syncthreads();
+    const uint4 hv = reinterpret_cast<const uint4*>(tl.hist)[ITEM_BLOCK - 1 - threadIdx.x];
+    hc[0] = hv.w, hc[1] = hv.z, hc[2] = hv.y, hc[3] = hv.x;
+    cnt = hc[0] + hc[1] + hc[2] + hc[3];
+  }
+  uint32_t above = block_excl_scan<ITEM_BLOCK>(cnt, tl.scratch, &allowed_total);
   const int leff = (int)min((uint32_t)p.L, allowed_total);
   const int beff = min(p.B, leff);
   if (threadIdx.x == 0) {
@@ -332,7 +363,49 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
   // (every allowed key when the shortlist takes them all)
   uint32_t T = 0u;
   int need = 0x7FFFFFFF;
-  if (leff < (int)allowed_total) select_key_regs<ITEM_BLOCK, NPT>(e, NPT, leff, kor, kand, tl, &T, &need);
+  if (leff < (int)allowed_total) {
+    bool found = false;
+    if (linear) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (above < (uint32_t)leff && above + hc[j] >= (uint32_t)leff) {
+          shared[0] = (uint32_t)(TOP_BINS - 1 - 4 * (int)threadIdx.x - j);
+          shared[1] = above;
+          shared[2] = hc[j];
+        }
+        above += hc[j];
+      }
+      if (threadIdx.x == 0) shared[3] = 0u;
+      __syncthreads();
+      const uint32_t bb = shared[0], cb = shared[2];
+      const int rem = leff - (int)shared[1];
+      found = cb <= (uint32_t)TOP_SMALL;
+      if (found) {
+#pragma unroll
+        for (int i = 0; i < NPT; ++i) {
+          const uint32_t key = (uint32_t)(e[i] >> 32);
+          if (((okm >> i) & 1u) && bin_of(key2f(key)) == bb) tl.small[atomicAdd(&shared[3], 1u)] = key;
+        }
+        __syncthreads();
+        rank_last_bucket(tl, cb, rem);
+        __syncthreads();
+        T = shared[0];
+        need = (int)shared[1];
+      }
+      __syncthreads();
+    }
+    if (!found) {
+      uint32_t kor = 0u, kand = 0xFFFFFFFFu;
+#pragma unroll
+      for (int i = 0; i < NPT; ++i) {
+        if ((okm >> i) & 1u) {
+          kor |= (uint32_t)(e[i] >> 32);
+          kand &= (uint32_t)(e[i] >> 32);
+        }
+      }
+      select_key_regs<ITEM_BLOCK, NPT>(e, NPT, leff, kor, kand, tl, &T, &need);
+    }
+  }
 
   // shortlist in ascending key order: slot-major (i, wave, lane) is key order
   compact_selected<ITEM_BLOCK, NPT>(e, NPT, T, need, wbase, tl.scratch, [&](int i, uint32_t pos) {

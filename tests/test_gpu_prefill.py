@@ -108,6 +108,34 @@ def test_fused_item_matches_split_calls(device, N, S, C, Q, L, B, few):
     _run(device, codes, k_low, q, q_proj, scale, cb, N, L, B)
 
 
+@pytest.mark.parametrize("N,S,C,L,kind", [
+    (1025, 2, 256, 1024, "plain"),    # one key past a round; all but one key kept
+    (4096, 2, 256, 1, "plain"),       # the best key alone: the topmost bin that holds one
+    (4097, 4, 64, 2048, "plain"),     # the first size with eight keys a thread
+    (8193, 1, 256, 1000, "plain"),    # 256 scores: boundary bins of about 32 equal keys, ranked
+    (16384, 1, 64, 1000, "plain"),    # boundary bins of 256 equal keys: the radix select
+    (16383, 2, 256, 2048, "outlier"), # one table entry 1e4 away: every other key in a few bins
+    (5000, 2, 256, 2048, "inf"),      # a table with an infinity: no finite bounds
+    (5000, 2, 256, 512, "flat"),      # every score the same: bounds of no width
+])
+def test_fused_item_select_matches_oracle(device, N, S, C, L, kind):
+    """The register path's shortlist select, bit for bit against the oracle on the table the kernel read."""
+    from sva_amd import kernels
+
+    codes, k_low, q, q_proj, scale, cb = _inputs(device, N, S, C, 2, H=2, seed=N % 29)
+    q_low, lut, rng = kernels.query_lut(*(torch.from_numpy(x).to(device) for x in (q, q_proj, scale, cb)))
+    if kind in ("outlier", "inf"):
+        v = 1e4 if kind == "outlier" else float("inf")
+        lut[0, :, :, 0, 7], rng[0, :, :, 1] = v, v + (0.0 if kind == "inf" else 100.0)
+    if kind == "flat":
+        lut.fill_(0.5)
+        rng[..., :2] = 0.5 * S
+    fused = kernels.summon_select(lut, rng, q_low, torch.from_numpy(codes).to(device), k_low, N, L, min(L, 300))
+    torch.cuda.synchronize()
+    _oracle_check(codes, k_low, [t.cpu().numpy() for t in fused], q_low.cpu().numpy(), lut.cpu().numpy(), L,
+                  min(L, 300), N)
+
+
 def test_fused_item_masks(device):
     # a float mask with different rows per token, and a bool mask
     N, S, C, Q = 5000, 2, 256, 3
