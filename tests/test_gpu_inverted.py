@@ -276,6 +276,35 @@ def test_ragged_static_decode_matches_oracle(device, amin, amid, budget):
         assert float(stats[items, 1].sum()) == ref["stats"]["refill_pool"], f"sequence {b}"
 
 
+@pytest.mark.parametrize("C,cells", [(8, 3), (2, 2), (256, 1), (32, 16)])
+def test_ragged_static_list_sizes(device, C, cells):
+    """Lists past one copy round of 512 ids, one list a subspace, empty cells, more lists than waves; a cell that
+    nothing is in."""
+    from sva_amd import inverted
+
+    cat = _ragged_catalog(device, RAGGED_LENS, C=C, seed=C + cells)
+    if C > 2:
+        codes = np.where(cat.codes == 1, 0, cat.codes)
+        cat.codes, cat.codes_t = codes, cat.t(codes)
+    plens = cat.lens - np.asarray(RAGGED_TAILS)
+    post = inverted.build_postings_ragged(cat.codes_t, cat.t(cat.offs), cat.t(plens), int(plens.max()), C)
+    out, fin_idx, fin_count, stats = inverted.ragged_static_decode(
+        cat.t(cat.q), cat.t(cat.q_proj), cat.t(cat.scale), cat.t(cat.cb), cat.t(cat.keys), cat.t(cat.values),
+        cat.k_low_t, cat.codes_t, cat.t(cat.offs), cat.t(cat.lens), post, int(max(RAGGED_TAILS)), 64, cells,
+        cat.D ** -0.5, return_selection=True)
+    fin_idx, fin_count, stats = fin_idx.cpu().numpy(), fin_count.cpu().numpy(), stats.cpu().numpy()
+    for b, (r0, n, pl) in enumerate(zip(cat.offs, cat.lens, plens)):
+        sl = slice(r0, r0 + n)
+        ql = oracle.query_low(cat.q[b], cat.q_proj, cat.scale)
+        ref = oracle.static_decode(cat.q[b], cat.keys[:, sl], cat.values[:, sl], ql, cat.k_low[:, sl], cat.cb,
+                                   oracle.rebuild_postings(cat.codes[:, r0:r0 + pl], C), int(pl), 64, cells,
+                                   cat.D ** -0.5)
+        for h in range(cat.H):
+            it = b * cat.H + h
+            np.testing.assert_array_equal(fin_idx[it, : fin_count[it]], np.sort(ref["heads"][h]["final"]))
+        assert float(stats[b * cat.H:(b + 1) * cat.H, 0].sum()) == ref["stats"]["summoned"], f"sequence {b}"
+
+
 def test_config5_packed_batch_static_decode(device):
     # The ragged continuous-batch workload at its real shape: 32 sequences
     # with cache lengths log-uniform in [4096, 131072] packed contiguously,
