@@ -60,17 +60,19 @@ SVA_DEV void rank_last_bucket(const TopLds& s, uint32_t cb, int rem) {
 // key is a composite's high word): T and need such that the k largest by
 // (key desc, index asc) are the elements with key > T and the first need
 // elements with key == T in ascending index order.  kor / kand: this
-// thread's OR / AND of its elements' keys.  Radix passes of up to 12 bits
+// thread's OR / AND of its elements' keys.  MASKED: the elements are slots i
+// with bit i of live only.  Radix passes of up to 12 bits
 // from the highest bit where the keys differ; a tie class costs no pass (the
 // caller's compaction takes its first need members), and a boundary bucket
 // of at most TOP_SMALL keys is ranked directly.  Every thread of the block
 // must call it.
-template <int BLOCK, int NPT>
+template <int BLOCK, int NPT, bool MASKED = false>
 SVA_DEV void select_key_regs(const uint64_t (&e)[NPT], int slots, int k, uint32_t kor, uint32_t kand,
-                             const TopLds& s, uint32_t* T_out, int* need_out) {
+                             const TopLds& s, uint32_t* T_out, int* need_out, uint32_t live = 0u) {
   static_assert(BLOCK == 4 * 256 && TOP_BINS == 4 * BLOCK, "one uint4 of bins per thread");
   static_assert(TOP_SMALL * 16 == BLOCK, "16 lanes per key of the last bucket");
   const int t = (int)threadIdx.x, lane = lane_id();
+  auto held = [&](int i) { return MASKED ? ((live >> i) & 1u) != 0u : e[i] != 0ull; };
 #pragma unroll
   for (int o = 1; o <= 8; o <<= 1) {
     const uint32_t ko = o == 1 ? row_shr_keep<1>(kor) : o == 2 ? row_shr_keep<2>(kor)
@@ -114,7 +116,7 @@ SVA_DEV void select_key_regs(const uint64_t (&e)[NPT], int slots, int k, uint32_
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
       const uint32_t key = (uint32_t)(e[i] >> 32);
-      if (i < slots && e[i] != 0ull && (key & pmask) == prefix) atomicAdd(&s.hist[(key >> shift) & dmask], 1u);
+      if (i < slots && held(i) && (key & pmask) == prefix) atomicAdd(&s.hist[(key >> shift) & dmask], 1u);
     }
     __syncthreads();
     // thread t owns bins 4t .. 4t+3 counted from the top
@@ -148,7 +150,7 @@ SVA_DEV void select_key_regs(const uint64_t (&e)[NPT], int slots, int k, uint32_
       for (int i = 0; i < NPT; ++i) {
         if (i < slots) {  // uniform
           const uint32_t key = (uint32_t)(e[i] >> 32);
-          const bool match = e[i] != 0ull && (key & pmask) == prefix;
+          const bool match = held(i) && (key & pmask) == prefix;
           const uint64_t m = __builtin_amdgcn_ballot_w64(match);
           if (m != 0ull) {
             uint32_t base = 0;
@@ -296,11 +298,12 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
   // scan gives the allowed keys and the bin of the L-th largest, whose few
   // members are ranked.  The radix select (a pass over a thread's keys for
   // their common bits, then one or two histogram passes) remains for bounds
-  // that are not finite and for bins of more than TOP_SMALL.  Bound by the
+  // that are not finite, and for the members of a bin of more than TOP_SMALL
+  // (a model's own keys share codes: tie classes of hundreds).  Bound by the
   // wave's VALU issue, of which the radix select was a fifth: 4096 x 9 items
   // of up to 8192 keys, 2x256, 2048 kept, 1911 us against 2211; up to 4096
   // keys 1338 against 1434; the one-launch lookup at 8192 keys 43.2 against
-  // 45.5.
+  // 45.5; a 30-layer model's prefill of 8192 tokens 0.146 s against 0.157.
   const float lo_s = p.range[4 * item] * inv_sqrt_r, hi_s = p.range[4 * item + 1] * inv_sqrt_r;
   const float span = hi_s - lo_s;
   const float inv_w = (float)TOP_BINS / span, b0 = -lo_s * inv_w;
@@ -365,6 +368,8 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
   int need = 0x7FFFFFFF;
   if (leff < (int)allowed_total) {
     bool found = false;
+    uint32_t live = okm;  // the keys the radix select takes, rem of them
+    int rem = leff;
     if (linear) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -378,15 +383,22 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
       if (threadIdx.x == 0) shared[3] = 0u;
       __syncthreads();
       const uint32_t bb = shared[0], cb = shared[2];
-      const int rem = leff - (int)shared[1];
+      rem = leff - (int)shared[1];
       found = cb <= (uint32_t)TOP_SMALL;
-      if (found) {
+      // the bin's members: gathered and ranked, or too many (a tie class
+      // costs the radix select no pass)
+      uint32_t in = 0;
 #pragma unroll
-        for (int i = 0; i < NPT; ++i) {
-          const uint32_t key = (uint32_t)(e[i] >> 32);
-          if (((okm >> i) & 1u) && bin_of(key2f(key)) == bb) tl.small[atomicAdd(&shared[3], 1u)] = key;
+      for (int i = 0; i < NPT; ++i) {
+        const uint32_t key = (uint32_t)(e[i] >> 32);
+        if (((okm >> i) & 1u) && bin_of(key2f(key)) == bb) {
+          in |= 1u << i;
+          if (found) tl.small[atomicAdd(&shared[3], 1u)] = key;
         }
-        __syncthreads();
+      }
+      live = in;
+      __syncthreads();
+      if (found) {
         rank_last_bucket(tl, cb, rem);
         __syncthreads();
         T = shared[0];
@@ -398,12 +410,12 @@ SVA_DEV int regs_item(const SummonParams& p, int item, unsigned char* lds) {
       uint32_t kor = 0u, kand = 0xFFFFFFFFu;
 #pragma unroll
       for (int i = 0; i < NPT; ++i) {
-        if ((okm >> i) & 1u) {
+        if ((live >> i) & 1u) {
           kor |= (uint32_t)(e[i] >> 32);
           kand &= (uint32_t)(e[i] >> 32);
         }
       }
-      select_key_regs<ITEM_BLOCK, NPT>(e, NPT, leff, kor, kand, tl, &T, &need);
+      select_key_regs<ITEM_BLOCK, NPT, true>(e, NPT, rem, kor, kand, tl, &T, &need, live);
     }
   }
 
