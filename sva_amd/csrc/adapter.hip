@@ -60,7 +60,10 @@ SVA_DEV float round_to(float v, int dtype) {
   return __half2float(__float2half_rn(v));
 }
 
-__host__ __device__ inline int adapter_row(int H) { return (2 * H + 3) & ~3; }  // floats of a staged token
+// Floats of a staged token: whole rounds of a wave's float4s, the last one's
+// tail zeros.  A lane past the last input multiplies a zero weight by such a
+// zero (by an input it would make a NaN of an infinity there).
+__host__ __device__ inline int adapter_row(int H) { return (2 * H + 4 * WAVE - 1) / (4 * WAVE) * (4 * WAVE); }
 
 template <int NT>
 __global__ void __launch_bounds__(AB) residual_adapter_kernel(AdapterParams p) {
@@ -135,7 +138,7 @@ __global__ void __launch_bounds__(AB) residual_adapter_kernel(AdapterParams p) {
           if (k0 + 4 * WAVE * u < H2) {  // uniform
 #pragma unroll
             for (int q = 0; q < NT; ++q) {
-              const float4 x = *reinterpret_cast<const float4*>(xs + q * XS + min(k, XS - 4));
+              const float4 x = *reinterpret_cast<const float4*>(xs + q * XS + k);
               acc[q] = __builtin_fmaf(x.x, dw[u].x, acc[q]);
               acc[q] = __builtin_fmaf(x.y, dw[u].y, acc[q]);
               acc[q] = __builtin_fmaf(x.z, dw[u].z, acc[q]);

@@ -72,6 +72,23 @@ def test_adapter_workgroup_shapes(device, T, H, rank, dtype, odd):
     assert err <= {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 2e-2}[dtype], f"rel err {err}"
 
 
+@pytest.mark.parametrize("T,H", [(3, 576), (300, 576), (2, 130), (1, 8192)])
+def test_adapter_keeps_an_infinity(device, T, H):
+    """An infinity among a token's last attention values meets its own weights only: with positive weights for it,
+    every output of that token is +infinity (never a NaN) and the other tokens' outputs are what they are without it."""
+    from sva_amd import kernels
+
+    g = torch.Generator(device=device).manual_seed(H)
+    h, a = (torch.randn(T, H, device=device, generator=g) for _ in range(2))
+    down, up = torch.rand(4, 2 * H, device=device, generator=g) + 0.1, torch.rand(H, 4, device=device, generator=g) + 0.1
+    plain = kernels.residual_adapter(h, a, down, up, 1.0)
+    a[T // 2, H - 2] = float("inf")
+    out = kernels.residual_adapter(h, a, down, up, 1.0)
+    assert bool((out[T // 2] == float("inf")).all())
+    rest = torch.arange(T, device=device) != T // 2
+    assert torch.equal(out[rest], plain[rest])
+
+
 class _Fixed(nn.Module):
     def __init__(self, out):
         super().__init__()
