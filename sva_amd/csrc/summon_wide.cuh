@@ -574,8 +574,9 @@ __host__ __device__ inline int list_span(int W) {  // W rounded up to a power of
   while (p < W) p <<= 1;
   return p;
 }
+constexpr int kCapEntries = 16384;  // of all an item's lists, unless each is at its least
 __host__ __device__ inline int wg_cap(int W) {
-  const int c = 16384 / list_span(W);
+  const int c = kCapEntries / list_span(W);
   return c < WG_CAP ? WG_CAP : (c > NW * KL_CAP ? NW * KL_CAP : c);
 }
 
@@ -2424,9 +2425,13 @@ inline size_t over_bytes(int64_t items, int64_t L) {
   return align256((size_t)items * sizeof(uint32_t)) + align256((size_t)(items * K) * sizeof(uint32_t)) +
          align256((size_t)(items * K * L) * sizeof(uint64_t));
 }
+// (The compact lists' entries are bounded by a size that only grows with W:
+// W wg_cap(W) itself drops where W passes a power of two, and a buffer sized
+// for a longer cache would be refused at a shorter one.)
+inline int64_t list_entries(int64_t W) { return std::max<int64_t>(kCapEntries, W * WG_CAP); }
 inline size_t counters_bytes(int64_t items, int64_t W) {
   return align256((size_t)(2 * items * W * NW) * sizeof(uint32_t)) + align256((size_t)(2 * items * W) * sizeof(uint32_t)) +
-         align256((size_t)(items * W * wg_cap((int)W)) * (sizeof(uint64_t) + sizeof(float)));
+         align256((size_t)(items * list_entries(W)) * (sizeof(uint64_t) + sizeof(float)));
 }
 
 // the scan waves' own lists (composites, then ranks), kp keys a thread

@@ -47,6 +47,19 @@ def test_abi_version_and_workspace_queries():
     assert lib.sva_verify_workspace_bytes(1, 9, 3, 1, 64, 512) > 0
 
 
+def _key_counts(most):
+    edges = {m + d for e in range(10, 23) for m in (1 << e, 3 << e, 16384 + (1 << e)) for d in (-1, 0, 1)}
+    return sorted(n for n in edges | set(range(16384, 80000, 509)) | set(range(80000, most, 49999)) if n <= most)
+
+
+@pytest.mark.parametrize("heads,shortlist", [(1, 64), (9, 512), (9, 2048), (32, 8192), (64, 2048)])
+def test_one_token_workspace_grows_with_the_cache(heads, shortlist):
+    """A buffer sized for a cache's capacity serves every shorter cache: the size never drops as keys are added."""
+    lib = _lib()
+    sizes = [lib.sva_summon_workspace_bytes(1, heads, 1, n, shortlist) for n in _key_counts(4 << 20)]
+    assert sizes == sorted(sizes)
+
+
 def test_summon_strategy_selection():
     lib = _lib()
     # 1M keys, q = 1, 4x64 codes: many workgroups per item
