@@ -635,15 +635,32 @@ constexpr int DK = 8;                // lists per group
 constexpr int DL_LISTS = DQ * DK;    // 512 lists: caches up to 1M keys
 constexpr int NPD = 7;              // dense slots per thread
 
-// Rank score of a 64-float k_low row in torch's sum order, computed here
-// for the all-keys path: rows r of sl, one 16-lane DPP row each.
+// Rank scores of the 64-float k_low rows sl[0 .. n) in torch's sum order,
+// computed here for the all-keys path: eight lanes a row, RANK_U rows of an
+// octet in flight (a row of 16 lanes at a time, one after another, took 25 us
+// for 2048 rows).
+constexpr int RANK_U = 4;
 SVA_DEV void rank_rows(const SummonParams& p, int item, const float* klow, const uint32_t* sl, int n, float* out) {
 #pragma clang fp contract(off)
-  const int j = lane_id() & 15;
-  const float4 qq = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * p.R)[j];
-  for (int r = threadIdx.x >> 4; r < n; r += SB / 16) {
-    const float dot = rank_dot64_row16(reinterpret_cast<const float4*>(klow + (int64_t)sl[r] * p.R)[j], qq);
-    if (j == 0) out[r] = dot * kInvSqrtR;
+  const int oct = (int)threadIdx.x >> 3, c = (int)threadIdx.x & 7;
+  const float4* q4 = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * 64);
+  const float4* kl4 = reinterpret_cast<const float4*>(klow);
+  const float4 q0 = q4[c], q1 = q4[8 + c];
+  constexpr int STEP = SB / 8;
+  for (int r0 = 0; r0 < n; r0 += RANK_U * STEP) {  // uniform: the sums cross a row's octets
+    float4 a[RANK_U], b[RANK_U];
+#pragma unroll
+    for (int u = 0; u < RANK_U; ++u) {
+      const int64_t row = sl[min(r0 + u * STEP + oct, n - 1)];
+      a[u] = kl4[row * 16 + c];
+      b[u] = kl4[row * 16 + 8 + c];
+    }
+#pragma unroll
+    for (int u = 0; u < RANK_U; ++u) {
+      const float dot = rank_dot64_oct8(a[u], b[u], q0, q1);
+      const int r = r0 + u * STEP + oct;
+      if (c == 0 && r < n) out[r] = dot * kInvSqrtR;
+    }
   }
 }
 
@@ -1262,78 +1279,126 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
 // of them: no key outside a slice's top leff can be among the item's top
 // leff) and finishes the item.  No workgroup waits for another.
 //
-// A slice is selected in two passes over its codes, read as 16-byte words,
-// sixteen per thread in flight with every load instruction of a wave covering
-// 1 KB in a row, and scored from the table in LDS exactly as the scan scores
-// them:
+// A slice is selected in three passes over its codes, read as 16-byte words,
+// eight per thread in flight (the last pass: two) with every load instruction
+// of a wave covering 1 KB in a row, and scored from the table in LDS exactly
+// as the scan scores them:
 //   pass 1: histogram of the scores over 4096 bins linear in [lo, hi] (the
 //           bounds of any sum); b = the bin holding the k-th largest;
-//   pass 2: composites of higher bins (fewer than k) into a list, bin b's
-//           members (at most kOverBound) into LDS, sorted descending: the
-//           first `need` of them complete the list, which is then sorted into
-//           key order.
-// A boundary bin beyond kOverBound members (a tie class) falls back to the
-// radix select over the slice.
+//   pass 2: bin b's members into LDS, the k-th largest composite X among them
+//           by direct counting, or a sort past SB of them;
+//   pass 3: the composites >= X in key order, SB words at a time placed by
+//           one scan of the threads' counts.
+// A boundary bin beyond kOverBound members (a tie class) takes X by radix
+// passes over the bin's members instead.
 constexpr int kOverBound = 4096;     // boundary-bin members sorted in LDS
-constexpr int kOverWords = 16;       // code words per thread in flight
+constexpr int kOverWords = 8;        // code words per thread in flight
 constexpr int kOverSlicesMax = 16;   // slices per item
 constexpr int kOverGrid = 256;       // items * slices at most (one workgroup per CU)
-constexpr size_t kOverList = kFinSl;                                    // uint64[FIN_MAX_L] slice list
-constexpr size_t kOverBnd = kOverList + sizeof(uint64_t) * FIN_MAX_L;   // uint64[kOverBound]
+constexpr int kOverSlice = 65536;    // keys that are worth a slice
+constexpr size_t kOverBnd = kFinRk;  // uint64[kOverBound]
 static_assert(kOverBnd + sizeof(uint64_t) * kOverBound <= kFinSmall, "slice select LDS below the table");
 
-// Slices of the all-keys select for `items` items.
+// Slices of the all-keys select for `items` items (over_used: of an item of N keys).
 inline int over_slices(int64_t items) { return (int)std::max<int64_t>(1, std::min<int64_t>(kOverSlicesMax, kOverGrid / items)); }
+
+// A slice's fixed part and the merge of the slices cost more than a pass over
+// 65536 keys: a shorter item is one slice.
+SVA_DEV int over_used(int N, int K) { return min(K, max(1, (N + kOverSlice - 1) / kOverSlice)); }
 
 // Keys per slice: a multiple of 16, so every slice starts on a 16-byte code word.
 SVA_DEV int slice_keys(int N, int K) { return ((((N + K - 1) / K) + 15) / 16) * 16; }
 
-// Composite <-> (key index, score key) in key-major order, for sorting by key.
-SVA_DEV uint64_t by_key(uint64_t x) { return ((uint64_t)composite_index(x) << 32) | (x >> 32); }
-SVA_DEV uint64_t from_key(uint64_t y) { return composite((uint32_t)y, (uint32_t)(y >> 32)); }
-
-// Calls f(key, composite) for every key of [n0, n1) (n0 a multiple of 16):
-// the exact scan score's composite, 0 for a key the mask excludes.
-template <int S, typename F>
-SVA_DEV void overshoot_visit(const SummonParams& p, const uint8_t* __restrict__ codes, const float* lut_l, int n0,
-                             int n1, F&& f) {
+// The score composites of keys [n0, n1) (n0 a multiple of 16) by code words:
+// word w holds KPW keys, word w0 + u * SB + t is thread t's u-th.
+template <int S>
+struct OverKeys {
+  static constexpr int KPW = 16 / S;  // keys per 16-byte code word
+  const SummonParams& p;
+  const uint8_t* codes;
+  const float* lut;  // LDS
+  int n1;
+  bool masked;
+  SVA_DEV OverKeys(const SummonParams& p_, const uint8_t* codes_, const float* lut_, int n1_)
+      : p(p_), codes(codes_), lut(lut_), n1(n1_),
+        masked(p_.mask_type == MASK_F32 || p_.mask_type == MASK_BF16 || p_.mask_type == MASK_F16) {}
+  SVA_DEV u32x4 load(int word) const {
+    const int base = word * KPW;
+    if (base + KPW <= n1) return code_word(codes + (int64_t)base * S);
+    uint32_t wv[4] = {0u, 0u, 0u, 0u};
+    for (int j = 0; j < KPW * S; ++j)
+      if (base + j / S < n1) wv[j >> 2] |= (uint32_t)codes[(int64_t)base * S + j] << (8 * (j & 3));
+    return u32x4{wv[0], wv[1], wv[2], wv[3]};
+  }
+  // key j of a word: the reference's exact score ((0 + T0[c0]) + T1[c1]) + ...
+  // then / sqrt(R); 0 past the keys and for a key the mask excludes
+  SVA_DEV uint64_t key(const u32x4& w, int word, int j) const {
 #pragma clang fp contract(off)
-  constexpr int KPW = 16 / S;  // keys per 16-byte code word
-  const int C = p.C;
-  const uint32_t cm = (uint32_t)(C - 1);
-  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
+    const int n = word * KPW + j;
+    if (n >= n1) return 0ull;
+    const uint32_t cm = (uint32_t)(p.C - 1);
+    float acc = 0.0f;
+#pragma unroll
+    for (int s2 = 0; s2 < S; ++s2) acc = acc + lut[s2 * p.C + min(byte_of(w, j * S + s2), cm)];
+    const bool ok = !masked || mask_allows(p.mask, n, p.mask_type);
+    return ok ? composite(f2key(acc * kInvSqrtR), (uint32_t)n) : 0ull;
+  }
+};
+
+// Calls f(composite) for every key of [n0, k.n1), 0 for one that the mask
+// excludes or past the keys; every lane of a wave makes every call together.
+template <int S, typename F>
+SVA_DEV void overshoot_visit(const OverKeys<S>& k, int n0, F&& f) {
+  constexpr int KPW = OverKeys<S>::KPW;
   // (a slice past a short item's keys starts at its last key's end, not on a word: nothing to visit)
-  const int wbeg = n0 / KPW, wend = n0 < n1 ? (n1 + KPW - 1) / KPW : wbeg;
-  // word w0 + u * SB + t for u < kOverWords: every load instruction of a wave reads 1 KB in a row
+  const int wbeg = n0 / KPW, wend = n0 < k.n1 ? (k.n1 + KPW - 1) / KPW : wbeg;
   for (int w0 = wbeg; w0 < wend; w0 += kOverWords * SB) {
     u32x4 w[kOverWords];
 #pragma unroll
-    for (int u = 0; u < kOverWords; ++u) {
-      const int base = (w0 + u * SB + (int)threadIdx.x) * KPW;
-      if (base + KPW <= n1) {
-        w[u] = code_word(codes + (int64_t)base * S);
-      } else {
-        uint32_t wv[4] = {0u, 0u, 0u, 0u};
-        for (int j = 0; j < KPW * S; ++j)
-          if (base + j / S < n1) wv[j >> 2] |= (uint32_t)codes[(int64_t)base * S + j] << (8 * (j & 3));
-        w[u] = u32x4{wv[0], wv[1], wv[2], wv[3]};
-      }
-    }
+    for (int u = 0; u < kOverWords; ++u)
+      if (w0 + u * SB < wend) w[u] = k.load(w0 + u * SB + (int)threadIdx.x);  // uniform
 #pragma unroll
     for (int u = 0; u < kOverWords; ++u) {
-      const int base = (w0 + u * SB + (int)threadIdx.x) * KPW;
+      if (w0 + u * SB < wend) {
 #pragma unroll
-      for (int j = 0; j < KPW; ++j) {
-        const int key = base + j;
-        if (key < n1) {
-          float acc = 0.0f;
-#pragma unroll
-          for (int s2 = 0; s2 < S; ++s2) acc = acc + lut_l[s2 * C + min(byte_of(w[u], j * S + s2), cm)];
-          const bool ok = !masked || mask_allows(p.mask, key, p.mask_type);
-          f(key, ok ? composite(f2key(acc * kInvSqrtR), (uint32_t)key) : 0ull);
-        }
+        for (int j = 0; j < KPW; ++j) f(k.key(w[u], w0 + u * SB + (int)threadIdx.x, j));
       }
     }
+  }
+}
+
+// The composites >= X of keys [n0, k.n1), at most `most` of them, in key
+// order to out.
+template <int S>
+SVA_DEV void overshoot_emit(const OverKeys<S>& k, int n0, uint64_t X, uint32_t most, uint32_t* scratch,
+                            uint64_t* __restrict__ out) {
+  constexpr int KPW = OverKeys<S>::KPW;
+  const int wbeg = n0 / KPW, wend = n0 < k.n1 ? (k.n1 + KPW - 1) / KPW : wbeg;
+  uint32_t carry = 0;
+  u32x4 next = k.load(wbeg + (int)threadIdx.x);
+#pragma unroll 1
+  for (int w0 = wbeg; w0 < wend; w0 += SB) {
+    const int word = w0 + (int)threadIdx.x;
+    const u32x4 w = next;
+    next = k.load(word + SB);
+    uint64_t x[KPW];
+    uint32_t c = 0;
+#pragma unroll
+    for (int j = 0; j < KPW; ++j) {
+      x[j] = k.key(w, word, j);
+      if (x[j] < X) x[j] = 0ull;  // X is a composite, so not 0
+      c += x[j] != 0ull;
+    }
+    uint32_t total;
+    uint32_t o = carry + block_excl_scan<SB>(c, scratch, &total);
+#pragma unroll
+    for (int j = 0; j < KPW; ++j) {
+      if (x[j] != 0ull) {
+        if (o < most) out[o] = x[j];
+        ++o;
+      }
+    }
+    carry += total;
   }
 }
 
@@ -1396,106 +1461,110 @@ SVA_DEV Boundary hist_boundary(const uint32_t* hist, uint32_t k, uint32_t* scrat
   return r;
 }
 
-// Exact composite of key n (0 when masked out), scalar: the tie-class fallback's visitor.
-SVA_DEV uint64_t key_composite(const SummonParams& p, const uint8_t* codes, const float* lut_l, int n) {
-#pragma clang fp contract(off)
-  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
-  if (masked && !mask_allows(p.mask, n, p.mask_type)) return 0ull;
-  // the reference's exact score ((0 + T0[c0]) + T1[c1]) + ... then / sqrt(R)
-  float acc = 0.0f;
-  for (int s2 = 0; s2 < p.S; ++s2) {
-    uint32_t c = codes[(int64_t)n * p.S + s2];
-    c = c < (uint32_t)p.C ? c : (uint32_t)(p.C - 1);
-    acc = acc + lut_l[s2 * p.C + c];
+// The k-th largest of the cnt <= kOverBound composites in bnd (LDS; sorted in
+// place past SB of them); every thread must call it.
+SVA_DEV uint64_t kth_of(uint64_t* bnd, uint32_t cnt, uint32_t k, uint64_t* shared64) {
+  const int t = threadIdx.x;
+  if (cnt <= (uint32_t)SB) {  // a thread a member counts those above it
+    if (t < (int)cnt) {
+      const uint64_t x = bnd[t];
+      uint32_t above = 0;
+      for (uint32_t o = 0; o < cnt; ++o) above += bnd[o] > x ? 1u : 0u;
+      if (above == k - 1u) shared64[0] = x;
+    }
+    __syncthreads();
+    const uint64_t X = shared64[0];
+    __syncthreads();
+    return X;
   }
-  return composite(f2key(acc * kInvSqrtR), (uint32_t)n);
+  int P = 1;
+  while (P < (int)cnt) P <<= 1;
+  for (int i = (int)cnt + t; i < P; i += SB) bnd[i] = 0ull;
+  __syncthreads();
+  lds_bitonic<uint64_t, true>(bnd, P);
+  const uint64_t X = bnd[k - 1u];
+  __syncthreads();
+  return X;
 }
 
 // The top min(k, allowed) composites of keys [n0, n1) of an item, in key
 // order, to out (global); returns their number (block-uniform).
 template <int S>
-SVA_DEV uint32_t slice_select(const SummonParams& p, int item, const uint8_t* codes, uint32_t k, int n0, int n1, const float* lut_l,
-                              unsigned char* lds, uint32_t* scratch, uint32_t* shared, uint64_t* shared64,
-                              uint64_t* __restrict__ out) {
+SVA_DEV uint32_t slice_select(const SummonParams& p, int item, const uint8_t* codes, uint32_t k, int n0, int n1,
+                              const float* lut_l, unsigned char* lds, uint32_t* scratch, uint32_t* shared,
+                              uint64_t* shared64, uint64_t* __restrict__ out) {
   const int t = threadIdx.x;
   uint32_t* hist = (uint32_t*)(lds + kFinHist);
-  uint64_t* lst = (uint64_t*)(lds + kOverList);
   uint64_t* bnd = (uint64_t*)(lds + kOverBnd);
+  const OverKeys<S> keys(p, codes, lut_l, n1);
   const float lo = p.range[4 * item] * kInvSqrtR, hi = p.range[4 * item + 1] * kInvSqrtR;
   const float inv_w = lin_scale(lo, hi);
+  auto bin_of = [&](uint64_t x) { return (uint32_t)lin_bin(key2f((uint32_t)(x >> 32)), lo, inv_w); };
   reinterpret_cast<uint4*>(hist)[t] = uint4{0u, 0u, 0u, 0u};
+  if (t == 0) shared64[1] = 0ull;  // boundary-bin members
   __syncthreads();
-  overshoot_visit<S>(p, codes, lut_l, n0, n1, [&](int, uint64_t x) {
-    if (x != 0ull) atomicAdd(&hist[lin_bin(key2f((uint32_t)(x >> 32)), lo, inv_w)], 1u);
-  });
-  __syncthreads();
-  const Boundary bd = hist_boundary(hist, k, scratch, shared);
-  if (bd.k == 0u) return 0u;
-  if (bd.cnt > (uint32_t)kOverBound) {
-    // a tie class beyond the LDS sort: radix passes over the slice, then its keys >= X in key order
-    uint32_t(*whist)[256] = (uint32_t(*)[256])hist;
-    auto visit = [&](auto&& f) {
-      for (int n = n0 + t; n < n1; n += SB) {
-        const uint64_t x = key_composite(p, codes, lut_l, n);
-        if (x != 0ull) f(x);
+  Boundary bd{};
+  uint64_t vor = 0ull, vand = ~0ull;
+#pragma unroll 1
+  for (int pass = 1; pass <= 2; ++pass) {  // one copy of the visit's code
+    overshoot_visit<S>(keys, n0, [&](uint64_t x) {
+      const uint32_t bin = bin_of(x);
+      if (pass == 1) {
+        if (x != 0ull) atomicAdd(&hist[bin], 1u);
+        return;
       }
-    };
-    const uint64_t X = select_largest<SB>(visit, (int)bd.k, whist, scratch, shared64, shared);
-    const int per = (n1 - n0 + SB - 1) / SB;
-    const int m0 = min(n1, n0 + t * per), m1 = min(n1, m0 + per);
-    uint32_t cnt = 0;
-    for (int n = m0; n < m1; ++n) cnt += key_composite(p, codes, lut_l, n) >= X;
-    uint32_t o = block_excl_scan<SB>(cnt, scratch, nullptr);
-    for (int n = m0; n < m1; ++n) {
-      const uint64_t x = key_composite(p, codes, lut_l, n);
-      if (x >= X && o < bd.k) out[o++] = x;
+      const bool in = x != 0ull && bin == bd.b;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+      if (m == 0ull) return;
+      if (in) {
+        vor |= x;
+        vand &= x;
+      }
+      if (bd.cnt <= (uint32_t)kOverBound) {
+        uint32_t base = 0;
+        if (lane_id() == 0) base = atomicAdd((uint32_t*)&shared64[1], (uint32_t)__popcll(m));
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        if (in) bnd[base + lanes_below(m)] = x;
+      }
+    });
+    __syncthreads();
+    if (pass == 1) {
+      bd = hist_boundary(hist, k, scratch, shared);
+      if (bd.k == 0u) return 0u;
     }
-    return bd.k;
   }
-  if (t == 0) {
-    shared[0] = 0u;       // boundary-bin members
-    scratch[SNW] = 0u;    // higher-bin composites
-  }
-  __syncthreads();
-  overshoot_visit<S>(p, codes, lut_l, n0, n1, [&](int, uint64_t x) {
-    if (x == 0ull) return;
-    const uint32_t bin = (uint32_t)lin_bin(key2f((uint32_t)(x >> 32)), lo, inv_w);
-    if (bin > bd.b) lst[atomicAdd(&scratch[SNW], 1u)] = by_key(x);
-    else if (bin == bd.b) bnd[atomicAdd(&shared[0], 1u)] = x;
-  });
-  __syncthreads();
-  int P = 1;
-  while (P < (int)bd.cnt) P <<= 1;
-  for (int i = (int)bd.cnt + t; i < P; i += SB) bnd[i] = 0ull;
-  __syncthreads();
-  lds_bitonic<uint64_t, true>(bnd, P);
-  // the higher bins' composites, then the best `need` of the boundary bin, sorted by key
   const uint32_t need = bd.k - bd.above;
-  for (int i = t; i < (int)need; i += SB) lst[bd.above + i] = by_key(bnd[i]);
-  int PL = 1;
-  while (PL < (int)bd.k) PL <<= 1;
-  for (int i = (int)bd.k + t; i < PL; i += SB) lst[i] = ~0ull;
-  __syncthreads();
-  lds_bitonic<uint64_t, false>(lst, PL);
-  for (int i = t; i < (int)bd.k; i += SB) out[i] = from_key(lst[i]);
+  uint64_t X;
+  if (bd.cnt <= (uint32_t)kOverBound) {
+    X = kth_of(bnd, bd.cnt, need, shared64);
+  } else {
+    auto members = [&](auto&& f) {
+      overshoot_visit<S>(keys, n0, [&](uint64_t x) {
+        if (x != 0ull && bin_of(x) == bd.b) f(x);
+      });
+    };
+    X = select_largest_with_bounds<SB>(members, (int)need, vor, vand, (uint32_t(*)[256])hist, scratch, shared64, shared);
+    __syncthreads();
+  }
+  overshoot_emit<S>(keys, n0, X, bd.k, scratch, out);
   return bd.k;
 }
 
 // The item's leff largest composites among its K slice lists (key order
 // within a list, lists in key-range order), as key indices in key order into
 // sl (LDS).  offs: LDS uint32[K + 1].
-SVA_DEV void merge_slices(const WideArgs& a, int item, uint32_t leff, unsigned char* lds, uint32_t* sl, uint32_t* offs,
-                          uint32_t* scratch, uint32_t* shared, uint64_t* shared64) {
+SVA_DEV void merge_slices(const WideArgs& a, int item, int K, uint32_t leff, unsigned char* lds, uint32_t* sl,
+                          uint32_t* offs, uint32_t* scratch, uint32_t* shared, uint64_t* shared64) {
   const SummonParams& p = a.p;
-  const int t = threadIdx.x, K = a.K;
+  const int t = threadIdx.x;
   uint32_t* hist = (uint32_t*)(lds + kFinHist);
   uint64_t* bnd = (uint64_t*)(lds + kOverBnd);
-  const uint64_t* lists = a.slice_list + (int64_t)item * K * p.L;
+  const uint64_t* lists = a.slice_list + (int64_t)item * a.K * p.L;
   if (t == 0) {
     uint32_t o = 0u;
     for (int j = 0; j < K; ++j) {
       offs[j] = o;
-      o += a.slice_n[(int64_t)item * K + j];
+      o += a.slice_n[(int64_t)item * a.K + j];
     }
     offs[K] = o;
   }
@@ -1525,13 +1594,7 @@ SVA_DEV void merge_slices(const WideArgs& a, int item, uint32_t leff, unsigned c
         if ((uint32_t)lin_bin(key2f((uint32_t)(x >> 32)), lo, inv_w) == bd.b) bnd[atomicAdd(&shared[0], 1u)] = x;
       });
       __syncthreads();
-      int P = 1;
-      while (P < (int)bd.cnt) P <<= 1;
-      for (int i = (int)bd.cnt + t; i < P; i += SB) bnd[i] = 0ull;
-      __syncthreads();
-      lds_bitonic<uint64_t, true>(bnd, P);
-      X = bnd[leff - bd.above - 1];
-      __syncthreads();
+      X = kth_of(bnd, bd.cnt, leff - bd.above, shared64);
     }
   }
   // composites >= X in key order: thread t takes entries [t c, (t + 1) c) of the lists laid end to end
@@ -1786,8 +1849,9 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   } else {
     // all keys: the sampled floor overshot; this workgroup selects slice `slice`
     dense = false;
+    const int N = it.n, K = over_used(N, a.K);
+    if (slice >= K) return -1;
     if (t == 0 && slice == 0 && a.overshoot != nullptr) a.overshoot[item] = 1;
-    const int N = it.n, K = a.K;
     const uint8_t* codes = item_codes(p, it);
     // the item's table in LDS: the slice select scores every key of the slice from it
     float* lut_l = (float*)(lds + kFinLut);
@@ -1796,7 +1860,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     __syncthreads();
     const int per = slice_keys(N, K);
     const int n0 = min(N, slice * per), n1 = min(N, n0 + per);
-    uint64_t* out = a.slice_list + ((int64_t)item * K + slice) * p.L;
+    uint64_t* out = a.slice_list + ((int64_t)item * a.K + slice) * p.L;
     uint32_t nj;
     switch (p.S) {
       case 1: nj = slice_select<1>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
@@ -1804,19 +1868,25 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
       case 4: nj = slice_select<4>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
       default: nj = slice_select<8>(p, item, codes, (uint32_t)leff, n0, n1, lut_l, lds, scratch, shared, shared64, out); break;
     }
-    // publish the slice (release), then count it in; the item's last slice finishes the item
-    if (t == 0) a.slice_n[(int64_t)item * K + slice] = nj;
-    __threadfence();
+    // publish the slice (release), then count it in; the item's last slice
+    // finishes the item.  An item of one slice has nobody to tell: device-wide
+    // fences by every wave of every workgroup (L2 write-backs and invalidates)
+    // took most of a full chip's time (2304 items of 16400 keys, 2x256, 3584
+    // kept: 2384 us a call with them, 902 without, 771 with idle words skipped
+    // and ranks by octets).
+    if (t == 0) a.slice_n[(int64_t)item * a.K + slice] = nj;
     __syncthreads();
-    if (t == 0) {
-      const uint32_t done = atomicAdd(&a.arrive[item], 1u);
-      __threadfence();
-      shared[0] = done == (uint32_t)(K - 1) ? 1u : 0u;
+    if (K > 1) {
+      if (t == 0) {
+        __threadfence();
+        const uint32_t done = atomicAdd(&a.arrive[item], 1u);
+        shared[0] = done == (uint32_t)(K - 1) ? 1u : 0u;
+      }
+      __syncthreads();
+      if (shared[0] == 0u) return -1;
+      __threadfence();  // acquire: the other slices' lists
     }
-    __syncthreads();
-    if (shared[0] == 0u) return -1;
-    __threadfence();  // acquire: the other slices' lists
-    merge_slices(a, item, (uint32_t)leff, lds, sl, lcnt, scratch, shared, shared64);
+    merge_slices(a, item, K, (uint32_t)leff, lds, sl, lcnt, scratch, shared, shared64);
     rank_rows(p, item, item_klow(p, it), sl, leff, (float*)rk);
   }
   // bounds of the emitted rank keys (direct and staged paths) for the budget select

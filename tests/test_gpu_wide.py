@@ -216,6 +216,39 @@ def test_wide_sampled_floor_overshoot(device):
                sl_rank.cpu().numpy(), sl_count.cpu().numpy(), L)
 
 
+@pytest.mark.parametrize("N,S,C,L,masked", [
+    (40000, 2, 256, 2048, False),   # one slice of the item's keys, a boundary bin of a few
+    (65536, 4, 64, 512, False), (65537, 4, 64, 512, False),  # the last size of one slice, the first of two
+    (131073, 2, 256, 2048, True),   # three slices, a mask that leaves half the keys
+    (300007, 8, 32, 2048, False),   # five slices, their lists merged
+    (40000, 2, 4, 3000, False),     # tie classes of about 2500: the boundary members are sorted
+    (40000, 2, 3, 1024, False),     # classes past 4096: radix passes over the boundary bin
+    (100003, 1, 16, 8000, False),   # one subspace: classes of 6250, codes at odd addresses
+    (33000, 2, 256, 8192, True),    # the largest shortlist
+])
+def test_all_keys_select_sizes(device, N, S, C, L, masked):
+    """A floor above every score leaves no candidate: the selection over every key, against the oracle, and in
+    ascending key order."""
+    from sva_amd import kernels
+
+    codes, k_low, q, q_proj, scale, cb = _setup(device, N, S, C, H=2, seed=N % 53 + S)
+    t = lambda a: torch.from_numpy(a).to(device)  # noqa: E731
+    q_low, lut, rng = kernels.query_lut(t(q), t(q_proj), t(scale), t(cb), t(codes), N, L)
+    rng[..., 2] = rng[..., 1].abs() * 2 + 1
+    mask = allowed = None
+    if masked:
+        allowed = np.random.default_rng(3).random(N) < 0.5
+        mask = torch.where(t(allowed), 0.0, torch.finfo(torch.float32).min)[None, None, None].contiguous()
+    out = [x.cpu().numpy() for x in kernels.summon_select(lut, rng, q_low, t(codes), k_low, N, L, 300, mask=mask)]
+    torch.cuda.synchronize()
+    _check(codes, k_low, q_low[0, :, 0].cpu().numpy(), lut[0, :, 0].cpu().numpy(), *out[:3], L, allowed=allowed)
+    for h in range(2):
+        c, b = int(out[2][h]), int(out[4][h])
+        assert b == min(300, c) and bool((np.diff(out[0][h, :c]) > 0).all())
+        keep = oracle.topk(out[1][h, :c], b, key_index=out[0][h, :c])
+        np.testing.assert_array_equal(out[3][h, :b], np.sort(out[0][h, :c][keep]))
+
+
 def test_wide_candidates_beyond_lds_stage(device):
     # 3 codewords over 2 subspaces at 1M keys: the top score class holds
     # ~1/9 of the keys, far more candidates than the select kernel stages in
