@@ -1875,11 +1875,12 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     // kept: 2384 us a call with them, 902 without, 771 with idle words skipped
     // and ranks by octets).
     if (t == 0) a.slice_n[(int64_t)item * a.K + slice] = nj;
+    if (K > 1) __threadfence();  // by every wave: a barrier alone does not wait for the others' stores
     __syncthreads();
     if (K > 1) {
       if (t == 0) {
-        __threadfence();
         const uint32_t done = atomicAdd(&a.arrive[item], 1u);
+        __threadfence();
         shared[0] = done == (uint32_t)(K - 1) ? 1u : 0u;
       }
       __syncthreads();
