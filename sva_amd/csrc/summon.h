@@ -152,7 +152,9 @@ int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_by
 // Several tokens or sequences over a long cache (see summon_wide_multi.hip).
 bool summon_multi_eligible(const SummonParams& p, int64_t items);
 size_t summon_multi_workspace_bytes(int64_t items, int64_t n_keys, int64_t L);
-int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, hipStream_t stream);
+bool summon_multi_taken(const SummonParams& p, int64_t items, const void* workspace, size_t workspace_bytes);
+int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, size_t workspace_bytes,
+                      hipStream_t stream);
 // One subspace of at most 256 codewords with a shortlist of at most
 // CLASS_MAX_L: the wide path selects by code class (no sampled floor needed).
 constexpr int CLASS_MAX_L = 7168;

@@ -633,10 +633,8 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
     if (rc == SVA_OK && fused != nullptr) *fused = with_fv;
     return rc;
   }
-  if (sl_idx != nullptr && sva::summon_multi_eligible(p, items) && workspace != nullptr &&
-      ((uintptr_t)workspace & 255u) == 0 &&
-      workspace_bytes >= sva::summon_multi_workspace_bytes(items, n_keys, L) && (Q > 1 || seq_offsets != nullptr))
-    return sva::summon_multi_path(p, items, workspace, (hipStream_t)stream);
+  if ((Q > 1 || seq_offsets != nullptr) && sva::summon_multi_taken(p, items, workspace, workspace_bytes))
+    return sva::summon_multi_path(p, items, workspace, workspace_bytes, (hipStream_t)stream);
   if (overshoot != nullptr) {  // the per-item paths use no sampled floor
     const int rc = sva::fill_i32(overshoot, items, 0, (hipStream_t)stream);
     if (rc != SVA_OK) return rc;

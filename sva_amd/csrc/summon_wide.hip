@@ -72,47 +72,75 @@ bool summon_multi_eligible(const SummonParams& p, int64_t items) {
 
 namespace {
 
-// Items a launch takes: the candidate lists of a group stay within MULTI_BYTES.
-int64_t multi_group(int64_t items, int64_t W) {
-  const int64_t most = std::max<int64_t>(64, MULTI_BYTES / (W * MULTI_CAP * 12));
-  const int64_t groups = (items + most - 1) / most;
+struct MultiShape {
+  int kp, W, cap;
+};
+MultiShape multi_shape(int64_t items, int64_t n_keys, int S) {
+  MultiShape m;
+  m.kp = scan_keys_per_thread(items, n_keys, S, false);
+  m.W = (int)((n_keys + WB * m.kp - 1) / (WB * m.kp));
+  m.cap = MULTI_CAP;
+  return m;
+}
+
+// Bytes of an item's counts, compact lists and one slice of the all-keys
+// select, and what a call needs besides (bounds, more slices of few items,
+// alignment).  Both grow with W and L.
+int64_t multi_item_bytes(int64_t W, int64_t cap, int64_t L) { return 8 * W + 12 * W * cap + 8 + 8 * L; }
+int64_t multi_fixed_bytes(int64_t items, int64_t L) { return 16 * items + kOverGrid * (4 + 8 * L) + 8 * 256; }
+
+// Items a launch may take in `bytes` of workspace (at least 64, or all of
+// them, of the size that summon_multi_workspace_bytes gives); 0: too few.
+int64_t multi_group(int64_t items, const MultiShape& m, int64_t L, size_t bytes) {
+  const int64_t room = ((int64_t)bytes - multi_fixed_bytes(items, L)) / multi_item_bytes(m.W, m.cap, L);
+  if (room < std::min<int64_t>(items, 64)) return 0;
+  const int64_t groups = (items + room - 1) / room;
   return (items + groups - 1) / groups;
 }
-size_t multi_lists_bytes(int64_t group, int64_t W) {
+size_t multi_lists_bytes(int64_t group, int64_t W, int cap) {
   return align256((size_t)(2 * group * W) * sizeof(uint32_t)) +
-         align256((size_t)(group * W * MULTI_CAP) * (sizeof(uint64_t) + sizeof(float)));
+         align256((size_t)(group * W * cap) * (sizeof(uint64_t) + sizeof(float)));
 }
 
 }  // namespace
 
+// Grows with the key count: lists of the smallest chunks, all items' or
+// MULTI_BYTES of them (64 items' if those take more).
+// Where the path ends (kMultiMaxKeys) the size stays: the buffer of a longer
+// cache serves shorter ones.
 size_t summon_multi_workspace_bytes(int64_t items, int64_t n_keys, int64_t L) {
-  if (n_keys < kWideMinKeys || n_keys > kMultiMaxKeys || items > kMultiMaxItems || 2 * L > FAST_M) return 256;
-  size_t most = 0;  // over the chunk sizes a call may take
-  for (int kp = 8; kp <= MAX_KP; kp *= 2) {
-    const int64_t W = (n_keys + WB * kp - 1) / (WB * kp);
-    const int64_t group = multi_group(items, W);
-    most = std::max(most, multi_lists_bytes(group, W) + over_bytes(group, std::max<int64_t>(L, 1)));
-  }
-  return align256((size_t)(4 * items) * sizeof(float)) + most;
+  if (n_keys < kWideMinKeys || items > kMultiMaxItems || 2 * L > FAST_M) return 256;
+  const int64_t W = (std::min(n_keys, kMultiMaxKeys) + 8 * WB - 1) / (8 * WB);
+  const int64_t one = multi_item_bytes(W, MULTI_CAP, L);
+  return (size_t)(multi_fixed_bytes(items, L) + std::min(items * one, std::max<int64_t>(MULTI_BYTES, 64 * one)));
 }
 
-int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, hipStream_t stream) {
-  const int kp = scan_keys_per_thread(items, p.N, p.S, false);
+bool summon_multi_taken(const SummonParams& p, int64_t items, const void* workspace, size_t workspace_bytes) {
+  if (!summon_multi_eligible(p, items) || workspace == nullptr || ((uintptr_t)workspace & 255u) != 0) return false;
+  const MultiShape m = multi_shape(items, p.N, p.S);
+  return multi_group(items, m, p.L, workspace_bytes) > 0;
+}
+
+int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, size_t workspace_bytes,
+                      hipStream_t stream) {
+  const MultiShape m = multi_shape(items, p.N, p.S);
+  const int kp = m.kp;
   WideArgs a{};
   a.p = p;
-  a.W = (int)((p.N + WB * kp - 1) / (WB * kp));
-  a.cap = MULTI_CAP;
+  a.W = m.W;
+  a.cap = m.cap;
   a.span_log2 = __builtin_ctz((unsigned)list_span(a.W));
   a.wave_keys = WAVE * kp;
-  const int64_t group = multi_group(items, a.W);
+  const int64_t group = multi_group(items, m, p.L, workspace_bytes);
+  SVA_REQUIRE(group > 0, "summon_multi_path: workspace of %zu bytes is too small", workspace_bytes);
   char* ws = (char*)workspace;
   float* range = (float*)ws;  // the items' bounds and floors
   ws += align256((size_t)(4 * items) * sizeof(float));
   a.wg_count = (uint32_t*)ws;
   a.wg_cand = (uint64_t*)(ws + align256((size_t)(2 * group * a.W) * sizeof(uint32_t)));
-  a.wg_rank = (float*)(a.wg_cand + group * a.W * MULTI_CAP);
+  a.wg_rank = (float*)(a.wg_cand + group * a.W * a.cap);
   a.K = over_slices(group);
-  char* over = ws + multi_lists_bytes(group, a.W);
+  char* over = ws + multi_lists_bytes(group, a.W, a.cap);
   a.arrive = (uint32_t*)over;
   a.slice_n = (uint32_t*)(over + align256((size_t)group * sizeof(uint32_t)));
   a.slice_list = (uint64_t*)(over + align256((size_t)group * sizeof(uint32_t)) +

@@ -60,6 +60,17 @@ def test_one_token_workspace_grows_with_the_cache(heads, shortlist):
     assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("n_seq,heads,tokens,shortlist", [
+    (1, 9, 4, 2048), (1, 9, 128, 2048), (1, 9, 256, 2048), (1, 9, 512, 512), (8, 9, 1, 512), (32, 32, 1, 3584), (1, 9, 7000, 512)])
+def test_several_token_workspace_grows_with_the_cache(n_seq, heads, tokens, shortlist):
+    """As above for several tokens or sequences: a plan sized for the next multiple of 65536 keys serves all below."""
+    lib = _lib()
+    counts = _key_counts(4 << 20)
+    sizes = [lib.sva_summon_workspace_bytes(n_seq, heads, tokens, n, shortlist) for n in counts]
+    assert sizes == sorted(sizes)
+    assert sizes[-1] > 256 and max(sizes) < 1 << 30
+
+
 def test_summon_strategy_selection():
     lib = _lib()
     # 1M keys, q = 1, 4x64 codes: many workgroups per item

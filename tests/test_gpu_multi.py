@@ -88,6 +88,43 @@ def test_multi_equals_item_path(device, n_seq, Q, lens, S, C, H, L, B, few, mask
     np.testing.assert_array_equal(got[1][item, :cnt].cpu().numpy().view(np.uint32), ranks.view(np.uint32))
 
 
+@pytest.mark.parametrize("n_seq,Q,lens,S,C,H,L,B,few", [
+    (1, 401, (33000,), 2, 256, 9, 512, 128, False),                    # the requested size holds half of the items
+    (1, 37, (40000,), 2, 256, 4, 1024, 300, False),                    # two or three groups, cut inside a head's tokens
+    (1, 37, (50000,), 2, 256, 4, 512, 128, True),                      # items selected over all their keys in each group
+    (7, 7, (30000, 1, 5000, 41000, 300, 65537, 7), 4, 64, 3, 2048, 512, False),  # packed, cut inside a sequence
+])
+def test_groups_of_items_equal_item_path(device, n_seq, Q, lens, S, C, H, L, B, few):
+    """A call takes its items in groups that its workspace holds: each group's tables, floors, outputs and arrival
+    counters are its own.  Every item bit for bit against one workgroup an item."""
+    from sva_amd import kernels
+    from sva_amd._lib import lib
+
+    rows, n, items = sum(lens), max(lens), n_seq * H * Q
+    g = torch.Generator(device=device).manual_seed(rows)
+    codes = torch.randint(0, 3 if few else C, (H, rows, S), device=device, generator=g).to(torch.uint8)
+    k_low = torch.randn(H, rows, 64, device=device, generator=g)
+    q = torch.randn(n_seq, H, Q, 64, device=device, generator=g)
+    q_proj = torch.randn(H, 64, 64, device=device, generator=g) / 8
+    cb = torch.randn(H, S, C, 64 // S, device=device, generator=g)
+    q_low, lut, rng = kernels.query_lut(q, q_proj, torch.ones(H, device=device), cb)
+    offs = lens_t = None
+    if n_seq > 1:
+        offs = torch.tensor([0, *lens[:-1]], device=device).cumsum(0)
+        lens_t = torch.tensor(lens, device=device)
+    size = int(lib().sva_summon_workspace_bytes(n_seq, H, Q, n, L))
+    if items < 1000:  # what 70 items of the largest lists ask for
+        size = int(lib().sva_summon_workspace_bytes(70, 1, 1, n, L))
+    got = _select(lut, rng, q_low, codes, k_low, n, L, B, size, offs, lens_t)
+    ref = _select(lut, rng, q_low, codes, k_low, n, L, B, 256, offs, lens_t)
+    assert torch.equal(got[2], ref[2])
+    for a, b, count in ((got[0], ref[0], ref[2][0]), (got[1].view(torch.int32), ref[1].view(torch.int32), ref[2][0]),
+                        (got[3], ref[3], ref[2][1])):
+        kept = torch.arange(a.shape[1], device=device)[None] < count[:, None]
+        same = (a == b) | ~kept
+        assert bool(same.all()), f"items {(~same).any(-1).nonzero().flatten().tolist()[:8]} differ"
+
+
 @pytest.mark.parametrize("N,S,C,L,kind", [
     (32768, 2, 256, 8192, "plain"),     # keys and bins in LDS, the batch decode's shape
     (33001, 4, 64, 8192, "plain"),      # the last round of 1024 keys partial
