@@ -110,6 +110,7 @@ struct FusedVerify {
 int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S, int64_t C, int64_t L,
                     int code_type, int mask_type);
 int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream);
+bool item_keys_in_lds(const SummonParams& p);  // it scores every key once
 bool summon_regs_eligible(const SummonParams& p);
 int summon_regs_path(const SummonParams& p, int64_t items, hipStream_t stream);
 // One token of one sequence on the per-item register path with the verifier

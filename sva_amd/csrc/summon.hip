@@ -459,12 +459,15 @@ int summon_regs_path(const SummonParams& p, int64_t items, hipStream_t stream) {
   return launch_regs_codes<16>(p, items, lds, stream);
 }
 
+bool item_keys_in_lds(const SummonParams& p) {
+  return p.N <= kMaxLds / 4 && item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, p.N <= 65536, false).total <= kMaxLds;
+}
+
 int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream) {
   const bool idx16 = p.N <= 65536;  // every sequence's length is at most N
   const bool lin_fit = p.N <= (int64_t)LIN_ITERS * ITEM_BLOCK &&
                        item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, idx16, true).total <= kMaxLds;
-  const bool keys_fit = lin_fit || (p.N <= kMaxLds / 4 &&
-                                    item_lds_layout(p.S, p.C, p.R, p.L, p.N, true, idx16, false).total <= kMaxLds);
+  const bool keys_fit = item_keys_in_lds(p);
   const ItemLds layout = item_lds_layout(p.S, p.C, p.R, p.L, p.N, keys_fit, idx16, lin_fit);
   SVA_UNSUPPORTED(layout.total <= kMaxLds, "sva_summon: shortlist %d with %dx%d codes exceeds LDS", p.L, p.S, p.C);
   const bool apart = items <= RS_MAX_ITEMS && p.L >= RS_MIN_L && p.R == 64 && ((uintptr_t)p.k_low & 15u) == 0 &&

@@ -62,10 +62,14 @@ constexpr uint32_t kNoCompact = 0x80000000u;  // wg_count flag: the workgroup wr
 constexpr int64_t kWideMinKeys = 16385;  // caches past the register path's 16384 keys
 constexpr int64_t kMaxWideItems = 64;
 // Several tokens or sequences (item_at): compact lists of MULTI_CAP entries,
-// as many items a launch as MULTI_BYTES of them hold.
+// MULTI_CAP_DENSE where a list expects more than eleven sixteenths of them
+// (larger lists mean more groups of items: 2304 items of 20000 keys, 2x256,
+// 512 kept, 224 us with 1024 entries, 194 with 512), as many items a launch as MULTI_BYTES of them
+// hold.
 constexpr int MULTI_CAP = 512;
+constexpr int MULTI_CAP_DENSE = NW * KL_CAP;
 constexpr int64_t MULTI_BYTES = 256ll << 20;
-constexpr int64_t kMultiMaxItems = 1 << 16;
+constexpr int64_t kMultiMaxItems = 1 << 16;  // (larger calls were not measured)
 constexpr int64_t kMultiMaxKeys = 256ll * WB * MAX_KP;  // the fast finish's 256 lists
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -91,6 +95,7 @@ struct WideArgs {
   int span_log2;       // lists per item rounded up to a power of two (list_span(W))
   int wave_keys;       // keys of a scan wave (64 KP), the capacity of its own list
   int item0;           // multi calls: the first item of this launch
+  int scan_min;        // and the fewest keys of an item that its lists hold (multi_scan_min)
   int groups, per;     // KV groups the fused finish is laid out by and their heads (0: not grouped)
   uint32_t* wg_count;  // [items, W, 2] candidates (or kNoCompact) and allowed keys of each scan workgroup
   uint64_t* wg_cand;   // [items, W, cap] a workgroup's candidates in key order (when they fit)
@@ -302,6 +307,13 @@ SVA_DEV float item_floor(const SummonParams& p, int item) {
   return est > lo ? est : lo;
 }
 
+// A several-item call's floor is a NaN where the item is not scanned for
+// candidates (multi_floor_kernel).
+SVA_DEV bool item_skips_scan(const SummonParams& p, int item) {
+  const float est = p.range[4 * item + 2];
+  return est != est;
+}
+
 // LDS views of a scan wave's candidate lists.  A store that goes either to
 // LDS or to global memory would otherwise be merged into one flat store, and
 // a flat store makes the next round wait for every code load still in flight
@@ -486,6 +498,11 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, const ItemAt& it, int w, fl
   const float4 qq = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * p.R)[lane_id() & 15];
   u32x4 raw[KP * S / 16];
   load_chunk<S, KP, !CHECK>(codes, cs, ce, raw);
+  if (MULTI && item_skips_scan(p, item)) {  // uniform, behind the loads: a look ahead of them costs every scan 0.5 us
+    if (threadIdx.x < 2)
+      a.wg_count[2 * ((int64_t)item * a.W + w) + threadIdx.x] = threadIdx.x == 0 ? 0u : (uint32_t)(ce - cs);
+    return;
+  }
   T.store(tab_lds);
   __syncthreads();  // tables in LDS
   const int wid = threadIdx.x / WAVE;
@@ -845,6 +862,51 @@ static_assert(kFastSmallR + sizeof(float) * SMALL_CAP <= kFastRank, "budget hist
 static_assert(SNW * FAST_BATCH * WAVE == 8192, "wg_cap: entries the first loads cover");
 static_assert(kWideMinKeys > 2 * WB * MAX_KP, "at least three lists an item (list l and wave wid agree modulo four)");
 static_assert(kFastEnd <= kFinStage, "the fast finish stays inside the finish kernel's staging area");
+
+// The rank of a several-item call's sampled floor among the samples of an
+// item of n keys (n, shortlists and samples of these calls are small enough
+// for 32-bit products); 0: every key is a candidate.
+__host__ __device__ inline int multi_floor_rank(int n, int S, int L) {
+  static_assert((int64_t)FAST_M * SAMPLE_MAX_BLOCKS * SAMPLE_KEYS < (1ll << 31), "target * ns");
+  static_assert(SAMPLE_TARGET == 2.0, "two shortlists of candidates");
+  const int ns = sample_blocks(n, S) * SAMPLE_KEYS;
+  const int target = 2 * L > (int)SAMPLE_MIN_CAND ? 2 * L : (int)SAMPLE_MIN_CAND;
+  if (n < SAMPLE_KEYS || n <= target) return 0;
+  const int k = target * ns / n + 1 > SAMPLE_MIN_RANK ? target * ns / n + 1 : SAMPLE_MIN_RANK;
+  return k < ns ? k : 0;
+}
+// Candidates that a list of `chunk` keys expects.
+inline int multi_list_expects(int n, int S, int L, int chunk) {
+  static_assert((int64_t)SAMPLE_MAX_BLOCKS * SAMPLE_KEYS * WB * MAX_KP < (1ll << 31), "k * chunk");
+  const int k = multi_floor_rank(n, S, L), len = n < chunk ? n : chunk;
+  return k > 0 ? k * len / (sample_blocks(n, S) * SAMPLE_KEYS) : len;
+}
+// Whether an item's candidates fit its lists, at_most expected in each, and
+// the fast finish, with room there for the floor's own spread (two standard
+// deviations, k^-1/2 of the mean each).  An item that outgrows them is
+// selected over all its keys after a scan for nothing: 2304 items of 16400
+// keys, 2x256, 2048 kept, took 713 us with lists of 512 expecting as many, 477
+// with lists of 1024, 337 with a workgroup an item; the last two meet at about
+// MULTI_MOST a list (18700 keys).
+constexpr int MULTI_MOST = 448;
+inline bool multi_fits(int n, int S, int L, int chunk, int at_most) {
+  const int k = multi_floor_rank(n, S, L);
+  if (k == 0) return n <= KL_CAP;  // one wave's list
+  const float mean = (float)k * (float)n / (float)(sample_blocks(n, S) * SAMPLE_KEYS);
+  return multi_list_expects(n, S, L, chunk) <= at_most && mean * (1.0f + 2.0f / sqrtf((float)k)) <= (float)FAST_M;
+}
+// The fewest keys from which on items of up to n keys fit; items of at most
+// KL_CAP keys (a wave's list) fit besides.  Found on the host: the divisions
+// cost the floor kernel's 4608 workgroups of a 512-token call 8 us.
+inline int multi_scan_min(int n, int S, int L, int chunk, int at_most) {
+  if (n <= KL_CAP || !multi_fits(n, S, L, chunk, at_most)) return 0x7FFFFFFF;
+  int lo = KL_CAP, hi = n;  // lists expect fewer as n grows; hi fits
+  while (hi - lo > 1) {
+    const int mid = lo + (hi - lo) / 2;
+    (multi_floor_rank(mid, S, L) > 0 && multi_list_expects(mid, S, L, chunk) <= at_most ? hi : lo) = mid;
+  }
+  return hi;
+}
 
 // Exclusive scan within a wave (all 64 lanes active).
 SVA_DEV uint32_t wave_excl_scan(uint32_t v) { return wave_incl_scan(v) - v; }

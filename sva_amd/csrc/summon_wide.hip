@@ -75,11 +75,11 @@ namespace {
 struct MultiShape {
   int kp, W, cap;
 };
-MultiShape multi_shape(int64_t items, int64_t n_keys, int S) {
+MultiShape multi_shape(int64_t items, int64_t n_keys, int S, int L) {
   MultiShape m;
   m.kp = scan_keys_per_thread(items, n_keys, S, false);
   m.W = (int)((n_keys + WB * m.kp - 1) / (WB * m.kp));
-  m.cap = MULTI_CAP;
+  m.cap = 16 * multi_list_expects((int)n_keys, S, L, WB * m.kp) > 11 * MULTI_CAP ? MULTI_CAP_DENSE : MULTI_CAP;
   return m;
 }
 
@@ -104,26 +104,35 @@ size_t multi_lists_bytes(int64_t group, int64_t W, int cap) {
 
 }  // namespace
 
-// Grows with the key count: lists of the smallest chunks, all items' or
-// MULTI_BYTES of them (64 items' if those take more).
+// Grows with the key count: lists of the smallest chunks and the largest
+// capacity, all items' or MULTI_BYTES of them (64 items' if those take more).
 // Where the path ends (kMultiMaxKeys) the size stays: the buffer of a longer
 // cache serves shorter ones.
 size_t summon_multi_workspace_bytes(int64_t items, int64_t n_keys, int64_t L) {
   if (n_keys < kWideMinKeys || items > kMultiMaxItems || 2 * L > FAST_M) return 256;
   const int64_t W = (std::min(n_keys, kMultiMaxKeys) + 8 * WB - 1) / (8 * WB);
-  const int64_t one = multi_item_bytes(W, MULTI_CAP, L);
+  const int64_t one = multi_item_bytes(W, MULTI_CAP_DENSE, L);
   return (size_t)(multi_fixed_bytes(items, L) + std::min(items * one, std::max<int64_t>(MULTI_BYTES, 64 * one)));
 }
 
+// Whether the path is the better one and has room: the longest item's lists
+// expect at most eleven sixteenths of what they hold, and MULTI_MOST.  An item
+// that outgrows its lists costs an all-keys select of one workgroup: up to
+// twice the one-workgroup form while that holds its keys in LDS (up to about
+// 36000 keys; 2304 items of 16400 keys, 2x256, 3584 kept: 771 us against 385),
+// a quarter of it past that, where every select pass scores every key again
+// (65536 keys: 1107 us against 4614).
 bool summon_multi_taken(const SummonParams& p, int64_t items, const void* workspace, size_t workspace_bytes) {
   if (!summon_multi_eligible(p, items) || workspace == nullptr || ((uintptr_t)workspace & 255u) != 0) return false;
-  const MultiShape m = multi_shape(items, p.N, p.S);
+  const MultiShape m = multi_shape(items, p.N, p.S, p.L);
+  const int at_most = std::min(11 * m.cap / 16, MULTI_MOST);
+  if (!multi_fits((int)p.N, p.S, p.L, WB * m.kp, at_most) && item_keys_in_lds(p)) return false;
   return multi_group(items, m, p.L, workspace_bytes) > 0;
 }
 
 int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, size_t workspace_bytes,
                       hipStream_t stream) {
-  const MultiShape m = multi_shape(items, p.N, p.S);
+  const MultiShape m = multi_shape(items, p.N, p.S, p.L);
   const int kp = m.kp;
   WideArgs a{};
   a.p = p;
@@ -131,6 +140,9 @@ int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, siz
   a.cap = m.cap;
   a.span_log2 = __builtin_ctz((unsigned)list_span(a.W));
   a.wave_keys = WAVE * kp;
+  // (three quarters of a list: the tokens of a call at the route's line, of
+  // eleven sixteenths, differ by a few keys)
+  a.scan_min = multi_scan_min((int)p.N, p.S, p.L, WB * kp, 3 * m.cap / 4);
   const int64_t group = multi_group(items, m, p.L, workspace_bytes);
   SVA_REQUIRE(group > 0, "summon_multi_path: workspace of %zu bytes is too small", workspace_bytes);
   char* ws = (char*)workspace;

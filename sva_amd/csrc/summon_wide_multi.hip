@@ -9,8 +9,10 @@ namespace {
 
 // An item's sampled floor (the query kernels sample for one token of one
 // sequence only): the blocks, histogram and rank of summon.h over the item's
-// own keys, one workgroup an item; writes the items' [lo, hi, floor, 0].  Latency bound: one round of loads (table
-// and code words), a histogram in LDS and one scan, 6.4 us for 36 items of 262144 keys.
+// own keys, one workgroup an item; writes the items' [lo, hi, floor, 0], a NaN
+// for the floor where the item is not scanned.  Latency bound: one round of
+// loads (table and code words), a histogram in LDS and one scan, 6.4 us for 36
+// items of 262144 keys.
 constexpr int MFB = 512;
 
 template <int S>
@@ -22,14 +24,16 @@ __global__ void __launch_bounds__(MFB) multi_floor_kernel(WideArgs a, float* ran
   const int item = blockIdx.x, t = threadIdx.x;
   const ItemAt it = item_at<true>(a, item);
   const float lo = p.range[4 * item], hi = p.range[4 * item + 1];
-  const int nb = sample_blocks(it.n, S), ns = nb * SAMPLE_KEYS;
-  const int64_t target = max((int64_t)(SAMPLE_TARGET * p.L), (int64_t)SAMPLE_MIN_CAND);
-  const int64_t k64 = max(target * ns / max(it.n, 1) + 1, (int64_t)SAMPLE_MIN_RANK);
-  if (it.n < SAMPLE_KEYS || it.n <= target || k64 >= ns || !(hi > lo)) {  // uniform: every key is a candidate
-    if (t < 4) range[4 * item + t] = t == 0 ? lo : t == 1 ? hi : t == 2 ? -INFINITY : 0.0f;
+  const int nb = sample_blocks(it.n, S);
+  const int rank = multi_floor_rank(it.n, S, p.L);
+  // an item that its lists would not hold is not scanned for candidates, nor
+  // one whose bounds are not finite (infinities or NaN in the table): every key is selected over
+  const bool scanned = (it.n >= a.scan_min || it.n <= KL_CAP) && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY;
+  if (!scanned || rank == 0 || !(hi > lo)) {  // uniform: no sample is taken
+    if (t < 4) range[4 * item + t] = t == 0 ? lo : t == 1 ? hi : t == 2 ? (scanned ? -INFINITY : NAN) : 0.0f;
     return;
   }
-  const uint32_t k = (uint32_t)k64;
+  const uint32_t k = (uint32_t)rank;
   const uint8_t* codes = item_codes(p, it);
   constexpr int WPB = SAMPLE_KEYS * S / 16;                                  // code words per block
   constexpr int NWD = (SAMPLE_MAX_BYTES / 16 + MFB - 1) / MFB;               // words per thread at most

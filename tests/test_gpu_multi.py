@@ -15,7 +15,7 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 
-def _select(lut, rng, q_low, codes, k_low, n_keys, L, B, ws_bytes, offs=None, lens=None, mask_type=0):
+def _select(lut, rng, q_low, codes, k_low, n_keys, L, B, ws_bytes, offs=None, lens=None, mask_type=0, events=None):
     from sva_amd import kernels
     from sva_amd._lib import check, code_type, lib, ptr, stream_handle
 
@@ -27,10 +27,14 @@ def _select(lut, rng, q_low, codes, k_low, n_keys, L, B, ws_bytes, offs=None, le
     counts = torch.full((2, items), -1, device=dev, dtype=torch.int32)
     fin = torch.full((items, B), -1, device=dev, dtype=torch.int32)
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    if events:
+        events[0].record()
     check(lib().sva_summon_select(
         ptr(lut), ptr(rng), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low), k_low.stride(0),
         ptr(offs), ptr(lens), n_seq, H, Q, n_keys, 64, S, C, L, None, mask_type, 0, ptr(sl_idx), ptr(sl_rank),
         counts[0].data_ptr(), B, ptr(fin), counts[1].data_ptr(), ptr(ws), ws.numel(), stream_handle(dev)), "select")
+    if events:
+        events[1].record()
     torch.cuda.synchronize()
     return sl_idx, sl_rank, counts, fin
 
@@ -97,10 +101,19 @@ def test_multi_equals_item_path(device, n_seq, Q, lens, S, C, H, L, B, few, mask
 def test_groups_of_items_equal_item_path(device, n_seq, Q, lens, S, C, H, L, B, few):
     """A call takes its items in groups that its workspace holds: each group's tables, floors, outputs and arrival
     counters are its own.  Every item bit for bit against one workgroup an item."""
-    from sva_amd import kernels
     from sva_amd._lib import lib
 
-    rows, n, items = sum(lens), max(lens), n_seq * H * Q
+    args = _tables(device, n_seq, Q, lens, S, C, H, few)
+    size = int(lib().sva_summon_workspace_bytes(n_seq, H, Q, max(lens), L))
+    if n_seq * H * Q < 1000:  # what 70 items of the largest lists ask for
+        size = int(lib().sva_summon_workspace_bytes(70, 1, 1, max(lens), L))
+    _assert_equal_items(*(_select(*args[:5], max(lens), L, B, ws, *args[5:]) for ws in (size, 256)))
+
+
+def _tables(device, n_seq, Q, lens, S, C, H, few=False):
+    from sva_amd import kernels
+
+    rows = sum(lens)
     g = torch.Generator(device=device).manual_seed(rows)
     codes = torch.randint(0, 3 if few else C, (H, rows, S), device=device, generator=g).to(torch.uint8)
     k_low = torch.randn(H, rows, 64, device=device, generator=g)
@@ -112,17 +125,55 @@ def test_groups_of_items_equal_item_path(device, n_seq, Q, lens, S, C, H, L, B, 
     if n_seq > 1:
         offs = torch.tensor([0, *lens[:-1]], device=device).cumsum(0)
         lens_t = torch.tensor(lens, device=device)
-    size = int(lib().sva_summon_workspace_bytes(n_seq, H, Q, n, L))
-    if items < 1000:  # what 70 items of the largest lists ask for
-        size = int(lib().sva_summon_workspace_bytes(70, 1, 1, n, L))
-    got = _select(lut, rng, q_low, codes, k_low, n, L, B, size, offs, lens_t)
-    ref = _select(lut, rng, q_low, codes, k_low, n, L, B, 256, offs, lens_t)
+    return lut, rng, q_low, codes, k_low, offs, lens_t
+
+
+def _assert_equal_items(got, ref):
     assert torch.equal(got[2], ref[2])
     for a, b, count in ((got[0], ref[0], ref[2][0]), (got[1].view(torch.int32), ref[1].view(torch.int32), ref[2][0]),
                         (got[3], ref[3], ref[2][1])):
-        kept = torch.arange(a.shape[1], device=device)[None] < count[:, None]
+        kept = torch.arange(a.shape[1], device=a.device)[None] < count[:, None]
         same = (a == b) | ~kept
         assert bool(same.all()), f"items {(~same).any(-1).nonzero().flatten().tolist()[:8]} differ"
+
+
+@pytest.mark.parametrize("n_seq,Q,lens,S,C,H,L,B", [
+    (1, 8, (18690,), 2, 256, 3, 2048, 512),      # either side of the line between the two forms
+    (1, 8, (18740,), 2, 256, 3, 2048, 512),
+    (1, 300, (23900,), 2, 256, 3, 2048, 512),    # and between the two list capacities
+    (1, 300, (23700,), 2, 256, 3, 2048, 512),
+    (1, 3, (50000,), 2, 256, 3, 3584, 700),      # every item selected over all its keys without a scan
+    (9, 1, (256, 257, 1024, 1025, 4097, 9000, 15000, 40000, 70000), 2, 256, 3, 2048, 512),  # some scanned, some not
+    (6, 2, (300, 700, 1100, 2100, 5000, 33000), 1, 256, 3, 512, 128),
+])
+def test_items_scanned_or_not_equal_item_path(device, n_seq, Q, lens, S, C, H, L, B):
+    """Items whose candidates would not fit their lists are selected over every key: bit for bit as one workgroup."""
+    from sva_amd._lib import lib
+
+    args = _tables(device, n_seq, Q, lens, S, C, H)
+    size = int(lib().sva_summon_workspace_bytes(n_seq, H, Q, max(lens), L))
+    _assert_equal_items(*(_select(*args[:5], max(lens), L, B, ws, *args[5:]) for ws in (size, 256)))
+
+
+@pytest.mark.parametrize("n_seq,Q,lens,S,C,L,B", [
+    (1, 64, (16400,), 2, 256, 2048, 512), (1, 64, (20000,), 1, 256, 2048, 512), (1, 64, (20000,), 8, 32, 2048, 512),
+    (1, 16, (24576,), 4, 64, 3584, 1024), (32, 1, (32768,) + (2000,) * 31, 2, 256, 512, 128)])
+def test_dense_calls_cost_about_the_item_path(device, n_seq, Q, lens, S, C, L, B):
+    """Shapes whose candidates outgrow the lists of the many-workgroup form took three to six times the time of one
+    workgroup an item there; they may take at most twice (1.6 measured at most)."""
+    from sva_amd._lib import lib
+
+    args = _tables(device, n_seq, Q, lens, S, C, 9)
+    size = int(lib().sva_summon_workspace_bytes(n_seq, 9, Q, max(lens), L))
+    times = []
+    for ws in (size, 256):
+        best = float("inf")
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            _select(*args[:5], max(lens), L, B, ws, *args[5:], events=(start, end))
+            best = min(best, start.elapsed_time(end))
+        times.append(best)
+    assert times[0] <= 2 * times[1], f"{times[0] * 1e3:.0f} us against {times[1] * 1e3:.0f}"
 
 
 @pytest.mark.parametrize("N,S,C,L,kind", [
