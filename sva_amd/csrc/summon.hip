@@ -34,7 +34,7 @@ struct ItemLds {
 
 // The linear-bin select of keys held in LDS (see summon_item_kernel).
 constexpr int LIN_BINS = 4096;
-constexpr int LIN_CAP = 1024;   // boundary-bin members ranked directly
+constexpr int LIN_CAP = 256;    // boundary-bin members ranked directly (m of them: m^2 LDS reads)
 constexpr int LIN_ITERS = 40;   // rounds of ITEM_BLOCK keys (163840 bytes of LDS hold fewer)
 
 // idx16: shortlist slots as uint16 (every key index below 65536), which
@@ -66,10 +66,12 @@ __host__ __device__ inline ItemLds item_lds_layout(int S, int C, int R, int L, i
   return l;
 }
 
-// flags: bit 0 the keys sit in LDS, bit 1 the shortlist slots are uint16,
-// bit 2 LDS has room for the linear-bin select (item_lds_layout's arguments;
-// the host sets them from the largest length), bit 3 the rank scores are left
-// to rescore_kernel.
+// LIN: LDS has room for the linear-bin select; flags: bit 0 the keys sit in
+// LDS, bit 1 the shortlist slots are uint16 (item_lds_layout's arguments; the
+// host sets them from the largest length), bit 2 the rank scores are left to
+// rescore_kernel.  (LIN at compile time: the select's registers and branches
+// cost the form without it 4 % at 38000 keys.)
+template <bool LIN>
 __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p, int flags) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) unsigned char lds[];
@@ -79,8 +81,8 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   const int b = item / (p.Q * p.H);
   const int64_t len = p.lens ? p.lens[b] : p.N;
   const int64_t off = p.offs ? p.offs[b] : 0;
-  const bool keys_in_lds = (flags & 1) != 0, idx16 = (flags & 2) != 0, lin = (flags & 4) != 0;
-  const ItemLds L = item_lds_layout(p.S, p.C, p.R, p.L, len, keys_in_lds, idx16, lin);
+  const bool keys_in_lds = (flags & 1) != 0, idx16 = (flags & 2) != 0;
+  const ItemLds L = item_lds_layout(p.S, p.C, p.R, p.L, len, keys_in_lds, idx16, LIN);
   float* tab = (float*)(lds + L.tab);
   float* ql = (float*)(lds + L.ql);
   uint32_t* hist = (uint32_t*)(lds + L.hist);
@@ -131,10 +133,16 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   // the compaction reads keys in lane order, not in thread-contiguous
   // segments that meet in two banks.  72 items of 32768 keys, 2x256, 8192 of
   // them kept: the kernel 92 us against 125 (44 with the rank scores apart).
-  const float lo_s = r64 ? p.range[4 * item] * 0.125f : p.range[4 * item] / sqrt_r;
-  const float hi_s = r64 ? p.range[4 * item + 1] * 0.125f : p.range[4 * item + 1] / sqrt_r;
+  // Larger bins are tie classes: ranked one against the other, or left to the
+  // radix passes over every key, they cost 144 items of 24576 keys, one
+  // subspace, 512 kept, 72 us a call where the radix passes alone took 53.
+  float lo_s = 0.0f, hi_s = 0.0f;
+  if (LIN) {
+    lo_s = r64 ? p.range[4 * item] * 0.125f : p.range[4 * item] / sqrt_r;
+    hi_s = r64 ? p.range[4 * item + 1] * 0.125f : p.range[4 * item + 1] / sqrt_r;
+  }
   const float span = hi_s - lo_s;
-  const bool linear = lin && span > 0.0f && span < INFINITY;
+  const bool linear = LIN && span > 0.0f && span < INFINITY;
   const float inv_w = (float)LIN_BINS / span;
   uint32_t* bins = (uint32_t*)(lds + L.slidx);
   // a non-decreasing function of the score
@@ -206,8 +214,7 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
 
   uint32_t T = 0u;
   int keq = 0x7FFFFFFF;  // every allowed key (T = 0 is no key's)
-  bool done = false;
-  if (linear && leff < (int)allowed_total) {
+  if (LIN && linear && leff < (int)allowed_total) {
     // thread t owns bins 4 t .. 4 t + 3 counted from the top
     const uint4 hv = reinterpret_cast<const uint4*>(bins)[ITEM_BLOCK - 1 - threadIdx.x];
     const uint32_t c[4] = {hv.w, hv.z, hv.y, hv.x};
@@ -221,12 +228,16 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
       }
       a += c[j];
     }
-    if (threadIdx.x == 0) shared[3] = 0u;
+    if (threadIdx.x == 0) {
+      shared[3] = 0u;
+      scratch[0] = 0xFFFFFFFFu;  // smallest and largest key of the boundary bin
+      scratch[1] = 0u;
+    }
     __syncthreads();
     const int bb = (int)shared[0];
-    const uint32_t need = (uint32_t)leff - shared[1], members = shared[2];
-    done = members <= (uint32_t)LIN_CAP;
-    if (done) {
+    uint32_t need = (uint32_t)leff - shared[1];
+    const uint32_t members = shared[2];
+    if (members <= (uint32_t)LIN_CAP) {
       uint64_t* mem = (uint64_t*)bins;  // every thread has read its bins
       for (int64_t n = threadIdx.x; n < len; n += ITEM_BLOCK) {
         const uint32_t k = keys[n];
@@ -237,6 +248,7 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
       if (threadIdx.x < members) {
         const uint64_t x = mem[threadIdx.x];
         uint32_t above = 0, above_key = 0;
+#pragma unroll 8
         for (uint32_t o = 0; o < members; ++o) {
           above += mem[o] > x ? 1u : 0u;
           above_key += (mem[o] >> 32) > (x >> 32) ? 1u : 0u;
@@ -249,12 +261,55 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
       __syncthreads();
       T = shared[0];
       keq = (int)shared[1];
+    } else {
+      // tie classes (with one subspace a bin is a code's hundreds of keys):
+      // the members are the keys from the smallest to the largest of the bin;
+      // ten bits of that range a pass until one key is left
+      uint32_t mn = 0xFFFFFFFFu, mx = 0u;
+      for (int64_t n = threadIdx.x; n < len; n += ITEM_BLOCK) {
+        const uint32_t k = keys[n];
+        if (k != 0u && bin_of(k) == bb) {
+          mn = min(mn, k);
+          mx = max(mx, k);
+        }
+      }
+      wave_min_max_u32(mn, mx);
+      if (lane_id() == 0 && mn <= mx) {
+        atomicMin(&scratch[0], mn);
+        atomicMax(&scratch[1], mx);
+      }
+      __syncthreads();
+      mn = scratch[0];
+      mx = scratch[1];
+      __syncthreads();
+      while (mn != mx) {  // uniform
+        static_assert(ITEM_BLOCK == 1 << 10, "a bin a thread");
+        const int shift = max(22 - __clz((int)(mx - mn)), 0);
+        bins[threadIdx.x] = 0u;
+        __syncthreads();
+        for (int64_t n = threadIdx.x; n < len; n += ITEM_BLOCK) {
+          const uint32_t d = keys[n] - mn;
+          if (d <= mx - mn) atomicAdd(&bins[d >> shift], 1u);
+        }
+        __syncthreads();
+        const uint32_t c2 = bins[ITEM_BLOCK - 1 - threadIdx.x];
+        const uint32_t a2 = block_excl_scan<ITEM_BLOCK>(c2, scratch, nullptr);
+        if (a2 < need && a2 + c2 >= need) {
+          shared[0] = ITEM_BLOCK - 1 - threadIdx.x;
+          shared[1] = a2;
+        }
+        __syncthreads();
+        mn += shared[0] << shift;
+        mx = min(mx, mn + ((1u << shift) - 1u));
+        need -= shared[1];
+        __syncthreads();
+      }
+      T = mn;
+      keq = (int)need;
     }
     __syncthreads();
-  } else if (linear) {
-    done = true;
   }
-  if (linear && done) {
+  if (LIN && linear) {
     // compaction in key-index order: round i of the block takes keys
     // i ITEM_BLOCK .., so (round, wave, lane) is key order; per (round, wave)
     // counts of both kinds in one word, one scan, then the slots
@@ -327,7 +382,7 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   const float* kl = p.k_low + (int64_t)h * p.klow_hs + off * p.R;
   int32_t* out_idx = p.sl_idx + (int64_t)item * p.L;
   float* out_rank = p.sl_rank + (int64_t)item * p.L;
-  if ((flags & 8) != 0) {
+  if ((flags & 4) != 0) {
     for (int j = threadIdx.x; j < leff; j += ITEM_BLOCK) out_idx[j] = (int32_t)slot(j);
   } else if (r64 && ((uintptr_t)kl & 15u) == 0) {  // block-uniform
     // lane octet o takes shortlist entries o, o + 128, ...: eight lanes per
@@ -472,9 +527,15 @@ int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream) {
   SVA_UNSUPPORTED(layout.total <= kMaxLds, "sva_summon: shortlist %d with %dx%d codes exceeds LDS", p.L, p.S, p.C);
   const bool apart = items <= RS_MAX_ITEMS && p.L >= RS_MIN_L && p.R == 64 && ((uintptr_t)p.k_low & 15u) == 0 &&
                      p.klow_hs % 4 == 0 && ((uintptr_t)p.q_low & 15u) == 0;
-  SVA_SET_MAX_LDS_ONCE(summon_item_kernel, kMaxLds, "hipFuncSetAttribute(summon_item_kernel)");
-  hipLaunchKernelGGL(summon_item_kernel, dim3((unsigned)items), dim3(ITEM_BLOCK), (size_t)layout.total, stream, p,
-                     (keys_fit ? 1 : 0) | (idx16 ? 2 : 0) | (lin_fit ? 4 : 0) | (apart ? 8 : 0));
+  const int flags = (keys_fit ? 1 : 0) | (idx16 ? 2 : 0) | (apart ? 4 : 0);
+  const dim3 grid((unsigned)items), block(ITEM_BLOCK);
+  if (lin_fit) {
+    SVA_SET_MAX_LDS_ONCE(summon_item_kernel<true>, kMaxLds, "hipFuncSetAttribute(summon_item_kernel)");
+    hipLaunchKernelGGL(summon_item_kernel<true>, grid, block, (size_t)layout.total, stream, p, flags);
+  } else {
+    SVA_SET_MAX_LDS_ONCE(summon_item_kernel<false>, kMaxLds, "hipFuncSetAttribute(summon_item_kernel)");
+    hipLaunchKernelGGL(summon_item_kernel<false>, grid, block, (size_t)layout.total, stream, p, flags);
+  }
   SVA_CHECK_LAUNCH("summon_item_kernel");
   if (apart) {
     hipLaunchKernelGGL(rescore_kernel, dim3((unsigned)((p.L + RS_PER - 1) / RS_PER), (unsigned)items), dim3(RS_BLOCK), 0,

@@ -220,3 +220,41 @@ def test_item_select_matches_oracle(device, N, S, C, L, kind):
             np.testing.assert_array_equal(idx[h * Q + t, :n].cpu().numpy(), want)
             ref = oracle.rank_scores(k_low[h].cpu().numpy(), want, q_low[0, h, t].cpu().numpy(), 64)
             np.testing.assert_array_equal(rank[h * Q + t, :n].cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("N,C,L,kind", [
+    (20000, 256, 4000, "near"),    # every key but an outlier's in one bin, 255 values: two or three passes over it
+    (30000, 256, 8192, "zero"),    # the bin's values about zero: a key range of nearly 32 bits
+    (33000, 16, 3999, "plain"),    # classes of two thousand keys
+    (9000, 2, 4500, "plain"),      # two classes, one taken in part
+    (20000, 200, 1, "near"),       # the best key alone, among ties
+])
+def test_item_select_boundary_bin_of_hundreds(device, N, C, L, kind):
+    """One workgroup an item with one subspace: a boundary bin past the directly ranked members, against the oracle."""
+    from sva_amd import kernels
+
+    H = 2
+    g = torch.Generator(device=device).manual_seed(N + C)
+    codes = torch.randint(0, C, (H, N, 1), device=device, generator=g).to(torch.uint8)
+    k_low = torch.randn(H, N, 64, device=device, generator=g)
+    q_low = torch.randn(1, H, 1, 64, device=device, generator=g)
+    lut = torch.randn(1, H, 1, 1, C, device=device, generator=g)
+    if kind != "plain":
+        lut = 1e-6 * torch.randperm(C, device=device, generator=g).float().expand(1, H, 1, 1, C) + (0.25 if kind == "near" else 0)
+        if kind == "zero":
+            lut = lut - 1e-6 * C / 2
+        lut = lut.contiguous()
+        lut[..., 0] = 1e3
+    rng = torch.zeros(1, H, 1, 4, device=device)
+    rng[..., 0], rng[..., 1] = lut.amin((-1, -2)), lut.amax((-1, -2))
+    # (a float mask keeps these calls on one workgroup an item)
+    mask = torch.zeros(1, 1, 1, N, device=device)
+    args = (lut.expand(1, H, 2, 1, C).contiguous(), rng.expand(1, H, 2, 4).contiguous(),
+            q_low.expand(1, H, 2, 64).contiguous(), codes, k_low, N, L)
+    idx, rank, count = kernels.summon(*args, mask=mask.expand(1, 1, 2, N).contiguous())
+    torch.cuda.synchronize()
+    for item in range(2 * H):
+        h = item // 2
+        scores = oracle.pq_scores_from_lut(lut[0, h, 0].cpu().numpy(), codes[h].cpu().numpy(), 64)
+        want = np.sort(oracle.topk(scores, L))
+        np.testing.assert_array_equal(idx[item, :int(count[item])].cpu().numpy(), want)
