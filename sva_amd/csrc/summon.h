@@ -146,6 +146,7 @@ int budget_select_launch(const int32_t* sl_idx, const float* sl_rank, const int3
                          int64_t L, int64_t B, int32_t* fin_idx, int32_t* fin_count, bool ordered,
                          hipStream_t stream);
 bool summon_wide_eligible(const SummonParams& p, int64_t items);
+bool summon_wide_taken(const SummonParams& p, int64_t items);  // and the better path
 // overshoot (optional, [items]): 1 where the sampled floor overshot and the
 // finish selected over every key, else 0.
 int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_bytes, hipStream_t stream,

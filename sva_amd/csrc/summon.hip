@@ -135,7 +135,8 @@ __global__ void __launch_bounds__(ITEM_BLOCK) summon_item_kernel(SummonParams p,
   // them kept: the kernel 92 us against 125 (44 with the rank scores apart).
   // Larger bins are tie classes: ranked one against the other, or left to the
   // radix passes over every key, they cost 144 items of 24576 keys, one
-  // subspace, 512 kept, 72 us a call where the radix passes alone took 53.
+  // subspace, 512 kept, 72 us a call where the radix passes alone took 53;
+  // narrowed by key range (below) 44.
   float lo_s = 0.0f, hi_s = 0.0f;
   if (LIN) {
     lo_s = r64 ? p.range[4 * item] * 0.125f : p.range[4 * item] / sqrt_r;
@@ -566,8 +567,7 @@ int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t
   p.L = (int)L;
   p.mask = dummy;
   p.mask_type = mask_type;
-  if (summon_class_eligible(p, n_seq * H * Q)) return 2;
-  if (summon_wide_eligible(p, n_seq * H * Q)) return 1;
+  if (summon_wide_taken(p, n_seq * H * Q)) return summon_class_eligible(p, n_seq * H * Q) ? 2 : 1;
   p.B = 1;
   return summon_regs_eligible(p) ? 3 : 0;
 }
@@ -644,13 +644,13 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
   // a prepared query launch (the tables this call reads): the code-class
   // path runs its decode form in one grid with the code counts; every other
   // path launches it first
-  // (code heads off 16-byte addresses took the per-item path, which needs no
-  // workspace, before the wide kernels read codes at any address: a call
-  // whose workspace is short still takes it; so do caches below 32768 keys)
+  // (caches below 32768 keys and code heads off 16-byte addresses take the wide
+  // path where it is the better one and the workspace holds it; else one
+  // workgroup an item, which needs none)
   const bool code16 = ((uintptr_t)codes & 15u) == 0 && code_head_stride % 16 == 0;
   const bool room = (code16 && n_keys >= 32768) || (workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
                                workspace_bytes >= sva::summon_wide_workspace_bytes(n_seq, H, Q, n_keys, L));
-  const bool wide_path = n_keys > 0 && room && sva::summon_wide_eligible(p, items);
+  const bool wide_path = n_keys > 0 && room && sva::summon_wide_taken(p, items);
   const bool class_path = wide_path && sva::summon_class_eligible(p, items);
   SVA_REQUIRE(stats == nullptr || (n_keys > 0 && !wide_path && sva::summon_regs_eligible(p)),
               "%s: a statistics row is added on the per-item register path only", fn);

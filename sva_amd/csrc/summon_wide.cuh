@@ -299,12 +299,17 @@ SVA_DEV bool key_ok(const SummonParams& p, int n, int ce) {
   return ok;
 }
 
-// Candidate floor of an item: the sampled estimate, or the table minimum
-// (every allowed key is a candidate) when there is none.
+// Candidate floor of an item: the sampled estimate.  Without one (a table
+// that no floor was sampled for, a shortlist of too many of the keys, bounds
+// that are not finite) a one-token item has no candidates, and every key is
+// selected over: listing every key instead took 740 us of a lookup of 20003
+// keys that takes 42 with a workgroup an item.  A several-item call's items
+// of a few keys list them all.
+template <bool MULTI>
 SVA_DEV float item_floor(const SummonParams& p, int item) {
   const float lo = p.range[4 * item + 0];
   const float est = p.range[4 * item + 2];
-  return est > lo ? est : lo;
+  return est > lo ? est : MULTI ? lo : NAN;
 }
 
 // A several-item call's floor is a NaN where the item is not scanned for
@@ -494,13 +499,20 @@ SVA_DEV void scan_chunk(const WideArgs& a, int item, const ItemAt& it, int w, fl
   const uint8_t* codes = item_codes(p, it);
   ScanTables<S, SMALLC> T;
   T.load(p, item);
-  const float t_lo = item_floor(p, item);
+  const float t_lo = item_floor<MULTI>(p, item);
   const float4 qq = reinterpret_cast<const float4*>(p.q_low + (int64_t)item * p.R)[lane_id() & 15];
   u32x4 raw[KP * S / 16];
   load_chunk<S, KP, !CHECK>(codes, cs, ce, raw);
-  if (MULTI && item_skips_scan(p, item)) {  // uniform, behind the loads: a look ahead of them costs every scan 0.5 us
-    if (threadIdx.x < 2)
-      a.wg_count[2 * ((int64_t)item * a.W + w) + threadIdx.x] = threadIdx.x == 0 ? 0u : (uint32_t)(ce - cs);
+  // an item without candidates (every key is selected over): its counts only.
+  // Uniform, and behind the loads: a look ahead of them costs every scan 0.5 us.
+  if (!MASKED && (MULTI ? item_skips_scan(p, item) : t_lo != t_lo)) {
+    const int64_t g = (int64_t)item * a.W + w;
+    if (!MULTI && lane_id() == 0) {
+      const int first = cs + (int)(threadIdx.x / WAVE) * (WAVE * KP);
+      a.ncand[g * NW + threadIdx.x / WAVE] = 0u;
+      a.nallow[g * NW + threadIdx.x / WAVE] = (uint32_t)max(min(ce - first, WAVE * KP), 0);
+    }
+    if (threadIdx.x < 2) a.wg_count[2 * g + threadIdx.x] = threadIdx.x == 0 ? 0u : (uint32_t)(ce - cs);
     return;
   }
   T.store(tab_lds);
@@ -1110,7 +1122,7 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
   // placed: 4096 bins linear in [floor, bound of any sum] (zeroed while the
   // loads are in flight; the bounds are read before the barrier, which no
   // load may cross)
-  const float vlo = item_floor(p, item) * kInvSqrtR;
+  const float vlo = item_floor<MULTI>(p, item) * kInvSqrtR;
   const float vinv = lin_scale(vlo, p.range[4 * item + 1] * kInvSqrtR);
   uint32_t* hist = (uint32_t*)(lds + kFastHist);
   reinterpret_cast<uint4*>(hist)[t] = uint4{0u, 0u, 0u, 0u};
@@ -1324,9 +1336,10 @@ SVA_DEV bool finish_fast(const WideArgs& a, int item, unsigned char* lds, uint32
 //           list order, then into registers; the selected find their list
 //           (binary search over the staging offsets) for their ranks;
 //           slot-ordered compaction;
-//   lists   (more candidates): selection straight from the global lists;
-//   all keys (the sampled floor let fewer than L keys through): selection
-//           over every key of the item, ranks computed here.
+//   lists   (more lists): selection straight from the global lists;
+//   all keys (the sampled floor let fewer than L keys through, or more than
+//           LDS_CAND, or there is none): selection over every key of the
+//           item, ranks computed here.
 // The last two are slower and give the same result.  The shortlist's rank
 // composites go to LDS in shortlist order for the budget.
 // ---------------------------------------------------------------------------
@@ -1758,14 +1771,18 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
   const uint32_t longest = shared[1];
   const int leff = (int)min((uint32_t)p.L, A);
   const int beff = min(p.B, leff);
-  if (slice > 0 && (leff == 0 || M >= (uint32_t)leff)) return -1;  // the floor held: slice 0 finishes
+  // candidates past the staging area are left to the all-keys select (the
+  // selection straight from the lists: 362 us of a lookup of 40003 keys, 8192
+  // kept), unless there are too many lists to stage
+  const bool held = M >= (uint32_t)leff && (M <= (uint32_t)LDS_CAND || nsub > STAGE_LISTS);
+  if (slice > 0 && (leff == 0 || held)) return -1;  // the floor held: slice 0 finishes
   beff_out = p.B > 0 ? beff : 0;
   if (t == 0) {
     p.sl_count[item] = leff;
     if (p.B > 0) p.fin_count[item] = beff;
   }
   if (leff == 0) return 0;
-  if (!MULTI && M >= (uint32_t)leff) {
+  if (!MULTI && held) {
     // the per-wave lists of scan workgroups that wrote a compact list hold
     // only candidates past their wave's first KL_CAP (none: a compact list is
     // written only when every wave's candidates fit its LDS list): copy the
@@ -1789,7 +1806,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     __syncthreads();
   }
   // bounds of every candidate composite: sums in [floor, upper bound of any sum]
-  const uint64_t c_lo = (uint64_t)f2key(item_floor(p, item) * kInvSqrtR) << 32;
+  const uint64_t c_lo = (uint64_t)f2key(item_floor<MULTI>(p, item) * kInvSqrtR) << 32;
   const uint64_t c_hi = ((uint64_t)f2key(p.range[4 * item + 1] * kInvSqrtR) << 32) | 0xFFFFFFFFull;
   if (!MULTI && M >= (uint32_t)leff && M <= (uint32_t)(NPD * SB) && nsub <= DL_LISTS && longest <= 48u) {
     if (longest <= 32u) {
@@ -1873,7 +1890,7 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
     }
     compact_ordered<SB, NPT>(e, X, leff, wcnt, scratch, slots,
                              [&](uint32_t o, uint64_t x, int i) { emit(o, x, rnk[i]); });
-  } else if (!MULTI && M >= (uint32_t)leff) {
+  } else if (!MULTI && held) {
     // lists: select straight from the per-wave lists in global memory
     dense = false;
     float* rkf = (float*)rk;
@@ -1909,11 +1926,13 @@ SVA_DEV int finish_item(const WideArgs& a, int item, int slice, unsigned char* l
       __syncthreads();
     }
   } else {
-    // all keys: the sampled floor overshot; this workgroup selects slice `slice`
+    // all keys: the sampled floor overshot, or there are too many candidates;
+    // this workgroup selects slice `slice`
     dense = false;
     const int N = it.n, K = over_used(N, a.K);
     if (slice >= K) return -1;
-    if (t == 0 && slice == 0 && a.overshoot != nullptr) a.overshoot[item] = 1;
+    if (t == 0 && slice == 0 && a.overshoot != nullptr)  // (no floor, no overshoot)
+      a.overshoot[item] = M < (uint32_t)leff && p.range[4 * item + 2] > p.range[4 * item] ? 1 : 0;
     const uint8_t* codes = item_codes(p, it);
     // the item's table in LDS: the slice select scores every key of the slice from it
     float* lut_l = (float*)(lds + kFinLut);

@@ -35,6 +35,35 @@ bool summon_wide_eligible(const SummonParams& p, int64_t items) {
 
 namespace {
 
+// Caches that one workgroup an item holds in LDS (up to about 36000 keys): the
+// wide path where its lists are dense enough to be quick and no denser.  Nine
+// heads, us a lookup, wide / item: 2x256 at 16385 keys L 512 17 / 33, L 2048 24
+// / 38, L 4096 (no floor, or more candidates than the fast finish holds) 57 /
+// 39, a float mask (chunks of 8192 keys) and L 2048 96 / 39; 8x32
+// (the same chunks) L 2048 90 / 60 at 16385 keys, 75 / 79 at 24576.  By code class (one subspace) the time grows
+// with L, the item form's with the keys: L 2048 54 / 42 at 16385, 45 / 50 at
+// 24576; under a mask 52 / 38 and L 512.
+bool wide_beats_item(const SummonParams& p, int64_t items) {
+  const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
+  if (summon_class_eligible(p, items)) return !masked && 12 * (int64_t)p.L <= p.N;
+  const int kp = scan_keys_per_thread(items, p.N, p.S, masked);
+  const int cap = wg_cap((int)((p.N + WB * kp - 1) / (WB * kp)));
+  const int ns = sample_blocks(p.N, p.S) * SAMPLE_KEYS, k = sample_floor_rank(p.L, p.N, ns);
+  if (k == 0) return false;
+  const double all = (double)k * (double)p.N / ns, list = (double)k * (WB * kp) / ns;  // candidates expected
+  return all * (1.0 + 2.0 / sqrt((double)k)) <= FAST_M && list <= (masked && p.S < 8 ? 0.7 : 1.4) * cap;
+}
+
+}  // namespace
+
+bool summon_wide_taken(const SummonParams& p, int64_t items) {
+  if (!summon_wide_eligible(p, items)) return false;
+  if (p.N >= 32768 && ((uintptr_t)p.codes & 15u) == 0 && p.code_hs % 16 == 0) return true;
+  return !item_keys_in_lds(p) || wide_beats_item(p, items);
+}
+
+namespace {
+
 size_t wide_bytes(int64_t items, int64_t n_keys, int64_t L) {
   // the largest over the chunk sizes a call may take (scan_keys_per_thread)
   size_t most = 0;

@@ -258,3 +258,71 @@ def test_item_select_boundary_bin_of_hundreds(device, N, C, L, kind):
         scores = oracle.pq_scores_from_lut(lut[0, h, 0].cpu().numpy(), codes[h].cpu().numpy(), 64)
         want = np.sort(oracle.topk(scores, L))
         np.testing.assert_array_equal(idx[item, :int(count[item])].cpu().numpy(), want)
+
+
+def _one_token(device, N, S, C, L, floor=True, nan=False):
+    from sva_amd import kernels
+
+    H = 9
+    g = torch.Generator(device=device).manual_seed(N + L)
+    codes = torch.randint(0, C, (H, N, S), device=device, generator=g).to(torch.uint8)
+    k_low = torch.randn(H, N, 64, device=device, generator=g)
+    q = torch.randn(1, H, 1, 64, device=device, generator=g)
+    q_proj = torch.randn(H, 64, 64, device=device, generator=g) / 8
+    cb = torch.randn(H, S, C, 64 // S, device=device, generator=g)
+    if nan:
+        cb[:, 0, 5, 0] = float("nan")
+    sampled = (codes, N, L) if floor else ()
+    q_low, lut, rng = kernels.query_lut(q, q_proj, torch.ones(H, device=device), cb, *sampled)
+    return lut, rng, q_low, codes, k_low
+
+
+@pytest.mark.parametrize("N,S,C,L,B,floor", [
+    (16385, 2, 256, 8192, 2048, True),    # a shortlist of half the keys: no floor is sampled
+    (20003, 2, 256, 2048, 512, False),    # tables that no floor was sampled for
+    (40003, 2, 256, 2048, 512, False),    # the same past the caches held in LDS, codes at odd addresses
+    (40003, 2, 256, 8192, 2048, True),    # more candidates than the finish stages
+    (18001, 1, 256, 7168, 1024, True),    # code classes of a long shortlist
+    (24575, 8, 32, 2048, 512, True), (24577, 8, 32, 2048, 512, True),  # about the lines between the forms
+    (24575, 1, 256, 2048, 512, True), (24576, 1, 256, 2048, 512, True),
+    (17000, 4, 64, 2700, 700, True), (17000, 4, 64, 3600, 700, True),
+])
+def test_one_token_routes(device, N, S, C, L, B, floor):
+    """One token over caches whose form the sizes choose: bit for bit as one workgroup an item, and within
+    twice it (1.3 measured; shortlists of half the keys took 18 times, tables without a floor likewise)."""
+    from sva_amd._lib import lib
+
+    args = _one_token(device, N, S, C, L, floor)
+    size = int(lib().sva_summon_workspace_bytes(1, 9, 1, N, L))
+    outs, times = [], []
+    for ws in (size, 256):
+        best = float("inf")
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            out = _select(*args, N, L, B, ws, events=(start, end))
+            best = min(best, start.elapsed_time(end))
+        outs.append(out)
+        times.append(best)
+    _assert_equal_items(*outs)
+    assert times[0] <= 2 * times[1], f"{times[0] * 1e3:.0f} us against {times[1] * 1e3:.0f}"
+
+
+@pytest.mark.parametrize("N,Q,S,C,L", [(20003, 1, 2, 256, 512), (40003, 1, 4, 64, 2048), (65536, 1, 2, 256, 512),
+                                       (20003, 3, 2, 256, 512), (50000, 3, 8, 32, 2048)])
+def test_nan_scores_come_first(device, N, Q, S, C, L):
+    """A NaN in a codebook makes a NaN of some keys' scores, which rank above every number (torch.topk's order): the
+    forms of many workgroups an item take them too."""
+    from sva_amd import kernels
+    from sva_amd._lib import lib
+
+    lut, rng, q_low, codes, k_low = _one_token(device, N, S, C, L, nan=True)
+    if Q > 1:
+        lut, rng, q_low = (t.expand(1, 9, Q, *t.shape[3:]).contiguous() for t in (lut, rng, q_low))
+    size = int(lib().sva_summon_workspace_bytes(1, 9, Q, N, L))
+    got = _select(lut, rng, q_low, codes, k_low, N, L, 100, size)
+    first = (codes[..., 0] == 5)
+    if Q == 1 and codes.stride(0) % 16 == 0:  # such a call does not take the form of one workgroup: the NaN keys alone
+        kept = torch.zeros(9, N, device=device, dtype=torch.bool).scatter_(1, got[0].long(), True)
+        assert bool((kept >= (first & (first.cumsum(1) <= L))).all())
+    else:
+        _assert_equal_items(got, _select(lut, rng, q_low, codes, k_low, N, L, 100, 256))
