@@ -131,6 +131,17 @@ int sva_pq_scores(const float *lut, const void *codes, int code_type, int64_t co
  * workspace: sva_summon_workspace_bytes(...) bytes, 256-byte aligned.
  */
 size_t sva_summon_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L);
+/*
+ * The same for calls whose codes and mask are known: 256 where no such call of
+ * up to n_keys keys has a use for more (several tokens under a float mask,
+ * codes wider than a byte, other ranks or layouts).  packed: seq_offsets are
+ * given.  Both sizes only grow with n_keys, so the buffer of a longer cache
+ * serves every shorter one; a smaller buffer than a call could use is not an
+ * error but for one token over 32768 keys or more (sva_summon_strategy 1 and
+ * 2): the call then takes one workgroup per query item.
+ */
+size_t sva_summon_call_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S,
+                                       int64_t C, int64_t L, int code_type, int mask_type, int packed);
 int sva_summon(const float *lut, const float *score_range, const float *q_low, const void *codes, int code_type,
                int64_t code_head_stride, const float *k_low, int64_t k_low_head_stride, const int64_t *seq_offsets,
                const int64_t *seq_lens, int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S,

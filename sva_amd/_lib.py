@@ -37,6 +37,7 @@ _SIGNATURES: dict[str, tuple[type, list]] = {
                            _I64, _I64, _I64, _P, _P, _P, _P]),
     "sva_pq_scores": (_I, [_P, _P, _I, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P]),
     "sva_summon_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
+    "sva_summon_call_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I, _I, _I]),
     "sva_summon": (_I, [_P, _P, _P, _P, _I, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                         _P, _I, _I64, _P, _P, _P, _P, _SZ, _P]),
     "sva_summon_select": (_I, [_P, _P, _P, _P, _I, _I64, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,

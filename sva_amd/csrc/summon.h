@@ -168,6 +168,8 @@ int summon_class_path(const SummonParams& p, void* workspace, size_t workspace_b
 // Whether summon_wide_path can run `fv` in its finish kernel for these sizes.
 bool fused_verify_eligible(const SummonParams& p, int64_t items, const FusedVerify& fv);
 size_t summon_wide_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t L);
+size_t summon_call_workspace_bytes(int64_t items, int64_t n_keys, int64_t R, int64_t S, int64_t C, int64_t L,
+                                   int code_type, int mask_type, bool one_token);
 
 inline int next_pow2_host(int x) {
   int p = 1;

@@ -584,6 +584,13 @@ extern "C" size_t sva_summon_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q
   return sva::summon_wide_workspace_bytes(n_seq, H, Q, n_keys, L);
 }
 
+extern "C" size_t sva_summon_call_workspace_bytes(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R,
+                                                  int64_t S, int64_t C, int64_t L, int code_type, int mask_type,
+                                                  int packed) {
+  return sva::summon_call_workspace_bytes(n_seq * H * Q, n_keys, R, S, C, L, code_type, mask_type,
+                                          n_seq == 1 && Q == 1 && packed == 0);
+}
+
 namespace {
 
 int summon_impl(const char* fn, const float* lut, const float* score_range, const float* q_low, const void* codes,

@@ -159,6 +159,15 @@ bool summon_multi_taken(const SummonParams& p, int64_t items, const void* worksp
   return multi_group(items, m, p.L, workspace_bytes) > 0;
 }
 
+size_t summon_call_workspace_bytes(int64_t items, int64_t n_keys, int64_t R, int64_t S, int64_t C, int64_t L,
+                                   int code_type, int mask_type, bool one_token) {
+  if (n_keys < kWideMinKeys || code_type != CODE_U8 || C > 256 || R != 64) return 256;
+  if (S != 1 && S != 2 && S != 4 && S != 8) return 256;
+  if (one_token) return items <= kMaxWideItems && L <= FIN_MAX_L ? wide_bytes(items, n_keys, L) : 256;
+  if (mask_type != MASK_NONE && mask_type != MASK_BOOL) return 256;
+  return summon_multi_workspace_bytes(items, n_keys, L);
+}
+
 int summon_multi_path(const SummonParams& p, int64_t items, void* workspace, size_t workspace_bytes,
                       hipStream_t stream) {
   const MultiShape m = multi_shape(items, p.N, p.S, p.L);

@@ -231,8 +231,9 @@ def summon(lut, score_range, q_low, codes, k_low, n_keys: int, shortlist: int, m
     sl_rank = torch.empty(items, shortlist, device=device, dtype=torch.float32)
     sl_count = torch.empty(items, device=device, dtype=torch.int32)
     m, mtype, mstride = mask_args(mask, q_len, n_keys)
-    ws_bytes = int(lib().sva_summon_workspace_bytes(n_seq, heads, q_len, n_keys, shortlist))
-    ws = workspace(device, ws_bytes)
+    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(
+        n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist, code_type(codes), mtype,
+        seq_offsets is not None)))
     check(
         lib().sva_summon(
             ptr(lut), ptr(score_range), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low),
@@ -288,8 +289,9 @@ def summon_select(lut, score_range, q_low, codes, k_low, n_keys: int, shortlist:
     sl_count = torch.empty(items, device=device, dtype=torch.int32)
     fin_idx = torch.empty(items, budget, device=device, dtype=torch.int32)
     fin_count = torch.empty(items, device=device, dtype=torch.int32)
-    ws_bytes = int(lib().sva_summon_workspace_bytes(n_seq, heads, q_len, n_keys, shortlist))
-    ws = workspace(device, ws_bytes)
+    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(
+        n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist, code_type(codes), mtype,
+        seq_offsets is not None)))
     check(
         lib().sva_summon_select(
             ptr(lut), ptr(score_range), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low),
@@ -330,7 +332,8 @@ def lookup_select(q, q_proj, scale, codebooks, codes, k_low, n_keys: int, shortl
     fin_idx = torch.empty(heads, budget, device=device, dtype=i32)
     fin_count = torch.empty(heads, device=device, dtype=i32)
     m, mtype, mstride = mask_args(mask, 1, n_keys)
-    ws = workspace(device, int(lib().sva_summon_workspace_bytes(1, heads, 1, n_keys, shortlist)))
+    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(1, heads, 1, n_keys, rank, subspaces, codewords,
+                                                                     shortlist, code_type(codes), mtype, 0)))
     check(
         lib().sva_lookup_select(
             ptr(q), dtype_code(q), q.stride(1), heads, head_dim, rank, subspaces, codewords, ptr(q_proj), ptr(scale),
@@ -424,7 +427,7 @@ class ScanDecodePlan:
                       self.fin_count.data_ptr(), self.overshoot.data_ptr())
         # per stream: (summon workspace, keys it is sized for) and (verify workspace, KV heads), so that one
         # plan driven from two streams never shares a scratch buffer between them
-        self._ws: dict[int, tuple[torch.Tensor, int]] = {}
+        self._ws: dict[int | tuple, tuple[torch.Tensor, int]] = {}
         self._vws: dict[int, tuple[torch.Tensor, int]] = {}
         self._checked_weights = set()  # (data_ptr, version, dtype, shape, strides) of weights that passed
 
@@ -501,17 +504,18 @@ class ScanDecodePlan:
               "sva_lookup_verify")
         return out
 
-    def _summon_ws(self, n_keys: int, stream: int | None = None) -> torch.Tensor:
-        n_seq, heads, q_len, _, _, _, _, shortlist, _ = self.shape
+    def _summon_ws(self, n_keys: int, stream: int | None = None, ctype: int = 0, mtype: int = 0) -> torch.Tensor:
         stream = stream_handle(self.device) if stream is None else stream
-        ws, cap = self._ws.get(stream, (None, -1))
+        key = (stream, ctype, mtype) if ctype or mtype else stream
+        ws, cap = self._ws.get(key, (None, -1))
         if n_keys > cap:
             # the summon workspace grows with the key count: sized for the next
             # multiple of 64K keys, so a decode loop re-queries it rarely
             cap = (n_keys + 65535) // 65536 * 65536
-            ws = workspace(self.device, int(self._lib.sva_summon_workspace_bytes(
-                n_seq, heads, q_len, cap, shortlist)), "plan")
-            self._ws[stream] = (ws, cap)
+            n_seq, heads, q_len, _, rank, subspaces, codewords, shortlist, _ = self.shape
+            ws = workspace(self.device, int(self._lib.sva_summon_call_workspace_bytes(
+                n_seq, heads, q_len, cap, rank, subspaces, codewords, shortlist, ctype, mtype, 0)), "plan")
+            self._ws[key] = (ws, cap)
         return ws
 
     def _verify_ws(self, keys, stream: int | None = None, kv_heads: int | None = None) -> torch.Tensor:
@@ -547,7 +551,8 @@ class ScanDecodePlan:
         L = self._lib
         stream = stream_handle(self.device)
         m, mtype, mstride = mask_args(mask, q_len, n_keys)
-        ws = self._summon_ws(n_keys)
+        # (several tokens: codes wider than a byte and float masks need no workspace)
+        ws = self._summon_ws(n_keys) if q_len == 1 else self._summon_ws(n_keys, None, code_type(codes), mtype)
         if n_seq == 1 and q_len == 1:
             # one token: query side and summon in one call (fused where the shapes allow)
             check(L.sva_lookup_select(q.data_ptr(), dtype_code(q), q.stride(1), heads, head_dim, rank, subspaces,

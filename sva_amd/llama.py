@@ -291,8 +291,9 @@ class SVALlamaAttention(nn.Module):
     def _query_chunks(self, query, k_len, mask, shortlist, budget, codes):
         """(qs, qe, mask, n_keys) per chunk of query tokens (sva/llama.py:221-223,
         262-268).  Every token's result is independent of the chunking, so the
-        default chunk bounds the per-launch buffers (about 512 MiB) rather
-        than following the reference's 128: the shortlist buffers, or, where
+        default chunk bounds the per-launch buffers (about 512 MiB, besides a
+        summon workspace of up to about 300 MiB past 16384 keys) rather than
+        following the reference's 128: the shortlist buffers, or, where
         the fused per-item summon keeps the shortlist inside the kernel
         (sva_summon_strategy 3), the tables and budget lists.  Without a mask
         the kernels' causal rule (key n for token t of Q iff n <= N - Q + t)

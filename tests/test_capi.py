@@ -71,6 +71,22 @@ def test_several_token_workspace_grows_with_the_cache(n_seq, heads, tokens, shor
     assert sizes[-1] > 256 and max(sizes) < 1 << 30
 
 
+def test_call_workspace_asks_for_what_the_call_can_use():
+    lib = _lib()
+    size = lib.sva_summon_call_workspace_bytes
+    # (n_seq, heads, tokens, keys, rank, subspaces, codewords, shortlist, code type, mask type, packed)
+    plain = (1, 9, 256, 40000, 64, 2, 256, 2048, 0, 0, 0)
+    assert size(*plain) == lib.sva_summon_workspace_bytes(1, 9, 256, 40000, 2048) > 1 << 20
+    assert size(1, 9, 1, 40000, 64, 2, 256, 2048, 0, 1, 0) == lib.sva_summon_workspace_bytes(1, 9, 1, 40000, 2048)
+    for at, value in ((9, 1), (8, 1), (4, 32), (5, 16), (6, 300), (7, 4096), (3, 16384)):
+        args = list(plain)
+        args[at] = value
+        assert size(*args) == 256, f"argument {at} = {value}"
+    for tokens, packed in ((1, 0), (1, 1), (300, 0)):
+        sizes = [size(1, 9, tokens, n, 64, 4, 64, 512, 0, 0, packed) for n in _key_counts(4 << 20)]
+        assert sizes == sorted(sizes)
+
+
 def test_summon_strategy_selection():
     lib = _lib()
     # 1M keys, q = 1, 4x64 codes: many workgroups per item
