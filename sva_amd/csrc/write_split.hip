@@ -17,14 +17,26 @@
 //
 // E, in units of the scaled values (x and c times a power of two that puts
 // the codebook's largest entry in [64, 128), exact in fp32), with |x|, |c|
-// the norms: a half rounds to 11 bits, so x - xh - xl is within 2^-22 of |x|
-// and the products within 2^-20 |x| |c| of x.c; their fp32 sums, 99 additions
-// in any order, within 2^-16 (|x| |c| + |c|^2); the lane's codeword number in
-// the low six bits of a score costs 2^-17 of the score; half subnormals are
-// off by 2^-25 an entry; the fp32 distances themselves are within
-// 2^-19 |x| |c| + 2^-22 (|x| + |c|)^2, and 2^-117 unscaled where their
-// products fall below fp32's normal range.  A row beyond the halves' range,
-// or with an infinity or NaN, has no finite lead and is taken in fp32.
+// the norms and n = 64 / S <= 64 entries a subspace.  Every fp32 addition and
+// product below is taken to be off by an ulp, 2^-23 of its result, whichever
+// way the matrix unit rounds:
+//   the halves   round to 11 bits: x - xh - xl is within 2^-22 |x|, likewise
+//                c, and xl cl is left out, 3 * 2^-22 |x| |c| in all;
+//   their sums   start at -|c|^2 / 2; the 2 n small products (2^-10 |x| |c| at
+//                most) come first, so 3 n + 1 additions round sums of up to
+//                |c|^2 / 2 and n those of up to |x| |c|: n = 64, the largest,
+//                2^-17 |x| |c| and 193 * 2^-24 |c|^2;
+//   the number   of the lane's codeword in the low six bits of a score:
+//                2^-17 (|x| |c| + |c|^2 / 2);
+//   |c|^2        n additions: n 2^-24 |c|^2 of its half;
+//   the fp32 distances  decided against: n 2^-23 |x| |c| of the product sum
+//                and 2^-22 (|x| + |c|)^2 of the two that follow, and 2^-117
+//                unscaled where their products fall below fp32's normal range;
+//   half subnormals  are off by 2^-25 an entry.
+// At n = 64 that is 2.4e-5 |x| |c| + 1.9e-5 |c|^2 and the terms of (|x| + |c|);
+// E takes 2^-15 = 3.05e-5 for both and more than the others need.  A row beyond the
+// halves' range, or with an infinity or NaN, has no finite lead and is taken
+// in fp32.
 //
 // Layout: a wave works alone, 32 rows at a time, and never meets the others
 // after the codebooks are in LDS.  Its rows pass through its own LDS slice
@@ -378,17 +390,22 @@ __global__ void __launch_bounds__(sp_threads<KF32>(), KF32 ? 2 : 3) write_split_
             v[r] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, h, v[r], 0, 0, 0);
           }
         } else {
+          // the small products of every k first, so that only the high ones'
+          // additions round sums of the full size (the bound at the top)
+          half8 ah[NK];
 #pragma unroll
           for (int k = 0; k < NK; ++k) {
-            const half8 ah = *reinterpret_cast<const half8*>(cf + (b * NK + k) * WAVE * FE);
+            ah[k] = *reinterpret_cast<const half8*>(cf + (b * NK + k) * WAVE * FE);
             const half8 al = *reinterpret_cast<const half8*>(cf + (b * NK + k) * WAVE * FE + LO);
 #pragma unroll
-            for (int r = 0; r < SP_TR; ++r) v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, xl[r][k], k == 0 ? c0 : v[r], 0, 0, 0);
+            for (int r = 0; r < SP_TR; ++r) v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[k], xl[r][k], k == 0 ? c0 : v[r], 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < SP_TR; ++r) v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, xh[r][k], v[r], 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < SP_TR; ++r) v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, xh[r][k], v[r], 0, 0, 0);
           }
+#pragma unroll
+          for (int k = 0; k < NK; ++k)
+#pragma unroll
+            for (int r = 0; r < SP_TR; ++r) v[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[k], xh[r][k], v[r], 0, 0, 0);
         }
         // the lane's codeword number (4 b + i) in the low bits, then the two largest
 #pragma unroll
