@@ -2248,10 +2248,6 @@ template <int VD, int VKV, bool MULTI>
 __global__ void __launch_bounds__(SB) wide_finish_kernel(WideArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ float qsh[VD > 0 ? VD : 1];  // the verifier's query row
-  // the arguments ahead of the first loads, requested together: taken where
-  // each is used they are four scalar-cache misses in turn
-  asm volatile("" ::"s"(a.W), "s"(a.wg_count), "s"(a.wg_cand), "s"(a.wg_rank), "s"(a.p.range), "s"(a.overshoot));
-  if (VD > 0) asm volatile("" ::"s"(a.fv.q), "s"(a.fv.q_hs), "s"(a.fv.q_dtype));
   int item, slice;
   finish_slot(a, (int)blockIdx.x, item, slice);
   // the query row is requested before the finish starts and parked in LDS
