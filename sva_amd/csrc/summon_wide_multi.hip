@@ -24,13 +24,18 @@ __global__ void __launch_bounds__(MFB) multi_floor_kernel(WideArgs a, float* ran
   const int item = blockIdx.x, t = threadIdx.x;
   const ItemAt it = item_at<true>(a, item);
   const float lo = p.range[4 * item], hi = p.range[4 * item + 1];
+  auto unsampled = [&](bool scanned) {
+    if (t < 4) range[4 * item + t] = t == 0 ? lo : t == 1 ? hi : t == 2 ? (scanned ? -INFINITY : NAN) : 0.0f;
+  };
+  // an item that its lists would not hold is not scanned for candidates, nor
+  // one whose bounds are not finite (infinities or NaN in the table): every
+  // key is selected over.  (Exits uniform; the bounds are waited for behind
+  // the code words' requests.)
   const int nb = sample_blocks(it.n, S);
   const int rank = multi_floor_rank(it.n, S, p.L);
-  // an item that its lists would not hold is not scanned for candidates, nor
-  // one whose bounds are not finite (infinities or NaN in the table): every key is selected over
-  const bool scanned = (it.n >= a.scan_min || it.n <= KL_CAP) && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY;
-  if (!scanned || rank == 0 || !(hi > lo)) {  // uniform: no sample is taken
-    if (t < 4) range[4 * item + t] = t == 0 ? lo : t == 1 ? hi : t == 2 ? (scanned ? -INFINITY : NAN) : 0.0f;
+  const bool fits = it.n >= a.scan_min || it.n <= KL_CAP;
+  if (!fits || rank == 0) {
+    unsampled(fits && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY);
     return;
   }
   const uint32_t k = (uint32_t)rank;
@@ -45,6 +50,10 @@ __global__ void __launch_bounds__(MFB) multi_floor_kernel(WideArgs a, float* ran
     const int g = min(t + i * MFB, words - 1);
     const int64_t n0 = ((int64_t)(g / WPB) * (it.n - SAMPLE_KEYS) / (nb - 1)) & ~(int64_t)15;
     w[i] = code_word(codes + n0 * S + 16 * (g % WPB));
+  }
+  if (!(hi > lo) || !(fabsf(lo) < INFINITY && fabsf(hi) < INFINITY)) {
+    unsampled(fabsf(lo) < INFINITY && fabsf(hi) < INFINITY);
+    return;
   }
   const int C = p.C;
   for (int e = t; e < S * C; e += MFB) tab[e] = p.lut[(int64_t)item * S * C + e];
