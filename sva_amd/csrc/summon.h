@@ -105,8 +105,8 @@ struct FusedVerify {
   int64_t o_hs;
 };
 
-// The route of a call with these shapes (sva_summon_strategy's values, 1 and
-// 2 also below its 32768 keys).
+// The route of a lookup with its verifier of these shapes
+// (sva_summon_strategy's values, 1 and 2 also below its 32768 keys).
 int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t R, int64_t S, int64_t C, int64_t L,
                     int code_type, int mask_type);
 int summon_item_path(const SummonParams& p, int64_t items, hipStream_t stream);
@@ -146,7 +146,8 @@ int budget_select_launch(const int32_t* sl_idx, const float* sl_rank, const int3
                          int64_t L, int64_t B, int32_t* fin_idx, int32_t* fin_count, bool ordered,
                          hipStream_t stream);
 bool summon_wide_eligible(const SummonParams& p, int64_t items);
-bool summon_wide_taken(const SummonParams& p, int64_t items);  // and the better path
+// and the better path (verify: the call runs the verifier too)
+bool summon_wide_taken(const SummonParams& p, int64_t items, bool verify);
 // overshoot (optional, [items]): 1 where the sampled floor overshot and the
 // finish selected over every key, else 0.
 int summon_wide_path(const SummonParams& p, void* workspace, size_t workspace_bytes, hipStream_t stream,

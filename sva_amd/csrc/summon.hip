@@ -567,7 +567,7 @@ int summon_strategy(int64_t n_seq, int64_t H, int64_t Q, int64_t n_keys, int64_t
   p.L = (int)L;
   p.mask = dummy;
   p.mask_type = mask_type;
-  if (summon_wide_taken(p, n_seq * H * Q)) return summon_class_eligible(p, n_seq * H * Q) ? 2 : 1;
+  if (summon_wide_taken(p, n_seq * H * Q, true)) return summon_class_eligible(p, n_seq * H * Q) ? 2 : 1;
   p.B = 1;
   return summon_regs_eligible(p) ? 3 : 0;
 }
@@ -657,7 +657,7 @@ int summon_impl(const char* fn, const float* lut, const float* score_range, cons
   const bool code16 = ((uintptr_t)codes & 15u) == 0 && code_head_stride % 16 == 0;
   const bool room = (code16 && n_keys >= 32768) || (workspace != nullptr && ((uintptr_t)workspace & 255u) == 0 &&
                                workspace_bytes >= sva::summon_wide_workspace_bytes(n_seq, H, Q, n_keys, L));
-  const bool wide_path = n_keys > 0 && room && sva::summon_wide_taken(p, items);
+  const bool wide_path = n_keys > 0 && room && sva::summon_wide_taken(p, items, fv != nullptr);
   const bool class_path = wide_path && sva::summon_class_eligible(p, items);
   SVA_REQUIRE(stats == nullptr || (n_keys > 0 && !wide_path && sva::summon_regs_eligible(p)),
               "%s: a statistics row is added on the per-item register path only", fn);

@@ -43,9 +43,9 @@ namespace {
 // (the same chunks) L 2048 90 / 60 at 16385 keys, 75 / 79 at 24576.  By code class (one subspace) the time grows
 // with L, the item form's with the keys: L 2048 54 / 42 at 16385, 45 / 50 at
 // 24576; under a mask 52 / 38 and L 512.
-bool wide_beats_item(const SummonParams& p, int64_t items) {
+bool wide_beats_item(const SummonParams& p, int64_t items, bool verify) {
   const bool masked = p.mask_type == MASK_F32 || p.mask_type == MASK_BF16 || p.mask_type == MASK_F16;
-  if (summon_class_eligible(p, items)) return !masked && 12 * (int64_t)p.L <= p.N;
+  if (summon_class_eligible(p, items)) return !masked && (verify ? 9 : 11) * (int64_t)p.L <= p.N;
   const int kp = scan_keys_per_thread(items, p.N, p.S, masked);
   const int cap = wg_cap((int)((p.N + WB * kp - 1) / (WB * kp)));
   const int ns = sample_blocks(p.N, p.S) * SAMPLE_KEYS, k = sample_floor_rank(p.L, p.N, ns);
@@ -56,10 +56,10 @@ bool wide_beats_item(const SummonParams& p, int64_t items) {
 
 }  // namespace
 
-bool summon_wide_taken(const SummonParams& p, int64_t items) {
+bool summon_wide_taken(const SummonParams& p, int64_t items, bool verify) {
   if (!summon_wide_eligible(p, items)) return false;
   if (p.N >= 32768 && ((uintptr_t)p.codes & 15u) == 0 && p.code_hs % 16 == 0) return true;
-  return !item_keys_in_lds(p) || wide_beats_item(p, items);
+  return !item_keys_in_lds(p) || wide_beats_item(p, items, verify);
 }
 
 namespace {

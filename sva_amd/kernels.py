@@ -217,6 +217,13 @@ def mask_args(mask: torch.Tensor | None, q_len: int, n_keys: int):
     return m, _lib.MASK_TYPES[m.dtype], m.stride(0)
 
 
+def _summon_bytes(n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist, ctype, mtype, packed) -> int:
+    if n_keys <= 16384:  # one workgroup per item keeps no workspace
+        return 256
+    return int(lib().sva_summon_call_workspace_bytes(n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist,
+                                                     ctype, mtype, packed))
+
+
 def summon(lut, score_range, q_low, codes, k_low, n_keys: int, shortlist: int, mask: torch.Tensor | None = None,
            seq_offsets: torch.Tensor | None = None, seq_lens: torch.Tensor | None = None):
     """Shortlist (idx, rank score, count) per query item (sva/llama.py:270-292)."""
@@ -231,9 +238,8 @@ def summon(lut, score_range, q_low, codes, k_low, n_keys: int, shortlist: int, m
     sl_rank = torch.empty(items, shortlist, device=device, dtype=torch.float32)
     sl_count = torch.empty(items, device=device, dtype=torch.int32)
     m, mtype, mstride = mask_args(mask, q_len, n_keys)
-    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(
-        n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist, code_type(codes), mtype,
-        seq_offsets is not None)))
+    ws = workspace(device, _summon_bytes(n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist,
+                                         code_type(codes), mtype, seq_offsets is not None))
     check(
         lib().sva_summon(
             ptr(lut), ptr(score_range), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low),
@@ -289,9 +295,8 @@ def summon_select(lut, score_range, q_low, codes, k_low, n_keys: int, shortlist:
     sl_count = torch.empty(items, device=device, dtype=torch.int32)
     fin_idx = torch.empty(items, budget, device=device, dtype=torch.int32)
     fin_count = torch.empty(items, device=device, dtype=torch.int32)
-    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(
-        n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist, code_type(codes), mtype,
-        seq_offsets is not None)))
+    ws = workspace(device, _summon_bytes(n_seq, heads, q_len, n_keys, rank, subspaces, codewords, shortlist,
+                                         code_type(codes), mtype, seq_offsets is not None))
     check(
         lib().sva_summon_select(
             ptr(lut), ptr(score_range), ptr(q_low), ptr(codes), code_type(codes), codes.stride(0), ptr(k_low),
@@ -332,8 +337,8 @@ def lookup_select(q, q_proj, scale, codebooks, codes, k_low, n_keys: int, shortl
     fin_idx = torch.empty(heads, budget, device=device, dtype=i32)
     fin_count = torch.empty(heads, device=device, dtype=i32)
     m, mtype, mstride = mask_args(mask, 1, n_keys)
-    ws = workspace(device, int(lib().sva_summon_call_workspace_bytes(1, heads, 1, n_keys, rank, subspaces, codewords,
-                                                                     shortlist, code_type(codes), mtype, 0)))
+    ws = workspace(device, _summon_bytes(1, heads, 1, n_keys, rank, subspaces, codewords, shortlist, code_type(codes),
+                                         mtype, False))
     check(
         lib().sva_lookup_select(
             ptr(q), dtype_code(q), q.stride(1), heads, head_dim, rank, subspaces, codewords, ptr(q_proj), ptr(scale),

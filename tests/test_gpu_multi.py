@@ -284,7 +284,7 @@ def _one_token(device, N, S, C, L, floor=True, nan=False):
     (40003, 2, 256, 8192, 2048, True),    # more candidates than the finish stages
     (18001, 1, 256, 7168, 1024, True),    # code classes of a long shortlist
     (24575, 8, 32, 2048, 512, True), (24577, 8, 32, 2048, 512, True),  # about the lines between the forms
-    (24575, 1, 256, 2048, 512, True), (24576, 1, 256, 2048, 512, True),
+    (22527, 1, 256, 2048, 512, True), (22528, 1, 256, 2048, 512, True),
     (17000, 4, 64, 2700, 700, True), (17000, 4, 64, 3600, 700, True),
 ])
 def test_one_token_routes(device, N, S, C, L, B, floor):
