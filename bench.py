@@ -508,6 +508,7 @@ def write_profiles(args):
 
 
 MFMA_F32_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix peak (AMD spec)
+MFMA_F16_PEAK_TFLOPS = 2500.0  # MI355X dense f16 MFMA
 
 
 def write_suite(args):
@@ -541,13 +542,16 @@ def write_suite(args):
     ms = e0.elapsed_time(e1) / steps
     flop = 2.0 * heads * n * (d * r + r * codewords)  # projection + x.c products of every subspace
     tflops = flop / (ms * 1e-3) / 1e12
+    least_ms = 2e3 * heads * n * (d * r / (MFMA_F32_PEAK_TFLOPS * 1e12) + 3 * r * codewords / (MFMA_F16_PEAK_TFLOPS * 1e12))
     print(json.dumps({
         "metric": "catalog build (k_low projection + PQ assignment)", "value": round(n / (ms * 1e-3) / 1e6, 2),
         "unit": "Mkeys/s", "n_gpus": 1, "steps": steps, "ms_per_step": round(ms, 4), "higher_is_better": True,
         "dtype": "fp32 (bf16 K in)", "data": "synthetic", "config": {"workload": f"{n}-key catalog, 9 heads, "
                                                                                    f"{args.layout} codes"},
-        "roofline": {"kernel": "write_encode_persistent_kernel", "bound": "mfma", "achieved": round(tflops, 2),
-                     "peak": MFMA_F32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(tflops / MFMA_F32_PEAK_TFLOPS, 4),
+        # the least time: the projection on fp32 MFMA, then three half products a score (write_split.hip)
+        "roofline": {"kernel": "write_split_kernel", "bound": "mfma", "achieved": round(tflops, 2),
+                     "peak": round(flop / (least_ms * 1e-3) / 1e12, 2), "unit": "TFLOP/s",
+                     "frac": round(least_ms / ms, 4),
                      "flop_per_launch": flop, "traffic": None},
     }), flush=True)
 
