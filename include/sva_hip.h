@@ -213,10 +213,11 @@ int sva_lookup_verify(const void *q, int q_dtype, int64_t q_head_stride, int64_t
 
 /*
  * Which summon strategy a call with these shapes takes (16-byte aligned
- * k_low assumed): 0 = one workgroup per query item (caches of 16385 to
- * 32767 keys at q = 1 run the kernels of 1 and 2, and several tokens or
- * sequences over 16385 keys or more, shortlists of at most 3584, those of 1,
- * where the workspace holds sva_summon_workspace_bytes), 1 = wide path (q = 1
+ * k_low assumed): 0 = one workgroup per query item, or, where the workspace
+ * holds sva_summon_workspace_bytes and the sizes make it the quicker form, the
+ * kernels of 1 and 2 (q = 1 over 16385 to 32767 keys; several tokens or
+ * sequences over 16385 keys or more, shortlists of at most 3584): 0 promises
+ * nothing about outputs beyond sva_summon's, 1 = wide path (q = 1
  * over a long cache: many workgroups per item, one pass over the codes),
  * 2 = code-class path (the wide path's shapes with one subspace of at most
  * 256 codewords: the shortlist taken by code class from per-chunk code

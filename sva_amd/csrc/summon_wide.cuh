@@ -79,7 +79,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // heads 200006 bytes apart), and one global_load_dwordx4 reads them either
 // way, at worst from one more cache line a wave.  Asking for 16-byte aligned
 // heads instead sent every such cache to the per-item path: 579 us a lookup
-// of 100003 keys (2x256, 512 / 128) against 58 here.
+// of 100003 keys (2x256, 512 / 128) against 27 here.
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 SVA_DEV u32x4 code_word(const uint8_t* c) { return *reinterpret_cast<const u32x4_any*>(c); }
 SVA_DEV u32x4 code_word_nt(const uint8_t* c) {

@@ -530,7 +530,7 @@ bool write_split_eligible(const WriteParams& p) {
   if (p.D != 64 || p.R != 64 || p.codes == nullptr || p.n_rows >= (1ll << 31)) return false;
   // below, the per-workgroup set-up (map, norms, halves: about 35 us) is what
   // counts: nine heads of 4096 rows 44 us here and 43 in fp32, 8192 rows 48
-  // and 59, 262144 rows 462 and 1061
+  // and 59, 262144 rows 468 and 1052 (timed calls; 540 under the profiler)
   if (p.n_rows * p.H < 49152) return false;
   if (p.kv_rs < 0 || p.kv_rs > (1ll << 24)) return false;  // 32 rows by 32-bit offsets
   return (p.S == 1 && p.C == 256) || (p.S == 2 && p.C == 256) || (p.S == 4 && p.C == 64);
