@@ -22,6 +22,7 @@ batch-8 socket model's tok/s ("socket"), each measured at its own step count.
 from __future__ import annotations
 
 import argparse
+import gc
 import json
 import math
 import os
@@ -1152,6 +1153,10 @@ def main():
         torch.cuda.synchronize()
         del src, dst
 
+    # the interpreter's full collection of what the imports left (40 ms, once)
+    # otherwise fell among the timed steps or beside them as counts had it:
+    # 2000 steps took 39.4 or 48 us each
+    gc.collect()
     for i in range(args.warmup):
         step(i)
     torch.cuda.synchronize()
