@@ -2117,11 +2117,16 @@ SVA_DEV void verify_item(const SummonParams& p, const FusedVerify& v, int item, 
         vv[2 * j + 1][0] = KV == BF16 ? __uint_as_float(x & 0xFFFF0000u) : __half2float(__ushort_as_half((unsigned short)(x >> 16)));
       }
     } else {
+      // the rows are the wave's, so their addresses are scalars: one vector
+      // address a row took the registers that K and V rows of fp32 leave, and
+      // the spills made every lookup 4 us slower (9 heads x 1M keys 44.0)
+      static_assert(EPR <= WAVE, "a round's list entries, one a lane");
+      const int ids = kid[min(r0 + lane % EPR, cnt - 1)];
 #pragma unroll
       for (int j = 0; j < EPR; ++j) {
-        const int64_t row = kvb + (int64_t)kid[min(r0 + j, cnt - 1)] * v.kv_rs + lane;
+        const int64_t row = kvb + (int64_t)__builtin_amdgcn_readlane(ids, j) * v.kv_rs;
 #pragma unroll
-        for (int d = 0; d < DL; ++d) vv[j][d] = kv_one<KV>(v.values, row + WAVE * d);
+        for (int d = 0; d < DL; ++d) vv[j][d] = kv_one<KV>(v.values, row + WAVE * d + lane);
       }
     }
     float sc[KI], mr = -INFINITY;
